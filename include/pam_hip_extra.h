@@ -1,0 +1,23 @@
+/*
+ * pam_hip_extra.h -- entry points of libpam_hip.so beside the drop-in interface of pam_hip.h: the same computations for
+ * callers that have several of them to make at once, or something to learn from one.  Conventions as in pam_hip.h.
+ */
+#ifndef PAM_HIP_EXTRA_H
+#define PAM_HIP_EXTRA_H
+
+#include <stddef.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* pam_hip_logsumexp_fwd for a caller that requires finite inputs and wants to know on the host: *nonfinite (a word of page-locked host
+ * memory, cleared by the caller) becomes 1 if x holds an infinity or NaN, and `checked` (a hipEvent_t, or NULL) is recorded
+ * once that is settled, before the rows' own pass, so that the host can look while the GPU goes on. */
+int pam_hip_logsumexp_fwd_finite(const float *x, float *lse, float *log_softmax, float *shift, long rows, long n, float offset,
+                                 int *nonfinite, void *checked, void *workspace, size_t workspace_bytes, void *stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* PAM_HIP_EXTRA_H */

@@ -7,6 +7,7 @@ stream only.  There is no CPU fallback: a missing library or a non-GPU tensor ra
 """
 import ctypes
 import pathlib
+import threading
 
 import torch
 
@@ -68,6 +69,11 @@ _SIGNATURES = {
     "pam_hip_layer_norm_fwd": ([_p, _p, _p, _p, _l, _l, _f, _f, _p], _i),
 }
 
+# include/pam_hip_extra.h
+_EXTRA_SIGNATURES = {
+    "pam_hip_logsumexp_fwd_finite": ([_p, _p, _p, _p, _l, _l, _f, _p, _p, _p, _z, _p], _i),
+}
+
 _lib = None
 
 
@@ -84,7 +90,7 @@ def load_library():
                 f"{_LIB_PATH} is missing: build the HIP extension first (python -m pam_amd.build). "
                 "This package has no CPU or PyTorch fallback.")
         lib = ctypes.CDLL(str(_LIB_PATH))
-        for name, (argtypes, restype) in _SIGNATURES.items():
+        for name, (argtypes, restype) in {**_SIGNATURES, **_EXTRA_SIGNATURES}.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = restype
@@ -160,6 +166,26 @@ _CURRENT = _Current()
 def _on(device):
     """Context that makes `device` current for the launches inside it."""
     return _CURRENT if device.index is None or device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+class _FiniteWord(threading.local):
+    """Where a kernel reports to the host that its input is not finite: per thread and device a page-locked word and
+    the event behind its last write.  A thread reads its word before it makes its next call, so one is enough."""
+
+    def __init__(self):
+        self.by_device = {}
+
+    def get(self, device):
+        entry = self.by_device.get(device.index)
+        if entry is None:
+            word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            event = torch.cuda.Event()
+            event.record()                            # (creates it)
+            entry = self.by_device[device.index] = (word, ctypes.c_int.from_address(word.data_ptr()), event)
+        return entry
+
+
+_finite_word = _FiniteWord()
 
 
 def _check(*tensors):
@@ -382,8 +408,9 @@ class HipRowKernels:
                       int(bool(approx_exp)), _stream())
         return dX
 
-    def logsumexp_fwd(self, X, offset, want_lse=True, want_log_softmax=False):
-        """Returns (lse or None, log_softmax or None, shift)."""
+    def logsumexp_fwd(self, X, offset, want_lse=True, want_log_softmax=False, check_finite=False):
+        """Returns (lse or None, log_softmax or None, shift).  check_finite: an infinity or NaN in X raises
+        AssertionError; the host waits for the pass that looks (the one that finds the maximum), not for the rows'."""
         rows, n = self._rows("logsumexp_fwd", X)
         lse = torch.empty(rows, dtype=torch.float32, device=X.device) if want_lse else None
         Y = torch.empty_like(X) if want_log_softmax else None
@@ -391,11 +418,18 @@ class HipRowKernels:
         if X.numel():
             with _on(X.device):
                 ws, nbytes = self._workspace(X.device)
-                _call("pam_hip_logsumexp_fwd", X.data_ptr(), lse.data_ptr() if want_lse else None,
-                      Y.data_ptr() if want_log_softmax else None, shift.data_ptr(), rows, n, float(offset),
-                      ws.data_ptr(), nbytes, _stream())
+                outputs = (lse.data_ptr() if want_lse else None, Y.data_ptr() if want_log_softmax else None, shift.data_ptr())
+                if check_finite:
+                    word, nonfinite, event = _finite_word.get(X.device)
+                    nonfinite.value = 0
+                    _call("pam_hip_logsumexp_fwd_finite", X.data_ptr(), *outputs, rows, n, float(offset), word.data_ptr(),
+                          event.cuda_event, ws.data_ptr(), nbytes, _stream())
+                    event.synchronize()
+                    if nonfinite.value != 0:
+                        raise AssertionError("logsumexp and log_softmax need finite inputs")
+                else:
+                    _call("pam_hip_logsumexp_fwd", X.data_ptr(), *outputs, rows, n, float(offset), ws.data_ptr(), nbytes, _stream())
         return lse, Y, shift
-
 
     def logsumexp_bwd(self, X, grad, shift, offset, approx_a, approx_b, approx_exp, log_softmax):
         rows, n = self._rows("logsumexp_bwd", X, grad, shift)

@@ -75,6 +75,8 @@ def softmax(x, dim=None, *, offset=None, approx_bwd=False, use_kernel=True):
 def logsumexp(x, dim, keepdim=False, *, offset=None, approx_bwd=False, use_kernel=True):
     """pam/pam_ops.py:331-342; inputs must be finite."""
     kw = _pam_kwargs(offset, approx_bwd, use_kernel)
+    if _fused(x, dim, use_kernel, x) and fused.finite_in_kernel():
+        return fused.logsumexp(x, keepdim, offset, approx_bwd, check_finite=True)
     assert x.isfinite().all()
     if _fused(x, dim, use_kernel, x):
         return fused.logsumexp(x, keepdim, offset, approx_bwd)
@@ -88,6 +90,8 @@ def logsumexp(x, dim, keepdim=False, *, offset=None, approx_bwd=False, use_kerne
 def log_softmax(x, dim=None, *, offset=None, approx_bwd=False, use_kernel=True):
     """pam/pam_ops.py:345-347"""
     if _fused(x, dim, use_kernel, x):
+        if fused.finite_in_kernel():
+            return fused.log_softmax(x, offset, approx_bwd, check_finite=True)
         assert x.isfinite().all()
         return fused.log_softmax(x, offset, approx_bwd)
     return x - logsumexp(x, dim=dim, keepdim=True, **_pam_kwargs(offset, approx_bwd, use_kernel))

@@ -13,7 +13,7 @@ constexpr int kMaxPartials = 1024;          // per-block maxima of the scaled in
 #define PAM_ROW_DECLARE(FN) \
     int FN(softmax_fwd)(const float* x, float* y, float* row_sum, float* shift, long rows, long n, float offset, void* workspace, size_t workspace_bytes, void* stream); \
     int FN(softmax_bwd)(const float* x, const float* dy, const float* row_sum, const float* shift, float* dx, long rows, long n, float offset, int approx_a, int approx_b, int approx_exp, void* stream); \
-    int FN(logsumexp_fwd)(const float* x, float* lse, float* log_softmax, float* shift, long rows, long n, float offset, void* workspace, size_t workspace_bytes, void* stream); \
+    int FN(logsumexp_fwd)(const float* x, float* lse, float* log_softmax, float* shift, long rows, long n, float offset, int* nonfinite, void* checked, void* workspace, size_t workspace_bytes, void* stream); \
     int FN(row_mean_fwd)(const float* x, float* y, long rows, long n, float offset, void* stream); \
     int FN(layer_norm_fwd)(const float* x, const float* weight, const float* bias, float* y, long rows, long n, float eps, float offset, void* stream); \
     int FN(logsumexp_bwd)(const float* x, const float* grad, const float* shift, float* dx, long rows, long n, int log_softmax, float offset, int approx_a, int approx_b, int approx_exp, void* stream); \

@@ -1,6 +1,7 @@
 // Entry points of the row-wise kernels: the variant without the offset's code in its fast path for an offset of 1.0,
 // the other one otherwise (pam_rowops.h).
 #include "../../include/pam_hip.h"
+#include "../../include/pam_hip_extra.h"
 #include "pam_rowops.h"
 
 extern "C" {
@@ -21,8 +22,13 @@ int pam_hip_softmax_bwd(const float* x, const float* dy, const float* row_sum, c
 
 int pam_hip_logsumexp_fwd(const float* x, float* lse, float* log_softmax, float* shift, long rows, long n, float offset, void* workspace, size_t workspace_bytes, void* stream)
 {
-    return offset != 1.0f ? PAM_ROW_OFFSET(logsumexp_fwd)(x, lse, log_softmax, shift, rows, n, offset, workspace, workspace_bytes, stream)
-                          : PAM_ROW_PLAIN(logsumexp_fwd)(x, lse, log_softmax, shift, rows, n, offset, workspace, workspace_bytes, stream);
+    return pam_hip_logsumexp_fwd_finite(x, lse, log_softmax, shift, rows, n, offset, nullptr, nullptr, workspace, workspace_bytes, stream);
+}
+
+int pam_hip_logsumexp_fwd_finite(const float* x, float* lse, float* log_softmax, float* shift, long rows, long n, float offset, int* nonfinite, void* checked, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return offset != 1.0f ? PAM_ROW_OFFSET(logsumexp_fwd)(x, lse, log_softmax, shift, rows, n, offset, nonfinite, checked, workspace, workspace_bytes, stream)
+                          : PAM_ROW_PLAIN(logsumexp_fwd)(x, lse, log_softmax, shift, rows, n, offset, nonfinite, checked, workspace, workspace_bytes, stream);
 }
 
 int pam_hip_row_mean_fwd(const float* x, float* y, long rows, long n, float offset, void* stream)

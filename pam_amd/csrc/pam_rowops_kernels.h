@@ -140,10 +140,16 @@ __device__ __forceinline__ float exp2_op(float t, Offset o) { return exp2_entry(
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // 128-bit loads, four in flight per lane; the maximum does not depend on the order
+// NONFINITE: also sets *nonfinite to 1 if some value is an infinity or NaN (callers whose input must be finite; one
+// integer maximum per value of a pass that waits for memory, where a look of its own at 4096 x 10000 values took five
+// passes of 180 us)
+template <bool NONFINITE>
 __global__ __launch_bounds__(kThreads) void scaled_max_kernel(const float* __restrict__ x, size_t n, size_t nvec, Offset o,
-                                                             int mask_inf, float* __restrict__ partial)
+                                                             int mask_inf, float* __restrict__ partial, int* __restrict__ nonfinite)
 {
     MaxNan m;
+    uint32_t largest = 0u;                  // of the bit patterns without sign, shifted up by one
+    auto see = [&](float v) __attribute__((always_inline)) { if (NONFINITE) largest = max(largest, f2u(v) << 1); };
     const bool mask = mask_inf != 0;
     const v4f* xv = reinterpret_cast<const v4f*>(x);
     const size_t step = (size_t)gridDim.x * (kThreads * 4);
@@ -156,11 +162,15 @@ __global__ __launch_bounds__(kThreads) void scaled_max_kernel(const float* __res
             if (base + (size_t)u * kThreads < nvec) {
                 m.take(scaled(q[u].x, o, mask)); m.take(scaled(q[u].y, o, mask));
                 m.take(scaled(q[u].z, o, mask)); m.take(scaled(q[u].w, o, mask));
+                see(q[u].x); see(q[u].y); see(q[u].z); see(q[u].w);
             }
         }
     }
-    for (size_t i = nvec * 4 + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads)
-        m.take(scaled(x[i], o, mask));
+    for (size_t i = nvec * 4 + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads) {
+        const float v = x[i];
+        m.take(scaled(v, o, mask)); see(v);
+    }
+    if (NONFINITE && largest >= (kExpo << 1)) *nonfinite = 1;         // (whoever writes it, it is the same value)
     m.merge_wave();
     __shared__ float smx[kWaves]; __shared__ int snan[kWaves];
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -1647,7 +1657,7 @@ int check_rows(const char* what, long rows, long n)
 }
 
 int launch_max(const char* what, const float* x, long rows, long n, Offset o, int mask_inf, void* workspace,
-               size_t workspace_bytes, hipStream_t st, int* partials)
+               size_t workspace_bytes, hipStream_t st, int* partials, int* nonfinite = nullptr)
 {
     if (!workspace || workspace_bytes < (size_t)kMaxPartials * sizeof(float))
         return pamhost::fail(PAM_HIP_ERR_WORKSPACE, "%s: workspace of %zu bytes needed", what, (size_t)kMaxPartials * sizeof(float));
@@ -1657,8 +1667,12 @@ int launch_max(const char* what, const float* x, long rows, long n, Offset o, in
     if (blocks > (size_t)kMaxPartials) blocks = kMaxPartials;
     if (blocks < 1) blocks = 1;
     *partials = (int)blocks;
-    hipLaunchKernelGGL(scaled_max_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, x, total, nvec, o, mask_inf,
-                       (float*)workspace);
+    if (nonfinite)
+        hipLaunchKernelGGL(scaled_max_kernel<true>, dim3((unsigned)blocks), dim3(kThreads), 0, st, x, total, nvec, o, mask_inf,
+                           (float*)workspace, nonfinite);
+    else
+        hipLaunchKernelGGL(scaled_max_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, st, x, total, nvec, o, mask_inf,
+                           (float*)workspace, nonfinite);
     return pamhost::check_launch(what);
 }
 
@@ -1706,15 +1720,19 @@ int PAM_ROW_FN(softmax_bwd)(const float* x, const float* dy, const float* row_su
 }
 
 int PAM_ROW_FN(logsumexp_fwd)(const float* x, float* lse, float* log_softmax, float* shift, long rows, long n, float offset,
-                          void* workspace, size_t workspace_bytes, void* stream)
+                          int* nonfinite, void* checked, void* workspace, size_t workspace_bytes, void* stream)
 {
     int rc = check_rows("logsumexp_fwd", rows, n);
     if (rc != PAM_HIP_OK) return rc;
     if (rows == 0 || n == 0) return PAM_HIP_OK;
     if (!x || (!lse && !log_softmax)) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "logsumexp_fwd: null pointer");
     hipStream_t st = (hipStream_t)stream; Offset o{offset, offset != 1.0f}; int partials = 0;
-    rc = launch_max("logsumexp_fwd", x, rows, n, o, 0, workspace, workspace_bytes, st, &partials);
+    rc = launch_max("logsumexp_fwd", x, rows, n, o, 0, workspace, workspace_bytes, st, &partials, nonfinite);
     if (rc != PAM_HIP_OK) return rc;
+    if (checked) {
+        const hipError_t e = hipEventRecord((hipEvent_t)checked, st);
+        if (e != hipSuccess) return pamhost::fail(PAM_HIP_ERR_LAUNCH, "logsumexp_fwd: %s", hipGetErrorString(e));
+    }
     if (block_rows(n)) {
         PAM_BLOCK_DISPATCH(logsumexp_block_kernel, n, dim3(block_grid(rows)), st, x, lse, log_softmax, shift, rows, n, o,
                            (const float*)workspace, partials);

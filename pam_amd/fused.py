@@ -76,12 +76,12 @@ class logsumexp_autograd(torch.autograd.Function):
     """logsumexp (as_log_softmax False) or log_softmax = x - logsumexp(x) over the last dimension."""
 
     @staticmethod
-    def forward(ctx, x, offset, approx_bwd, as_log_softmax, keepdim):
+    def forward(ctx, x, offset, approx_bwd, as_log_softmax, keepdim, check_finite=False):
         ctx.offset = _offset_value(offset)
         ctx.approx_bwd = approx_bwd
         ctx.as_log_softmax = as_log_softmax
         rows = x.reshape(-1, x.shape[-1])
-        lse, y, shift = row_kernels.logsumexp_fwd(rows, ctx.offset, not as_log_softmax, as_log_softmax)
+        lse, y, shift = row_kernels.logsumexp_fwd(rows, ctx.offset, not as_log_softmax, as_log_softmax, check_finite)
         ctx.save_for_backward(rows, shift)
         if as_log_softmax:
             return y.view(x.shape)
@@ -92,16 +92,21 @@ class logsumexp_autograd(torch.autograd.Function):
         rows, shift = ctx.saved_tensors
         g = grad.contiguous().view(rows.shape if ctx.as_log_softmax else (rows.shape[0],))
         dx = row_kernels.logsumexp_bwd(rows, g, shift, ctx.offset, *_flags(ctx.approx_bwd), ctx.as_log_softmax)
-        return dx, None, None, None, None
+        return dx, None, None, None, None, None
 
 
-def logsumexp(x, keepdim, offset=None, approx_bwd=False):
-    out = logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, False, True)
+def logsumexp(x, keepdim, offset=None, approx_bwd=False, check_finite=False):
+    out = logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, False, True, check_finite)
     return out.view(x.shape[:-1] + ((1,) if keepdim else ()))
 
 
-def log_softmax(x, offset=None, approx_bwd=False):
-    return logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, True, True).view(x.shape)
+def log_softmax(x, offset=None, approx_bwd=False, check_finite=False):
+    return logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, True, True, check_finite).view(x.shape)
+
+
+def finite_in_kernel():
+    """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded."""
+    return not torch.cuda.is_current_stream_capturing()
 
 
 class mean_autograd(torch.autograd.Function):

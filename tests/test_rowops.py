@@ -632,3 +632,29 @@ def test_gpu_mean_gradient(oracle, off):
     xt = _dev(x).requires_grad_()
     pam_amd.mean(xt, dim=-1, offset=off, approx_bwd=False).backward(_dev(g))                             # exact: the chain
     assert torch.isfinite(xt.grad).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 5), (5, 197), (2, 4097), (1, 17001)])
+def test_nonfinite_input_is_refused_and_the_largest_finite_one_is_not(rows, n):
+    """logsumexp and log_softmax refuse an infinity or NaN anywhere in the input (first value, last value, in the part
+    behind the last full 128-bit vector), on any stream, and accept every finite value."""
+    x = torch.randn(rows, n, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            for at in {0, rows * n // 2, rows * n - 1}:
+                for value in (math.inf, -math.inf, math.nan):
+                    bad = x.clone()
+                    bad.view(-1)[at] = value
+                    for call in (lambda: pam_amd.log_softmax(bad, dim=-1), lambda: pam_amd.logsumexp(bad, dim=-1)):
+                        with pytest.raises(AssertionError):
+                            call()
+                largest = x.clone()
+                largest.view(-1)[at] = torch.finfo(torch.float32).max
+                pam_amd.log_softmax(largest, dim=-1)
+                pam_amd.logsumexp(largest, dim=-1)
+        side.synchronize()
+    y = pam_amd.log_softmax(x, dim=-1)                    # and a refused call leaves nothing behind
+    assert torch.equal(y, pam_amd.log_softmax(x, dim=-1))
