@@ -17,6 +17,14 @@ extern "C" {
 int pam_hip_logsumexp_fwd_finite(const float *x, float *lse, float *log_softmax, float *shift, long rows, long n, float offset,
                                  int *nonfinite, void *checked, void *workspace, size_t workspace_bytes, void *stream);
 
+/* pam_hip_adam_step for `count` tensors with the same scalars, in one launch per 96 of them.  The table is read before the
+ * call returns.  Tensors whose p, m or v share memory with another buffer of the list are updated one after the other, in
+ * the list's order. */
+typedef struct { float *p; const float *g; float *m; float *v; size_t n; } pam_hip_adam_tensor;
+int pam_hip_adam_step_many(const pam_hip_adam_tensor *tensors, long count, float beta1, float one_minus_beta1, float beta2,
+                           float one_minus_beta2, float eps, float decay, int has_decay, float step_size, float offset,
+                           void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -5,6 +5,7 @@
 (a new tensor; inputs untouched).  PyTorch is used for device memory and the current
 stream only.  There is no CPU fallback: a missing library or a non-GPU tensor raises.
 """
+import array
 import ctypes
 import pathlib
 import threading
@@ -72,6 +73,7 @@ _SIGNATURES = {
 # include/pam_hip_extra.h
 _EXTRA_SIGNATURES = {
     "pam_hip_logsumexp_fwd_finite": ([_p, _p, _p, _p, _l, _l, _f, _p, _p, _p, _z, _p], _i),
+    "pam_hip_adam_step_many": ([_p, _l, _f, _f, _f, _f, _f, _f, _i, _f, _f, _p], _i),
 }
 
 _lib = None
@@ -535,6 +537,17 @@ def adam_step(p, g, m, v, beta1, one_minus_beta1, beta2, one_minus_beta2, eps, d
             _call("pam_hip_adam_step", p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel(), float(beta1),
                   float(one_minus_beta1), float(beta2), float(one_minus_beta2), float(eps), float(decay or 0.0),
                   int(bool(decay)), float(step_size), float(offset), _stream())
+
+
+def adam_step_many(table, device, beta1, one_minus_beta1, beta2, one_minus_beta2, eps, decay, step_size, offset):
+    """adam_step for many tensors on `device` with the same scalars.  table: a flat list of p, g, m, v addresses and
+    element count per tensor; the caller has checked what adam_step checks."""
+    if table:
+        words = array.array("Q", table)
+        with _on(device):
+            _call("pam_hip_adam_step_many", words.buffer_info()[0], len(table) // 5, float(beta1), float(one_minus_beta1),
+                  float(beta2), float(one_minus_beta2), float(eps), float(decay or 0.0), int(bool(decay)), float(step_size),
+                  float(offset), _stream())
 
 
 def _conv_geometry(X, W, stride, padding, groups=1):

@@ -9,6 +9,10 @@
 // 12 B/element for the pa_exp/pa_log backwards.
 #include <math.h>
 
+#include <algorithm>
+#include <vector>
+
+#include "../../include/pam_hip_extra.h"
 #include "pam_common.h"
 #include "pam_device.h"
 
@@ -340,44 +344,93 @@ __device__ __forceinline__ void adam_vector(v4f& pp, const v4f& gg, v4f& mm, v4f
 }
 
 constexpr int kAdamVectors = 2;               // 128-bit vectors per lane and stream (four measured the same)
-__global__ __launch_bounds__(kThreads) void adam_vec_kernel(v4f* __restrict__ p, const v4f* __restrict__ g,
-                                                           v4f* __restrict__ m, v4f* __restrict__ v, size_t nvec, AdamArgs a)
+constexpr unsigned kAdamChunk = 4 * kAdamVectors * kThreads;        // parameters per work-group
+
+// The update of many parameter tensors in one launch.  A transformer's parameters are hundreds of tensors, most of them a
+// few hundred values: one launch each was 253 launches of 3 us at least behind 8 us of host work apiece, where the bytes of all
+// of them take 0.2 ms.  The table of tensors travels in the kernel's arguments (no copy to wait for); a work-group takes
+// kAdamChunk consecutive parameters of one tensor and finds which by a binary search over the tensors' first work-groups
+// on the scalar unit.  Bound by memory: 28 B per parameter.
+constexpr int kAdamTensors = 96;              // 40 bytes each: the arguments stay below 4 KB
+struct AdamMany {
+    float* p[kAdamTensors]; const float* g[kAdamTensors]; float* m[kAdamTensors]; float* v[kAdamTensors];
+    unsigned n[kAdamTensors];                 // parameters of the tensor
+    unsigned first[kAdamTensors];             // its first work-group; past the last tensor: all ones
+    AdamArgs a;
+};
+static_assert(sizeof(AdamMany) <= 4096, "kernel arguments");
+typedef const __attribute__((address_space(4))) AdamMany* AdamTable;
+
+__global__ __launch_bounds__(kThreads) void adam_many_kernel(AdamMany)
 {
-    // work-group b takes kAdamVectors x kThreads consecutive vectors: lane t the vectors t, t + kThreads, ... of them
-    const size_t first = (size_t)blockIdx.x * (kAdamVectors * kThreads) + threadIdx.x;
-    if (first + (kAdamVectors - 1) * kThreads < nvec) {
+    // (read where they are: a run-time index into a by-value argument would copy the table to scratch memory)
+    const AdamTable t = (AdamTable)__builtin_amdgcn_kernarg_segment_ptr();
+    int at = 0;
+#pragma unroll
+    for (int half = 64; half >= 1; half >>= 1)
+        if (at + half < kAdamTensors && t->first[at + half] <= blockIdx.x) at += half;
+    float* p = t->p[at]; const float* g = t->g[at]; float* m = t->m[at]; float* v = t->v[at];
+    const unsigned n = t->n[at], begin = (blockIdx.x - t->first[at]) * kAdamChunk;
+    AdamArgs a;
+    a.beta1 = t->a.beta1; a.one_minus_beta1 = t->a.one_minus_beta1; a.beta2 = t->a.beta2; a.one_minus_beta2 = t->a.one_minus_beta2;
+    a.eps = t->a.eps; a.decay = t->a.decay; a.step_size = t->a.step_size; a.off = t->a.off;
+    a.has_decay = t->a.has_decay; a.has_off = t->a.has_off;
+    const unsigned left = n - begin;          // at least 1
+    p += begin; g += begin; m += begin; v += begin;
+    const bool aligned = (((uintptr_t)p | (uintptr_t)g | (uintptr_t)m | (uintptr_t)v) & 15u) == 0;
+    if (aligned && left >= kAdamChunk) {
         v4f pp[kAdamVectors], gg[kAdamVectors], mm[kAdamVectors], vv[kAdamVectors];
 #pragma unroll
         for (int u = 0; u < kAdamVectors; ++u) {
-            const size_t i = first + (size_t)u * kThreads;
-            pp[u] = __builtin_nontemporal_load(p + i); gg[u] = __builtin_nontemporal_load(g + i);
-            mm[u] = __builtin_nontemporal_load(m + i); vv[u] = __builtin_nontemporal_load(v + i);
+            const unsigned i = threadIdx.x + u * kThreads;
+            pp[u] = __builtin_nontemporal_load((const v4f*)p + i); gg[u] = __builtin_nontemporal_load((const v4f*)g + i);
+            mm[u] = __builtin_nontemporal_load((const v4f*)m + i); vv[u] = __builtin_nontemporal_load((const v4f*)v + i);
         }
 #pragma unroll
         for (int u = 0; u < kAdamVectors; ++u) {
-            const size_t i = first + (size_t)u * kThreads;
+            const unsigned i = threadIdx.x + u * kThreads;
             adam_vector(pp[u], gg[u], mm[u], vv[u], a);
-            __builtin_nontemporal_store(pp[u], p + i); __builtin_nontemporal_store(mm[u], m + i); __builtin_nontemporal_store(vv[u], v + i);
+            __builtin_nontemporal_store(pp[u], (v4f*)p + i); __builtin_nontemporal_store(mm[u], (v4f*)m + i);
+            __builtin_nontemporal_store(vv[u], (v4f*)v + i);
         }
-    } else {
-        for (size_t i = first; i < nvec; i += kThreads) {
-            v4f p0 = p[i], g0 = g[i], m0 = m[i], v0 = v[i];
-            adam_vector(p0, g0, m0, v0, a);
-            p[i] = p0; m[i] = m0; v[i] = v0;
-        }
+        return;
+    }
+    // a tensor's last work-group, or tensors off 16-byte boundaries
+    const unsigned here = left < kAdamChunk ? left : kAdamChunk, vectors = aligned ? here / 4 : 0;
+    for (unsigned i = threadIdx.x; i < vectors; i += kThreads) {
+        v4f p0 = ((v4f*)p)[i], g0 = ((const v4f*)g)[i], m0 = ((v4f*)m)[i], v0 = ((v4f*)v)[i];
+        adam_vector(p0, g0, m0, v0, a);
+        ((v4f*)p)[i] = p0; ((v4f*)m)[i] = m0; ((v4f*)v)[i] = v0;
+    }
+    for (unsigned i = vectors * 4 + threadIdx.x; i < here; i += kThreads) {
+        float p0 = p[i], m0 = m[i], v0 = v[i];
+        adam_one(p0, g[i], m0, v0, a);
+        p[i] = p0; m[i] = m0; v[i] = v0;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void adam_scalar_kernel(float* __restrict__ p, const float* __restrict__ g,
-                                                              float* __restrict__ m, float* __restrict__ v,
-                                                              size_t first, size_t n, AdamArgs a)
+// Whether some tensor's written memory (p, m, v) is also another buffer of the list: such tensors are updated one launch
+// after the other.
+bool adam_buffers_overlap(const pam_hip_adam_tensor* t, long count)
 {
-    const size_t step = (size_t)gridDim.x * kThreads;
-    for (size_t i = first + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += step) {
-        float pp = p[i], mm = m[i], vv = v[i];
-        adam_one(pp, g[i], mm, vv, a);
-        p[i] = pp; m[i] = mm; v[i] = vv;
+    struct Range { uintptr_t begin, end; bool written; };
+    std::vector<Range> r;
+    r.reserve((size_t)count * 4);
+    for (long i = 0; i < count; ++i) {
+        const size_t bytes = t[i].n * sizeof(float);
+        r.push_back({(uintptr_t)t[i].p, (uintptr_t)t[i].p + bytes, true});
+        r.push_back({(uintptr_t)t[i].g, (uintptr_t)t[i].g + bytes, false});
+        r.push_back({(uintptr_t)t[i].m, (uintptr_t)t[i].m + bytes, true});
+        r.push_back({(uintptr_t)t[i].v, (uintptr_t)t[i].v + bytes, true});
     }
+    std::sort(r.begin(), r.end(), [](const Range& a, const Range& b) { return a.begin < b.begin; });
+    uintptr_t any = 0, written = 0;           // the furthest end of the ranges so far
+    for (const Range& x : r) {
+        if (x.begin < written || (x.written && x.begin < any)) return true;
+        any = std::max(any, x.end);
+        if (x.written) written = std::max(written, x.end);
+    }
+    return false;
 }
 
 }  // namespace
@@ -463,29 +516,50 @@ int pam_hip_pow_bwd(const float* x, const float* dy, float* dx, size_t n, float 
                                OpPowBwd{exponent, offset, offset != 1.0f, approx_a != 0, approx_exp != 0}, stream);
 }
 
+int pam_hip_adam_step_many(const pam_hip_adam_tensor* tensors, long count, float beta1, float one_minus_beta1, float beta2,
+                           float one_minus_beta2, float eps, float decay, int has_decay, float step_size, float offset, void* stream)
+try {
+    if (count < 0 || (count > 0 && !tensors)) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step_many: null table or negative count");
+    size_t blocks = 0;
+    for (long i = 0; i < count; ++i) {
+        const pam_hip_adam_tensor& t = tensors[i];
+        if (t.n == 0) continue;
+        if (!t.p || !t.g || !t.m || !t.v) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step: null pointer");
+        if (t.n > (size_t)1 << 41) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step: more than 2^41 parameters");
+    }
+    const bool apart = count > 1 && adam_buffers_overlap(tensors, count);
+    AdamMany table;
+    table.a = AdamArgs{beta1, one_minus_beta1, beta2, one_minus_beta2, eps, decay, step_size, offset, has_decay != 0, offset != 1.0f};
+    int held = 0;
+    auto flush = [&]() -> int {
+        if (held == 0) return PAM_HIP_OK;
+        for (int i = held; i < kAdamTensors; ++i) table.first[i] = ~0u;
+        hipLaunchKernelGGL(adam_many_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, table);
+        held = 0; blocks = 0;
+        return pamhost::check_launch("adam_step");
+    };
+    // (a tensor of more than kPart values enters the table in parts, so that counts and indexes are 32-bit ones)
+    constexpr size_t kPart = (size_t)1 << 31;
+    static_assert(kPart % kAdamChunk == 0, "parts are whole chunks");
+    for (long i = 0; i < count; ++i) {
+        for (size_t at = 0; at < tensors[i].n; at += kPart) {
+            const size_t n = std::min(kPart, tensors[i].n - at), need = (n + kAdamChunk - 1) / kAdamChunk;
+            if (held == kAdamTensors || blocks + need > ((size_t)1 << 30)) { const int rc = flush(); if (rc != PAM_HIP_OK) return rc; }
+            table.p[held] = tensors[i].p + at; table.g[held] = tensors[i].g + at; table.m[held] = tensors[i].m + at; table.v[held] = tensors[i].v + at;
+            table.n[held] = (unsigned)n; table.first[held] = (unsigned)blocks;
+            ++held; blocks += need;
+        }
+        if (apart) { const int rc = flush(); if (rc != PAM_HIP_OK) return rc; }
+    }
+    return flush();
+} catch (...) { return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step: out of host memory"); }
+
 int pam_hip_adam_step(float* p, const float* g, float* m, float* v, size_t n, float beta1, float one_minus_beta1,
                       float beta2, float one_minus_beta2, float eps, float decay, int has_decay, float step_size,
                       float offset, void* stream)
 {
-    if (n == 0) return PAM_HIP_OK;
-    if (!p || !g || !m || !v) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step: null pointer");
-    AdamArgs a{beta1, one_minus_beta1, beta2, one_minus_beta2, eps, decay, step_size, offset, has_decay != 0, offset != 1.0f};
-    hipStream_t st = (hipStream_t)stream;
-    uintptr_t align = (uintptr_t)p | (uintptr_t)g | (uintptr_t)m | (uintptr_t)v;
-    size_t nvec = (align & 15u) ? 0 : n / 4;
-    const size_t cap = (size_t)1 << 30;
-    if (nvec) {
-        const size_t blocks = (nvec + kAdamVectors * kThreads - 1) / (kAdamVectors * kThreads);
-        if (blocks > cap) return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "adam_step: more than 2^41 parameters");
-        hipLaunchKernelGGL(adam_vec_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, (v4f*)p, (const v4f*)g, (v4f*)m,
-                           (v4f*)v, nvec, a);
-    }
-    if (nvec * 4 < n) {
-        size_t blocks = (n - nvec * 4 + kThreads - 1) / kThreads;
-        if (blocks > cap) blocks = cap;
-        hipLaunchKernelGGL(adam_scalar_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, p, g, m, v, nvec * 4, n, a);
-    }
-    return pamhost::check_launch("adam_step");
+    const pam_hip_adam_tensor t{p, g, m, v, n};
+    return pam_hip_adam_step_many(&t, 1, beta1, one_minus_beta1, beta2, one_minus_beta2, eps, decay, has_decay, step_size, offset, stream);
 }
 
 }  // extern "C"

@@ -4,8 +4,8 @@ fully multiplication-free training recipe (the `Adam` class of
 submodules/fairseq/fairseq/optim/adam.py:113-254 in the reference tree, selected there by
 `opt_functional_cfg`).
 
-With a PAM table and fp32 GPU tensors the whole update of a parameter is one kernel
-(28 B/element instead of eleven elementwise launches); with any other table, or tensors
+With a PAM table and fp32 GPU tensors the update of all parameters is one kernel over a table of
+them (28 B/element instead of eleven elementwise launches each); with any other table, or tensors
 the kernel does not take, the same formulas run op by op through the table.  Both paths
 give identical bits: the update has no reductions.
 """
@@ -66,53 +66,103 @@ class Adam(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        ops = self.op_dict
-        for group in self.param_groups:
-            beta1, beta2 = group["betas"]
-            for p in group["params"]:
-                if p.grad is None:
-                    continue
-                grad = p.grad.data
-                if grad.dtype in (torch.float16, torch.bfloat16):
-                    grad = grad.float()
-                if grad.is_sparse:
-                    raise RuntimeError("Adam does not support sparse gradients, please consider SparseAdam instead")
-                assert not group.get("amsgrad", False), "Not supported"
-                half = p.data.dtype in (torch.float16, torch.bfloat16)
-                p32 = p.data.float() if half else p.data
-
-                state = self.state[p]
-                if len(state) == 0:
-                    state["step"] = 0
-                    state["exp_avg"] = torch.zeros_like(p32)
-                    state["exp_avg_sq"] = torch.zeros_like(p32)
-                else:
-                    state["exp_avg"] = state["exp_avg"].to(p32)
-                    state["exp_avg_sq"] = state["exp_avg_sq"].to(p32)
-                exp_avg, exp_avg_sq = state["exp_avg"], state["exp_avg_sq"]
-                state["step"] += 1
-
-                # scalar work on the host, in double precision
-                correction1 = 1 - beta1 ** state["step"]
-                correction2 = 1 - beta2 ** state["step"]
-                step_size = group["lr"] * math.sqrt(correction2) / correction1
-                decay = group["weight_decay"] * group["lr"] if group["weight_decay"] != 0 else None
-
-                if (self.fused and p32.is_cuda and p32.dtype == torch.float32 and grad.dtype == torch.float32
-                        and all(t.is_contiguous() for t in (p32, grad, exp_avg, exp_avg_sq))):
-                    _abi.adam_step(p32, grad, exp_avg, exp_avg_sq, beta1, 1 - beta1, beta2, 1 - beta2, group["eps"],
-                                   decay, step_size, 1.0 if self.offset is None else self.offset)
-                else:
-                    exp_avg.copy_(ops["mul"](exp_avg, beta1) + ops["mul"](grad, 1 - beta1))
-                    exp_avg_sq.copy_(ops["mul"](exp_avg_sq, beta2))
-                    exp_avg_sq += ops["mul"](ops["mul"](grad, grad), 1 - beta2)
-                    denom = ops["pow"](exp_avg_sq, 0.5) + group["eps"]
-                    if decay is not None:
-                        p32 -= ops["mul"](p32, decay)
-                    p32 -= ops["mul"](ops["div"](exp_avg, denom), step_size)
-                if half:
-                    p.data.copy_(p32)
+        batch = _Batch(1.0 if self.offset is None else self.offset)
+        try:
+            for group in self.param_groups:
+                for p in group["params"]:
+                    if p.grad is not None and not (self.fused and self._add_to(batch, group, p)):
+                        batch.flush()                  # parameters are updated in their order
+                        self._update(group, p)
+        finally:
+            batch.flush()                              # also those before one that raised
         return loss
+
+    def _add_to(self, batch, group, p):
+        """Enters a parameter with moments into the batch that one kernel updates, if p, its gradient and moments are
+        contiguous fp32 tensors of one shape on one GPU; else returns False and changes nothing."""
+        state = self.state.get(p)
+        if not state or group.get("amsgrad", False):
+            return False
+        grad, exp_avg, exp_avg_sq, shape, device = p.grad, state["exp_avg"], state["exp_avg_sq"], p.shape, p.device
+        if device.type != "cuda":
+            return False
+        for t in (p, grad, exp_avg, exp_avg_sq):
+            if t.dtype is not torch.float32 or t.device != device or t.shape != shape or t.is_sparse or not t.is_contiguous():
+                return False
+        state["step"] += 1
+        batch.add(group, state["step"], device, (p.data_ptr(), grad.data_ptr(), exp_avg.data_ptr(), exp_avg_sq.data_ptr(), p.numel()))
+        return True
+
+    def _update(self, group, p):
+        """One parameter by itself, by the single-tensor kernel or op by op."""
+        ops = self.op_dict
+        beta1, beta2 = group["betas"]
+        grad = p.grad.data
+        if grad.dtype in (torch.float16, torch.bfloat16):
+            grad = grad.float()
+        if grad.is_sparse:
+            raise RuntimeError("Adam does not support sparse gradients, please consider SparseAdam instead")
+        assert not group.get("amsgrad", False), "Not supported"
+        half = p.data.dtype in (torch.float16, torch.bfloat16)
+        p32 = p.data.float() if half else p.data
+
+        state = self.state[p]
+        if len(state) == 0:
+            state["step"] = 0
+            state["exp_avg"] = torch.zeros_like(p32)
+            state["exp_avg_sq"] = torch.zeros_like(p32)
+        else:
+            state["exp_avg"] = state["exp_avg"].to(p32)
+            state["exp_avg_sq"] = state["exp_avg_sq"].to(p32)
+        exp_avg, exp_avg_sq = state["exp_avg"], state["exp_avg_sq"]
+        state["step"] += 1
+        decay, step_size = _step_scalars(group, state["step"])
+
+        if (self.fused and p32.is_cuda and p32.dtype == torch.float32 and grad.dtype == torch.float32
+                and all(t.is_contiguous() for t in (p32, grad, exp_avg, exp_avg_sq))):
+            _abi.adam_step(p32, grad, exp_avg, exp_avg_sq, beta1, 1 - beta1, beta2, 1 - beta2, group["eps"],
+                           decay, step_size, 1.0 if self.offset is None else self.offset)
+        else:
+            exp_avg.copy_(ops["mul"](exp_avg, beta1) + ops["mul"](grad, 1 - beta1))
+            exp_avg_sq.copy_(ops["mul"](exp_avg_sq, beta2))
+            exp_avg_sq += ops["mul"](ops["mul"](grad, grad), 1 - beta2)
+            denom = ops["pow"](exp_avg_sq, 0.5) + group["eps"]
+            if decay is not None:
+                p32 -= ops["mul"](p32, decay)
+            p32 -= ops["mul"](ops["div"](exp_avg, denom), step_size)
+        if half:
+            p.data.copy_(p32)
+
+
+def _step_scalars(group, step):
+    """(decay or None, step size): scalar work on the host, in double precision."""
+    beta1, beta2 = group["betas"]
+    correction1 = 1 - beta1 ** step
+    correction2 = 1 - beta2 ** step
+    decay = group["weight_decay"] * group["lr"] if group["weight_decay"] != 0 else None
+    return decay, group["lr"] * math.sqrt(correction2) / correction1
+
+
+class _Batch:
+    """The tensors of a step that one call updates: consecutive parameters of one group, step count and device."""
+
+    def __init__(self, offset):
+        self.offset, self.key, self.table = offset, None, []
+
+    def add(self, group, step, device, entry):
+        key = (id(group), step, device)
+        if key != self.key:
+            self.flush()
+            self.key, self.group = key, group
+        self.table.extend(entry)
+
+    def flush(self):
+        table, self.table = self.table, []
+        if table:
+            group, (_, step, device) = self.group, self.key
+            beta1, beta2 = group["betas"]
+            decay, step_size = _step_scalars(group, step)
+            _abi.adam_step_many(table, device, beta1, 1 - beta1, beta2, 1 - beta2, group["eps"], decay, step_size, self.offset)
 
 
 def multiply_grads(params, c, op_dict):

@@ -162,3 +162,56 @@ def test_multiply_grads_keeps_dense_gradients_like_the_reference():
     calls = []
     multiply_grads([p, q], 0.5, {"mul": lambda a, b: calls.append((a.clone(), b)) or a * b})
     assert len(calls) == 1 and calls[0][1] == 0.5 and torch.equal(p.grad, torch.full((4,), 3.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [None, OFF])
+def test_gpu_step_over_many_tensors(oracle, off):
+    """One call over a table of tensors: sizes around the kernel's chunks of 2048 values and its 128-bit vectors, more
+    tensors than one launch takes (96), some off 16-byte boundaries; each as the oracle updates it alone."""
+    sizes = [1, 3, 4, 2047, 2048, 2049, 4096, 4099, 6145] + [5 + 3 * i for i in range(100)]
+    data = [tuple(t[12:] for t in operands(n + 12, 7 + i)) if i % 2 else tuple(t[:n] for t in operands(n + 12, 7 + i))
+            for i, n in enumerate(sizes)]
+    step_size = 5e-4 * math.sqrt(1 - 0.98 ** 2) / (1 - 0.9 ** 2)
+    args = (0.9, 0.1, 0.98, 0.02, 1e-8, 3e-7, step_size)
+    tensors, table = [], []
+    for i, arrays in enumerate(data):
+        n = len(arrays[0])
+        shift = 1 if i % 5 == 4 else 0                     # unaligned
+        views = [torch.zeros(n + 4, device="cuda")[shift:shift + n] for _ in range(4)]
+        for view, a in zip(views, arrays):
+            view.copy_(torch.from_numpy(a))
+        tensors.append(views)
+        table += [t.data_ptr() for t in views] + [n]
+    pam_amd._abi.adam_step_many(table, tensors[0][0].device, *args, 1.0 if off is None else off)
+    for (tp, tg, tm, tv), (p, g, m, v) in zip(tensors, data):
+        want = oracle.adam_step(p, g, m, v, *args, off)
+        for got, w, name in zip((tp, tm, tv), want, ("p", "exp_avg", "exp_avg_sq")):
+            assert_same_bits(got.cpu().numpy(), w, f"{name} n={len(p)}")
+
+
+@pytest.mark.gpu
+def test_gpu_step_with_shared_and_mixed_parameters():
+    """Parameters that share memory are updated one after the other, half-precision and first-step ones by themselves
+    in their place, and an error in one leaves those before it updated: as a loop over the parameters does."""
+    g = torch.Generator().manual_seed(5)
+    results = []
+    for together in (True, False):
+        g.manual_seed(5)
+        base = torch.randn(5000, generator=g).cuda()
+        params = [torch.nn.Parameter(base[:3000]), torch.nn.Parameter(base[1000:4000]), torch.nn.Parameter(base[4000:].clone()),
+                  torch.nn.Parameter(torch.randn(64, generator=g).cuda().bfloat16()), torch.nn.Parameter(torch.randn(7, generator=g).cuda())]
+        opt = optim.Adam(params, lr=5e-4, betas=(0.9, 0.98), weight_decay=1e-4, opt_functional_cfg="pam")
+        opt.fused = together
+        for _ in range(3):
+            for p in params:
+                p.grad = (torch.randn(p.shape, generator=g) * 1e-2).cuda().to(p.dtype)
+            opt.step()
+        before = params[4].detach().clone()
+        opt.param_groups[0]["amsgrad"] = True
+        with pytest.raises(AssertionError):
+            opt.step()
+        assert torch.equal(params[4], before) and opt.state[params[0]]["step"] == 3
+        results.append([base.cpu().numpy()] + [p.detach().float().cpu().numpy() for p in params])
+    for a, b in zip(*results):
+        assert_same_bits(a, b, "together vs one by one")
