@@ -25,6 +25,12 @@ int pam_hip_adam_step_many(const pam_hip_adam_tensor *tensors, long count, float
                            float one_minus_beta2, float eps, float decay, int has_decay, float step_size, float offset,
                            void *stream);
 
+/* a_sums[j] = sum over i of a[i * a_row_stride + j], j < n, and the same for a second matrix of that shape unless b_sums is
+ * NULL: ordinary float32 additions in a fixed tree. */
+size_t pam_hip_column_sums_workspace_bytes(long rows, long n, int matrices);
+int pam_hip_column_sums(const float *a, long a_row_stride, float *a_sums, const float *b, long b_row_stride, float *b_sums,
+                        long rows, long n, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -73,6 +73,8 @@ _SIGNATURES = {
 # include/pam_hip_extra.h
 _EXTRA_SIGNATURES = {
     "pam_hip_logsumexp_fwd_finite": ([_p, _p, _p, _p, _l, _l, _f, _p, _p, _p, _z, _p], _i),
+    "pam_hip_column_sums_workspace_bytes": ([_l, _l, _i], _z),
+    "pam_hip_column_sums": ([_p, _l, _p, _p, _l, _p, _l, _l, _p, _z, _p], _i),
     "pam_hip_adam_step_many": ([_p, _l, _f, _f, _f, _f, _f, _f, _i, _f, _f, _p], _i),
 }
 
@@ -548,6 +550,20 @@ def adam_step_many(table, device, beta1, one_minus_beta1, beta2, one_minus_beta2
             _call("pam_hip_adam_step_many", words.buffer_info()[0], len(table) // 5, float(beta1), float(one_minus_beta1),
                   float(beta2), float(one_minus_beta2), float(eps), float(decay or 0.0), int(bool(decay)), float(step_size),
                   float(offset), _stream())
+
+
+def column_sums(A, B=None):
+    """A.sum(0), or (A.sum(0), B.sum(0)) of two matrices of one shape: fp32 GPU matrices whose rows are contiguous."""
+    rows, n = A.shape
+    a_sums = torch.empty(n, dtype=torch.float32, device=A.device)
+    b_sums = None if B is None else torch.empty(n, dtype=torch.float32, device=A.device)
+    with _on(A.device):
+        nbytes = load_library().pam_hip_column_sums_workspace_bytes(rows, n, 1 if B is None else 2)
+        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=A.device) if nbytes else None
+        _call("pam_hip_column_sums", A.data_ptr(), A.stride(0), a_sums.data_ptr(), None if B is None else B.data_ptr(),
+              0 if B is None else B.stride(0), None if B is None else b_sums.data_ptr(), rows, n,
+              None if ws is None else ws.data_ptr(), nbytes, _stream())
+    return a_sums if B is None else (a_sums, b_sums)
 
 
 def _conv_geometry(X, W, stride, padding, groups=1):

@@ -138,6 +138,16 @@ def mean_last(x, keepdim, offset=None):
     return y.view(x.shape[:-1] + ((1,) if keepdim else ()))
 
 
+def _summable(t):
+    """Whether the sum over the rows of t runs on the kernel: not where autograd is to record it (a gradient's gradient)."""
+    return (t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.numel() > 0
+            and not (t.requires_grad and torch.is_grad_enabled()))
+
+
+def _sum_rows(t):
+    return _abi.column_sums(t) if _summable(t) else t.sum(0)
+
+
 class layer_norm_autograd(torch.autograd.Function):
     """layer_norm over the last n values of each row; weight and bias of n values or None."""
 
@@ -159,8 +169,12 @@ class layer_norm_autograd(torch.autograd.Function):
         want_w = w is not None and ctx.needs_input_grad[1]
         dx, terms = row_kernels.layer_norm_bwd(rows, w, g, ctx.eps, ctx.offset, *_flags(ctx.approx_bwd), want_w)
         # the broadcast weight and bias collect their gradients by a sum over the rows, as autograd's expand does
-        dw = terms.sum(0) if want_w else None
-        db = g.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
+        want_b = ctx.has_bias and ctx.needs_input_grad[2]
+        if want_w and want_b and _summable(g):
+            dw, db = _abi.column_sums(terms, g)
+        else:
+            dw = _sum_rows(terms) if want_w else None
+            db = _sum_rows(g) if want_b else None
         return dx, dw, db, None, None, None
 
 
@@ -298,8 +312,24 @@ class linear_autograd(torch.autograd.Function):
             dB = k.pam_matmul_fwd(At, dY2, At_rm, dY_rm, off) if approx_b else k.pam_matmul_bwd(At, dY2, B, At_rm, dY_rm, False, off)
             dW = dB.t()
         if ctx.needs_input_grad[2]:
-            db = dY2.sum(0)
+            db = _sum_rows(dY2)
         return dX, dW, db, None, None
+
+
+class add_bias_autograd(torch.autograd.Function):
+    """rows + bias, with the bias gradient that linear_autograd forms."""
+
+    @staticmethod
+    def forward(ctx, rows, bias):
+        return rows + bias
+
+    @staticmethod
+    def backward(ctx, g):
+        return g, _sum_rows(g) if ctx.needs_input_grad[1] else None
+
+
+def add_bias(rows, bias):
+    return add_bias_autograd.apply(rows, bias)
 
 
 def linear_with_bias(X2d, W, bias, offset=None, approx_bwd=False):

@@ -658,3 +658,21 @@ def test_nonfinite_input_is_refused_and_the_largest_finite_one_is_not(rows, n):
         side.synchronize()
     y = pam_amd.log_softmax(x, dim=-1)                    # and a refused call leaves nothing behind
     assert torch.equal(y, pam_amd.log_softmax(x, dim=-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n", [(1, 1), (2, 4), (127, 64), (128, 68), (257, 63), (300, 192), (4097, 20), (12608, 768), (70001, 3), (3, 30011)])
+def test_column_sums(rows, n):
+    """Sums over the rows against 64-bit ones, on both load widths, on rows apart from each other and for two matrices in
+    one call.  A value takes part in at most 64 + 4 + 128 + 4 rounded additions at these sizes (a lane's chain and the tree,
+    twice), each off by 2^-24 of a partial sum that is at most the sum of magnitudes."""
+    from pam_amd import _abi
+    g = torch.Generator().manual_seed(rows + n)
+    a, b = (torch.randn(rows, n, generator=g).cuda() for _ in range(2))
+    apart = torch.randn(rows, n + 5, generator=g).cuda()[:, 1:n + 1]
+    sums = [_abi.column_sums(a), *_abi.column_sums(b, a), _abi.column_sums(apart), *_abi.column_sums(a, apart)]
+    for got, t in zip(sums, (a, b, a, apart, a, apart)):
+        t64 = t.cpu().double()
+        bound = 200 * 2.0 ** -24 * t64.abs().sum(0)
+        assert ((got.cpu().double() - t64.sum(0)).abs() <= bound).all()
+    assert torch.equal(sums[0], sums[2]) or rows > 128          # cut alike where nothing is cut
