@@ -7,6 +7,7 @@ stream only.  There is no CPU fallback: a missing library or a non-GPU tensor ra
 """
 import array
 import ctypes
+import importlib.util
 import pathlib
 import threading
 
@@ -104,6 +105,24 @@ def load_library():
     return _lib
 
 
+_HOST_PATH = _LIB_PATH.with_name("_pam_host.so")
+_host = None
+
+
+def host():
+    """The ops' host path in C++ (csrc/pam_host.cpp); raises if it has not been built."""
+    global _host
+    if _host is None:
+        load_library()
+        if not _HOST_PATH.exists():
+            raise RuntimeError(f"{_HOST_PATH} is missing: build the HIP extension first (python -m pam_amd.build).")
+        spec = importlib.util.spec_from_file_location("_pam_host", str(_HOST_PATH))
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def exported_symbols():
     return sorted(_SIGNATURES)
 
@@ -130,22 +149,6 @@ def gemm_plan(batch, m, n, k):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-
-# The matrix products' scratch (pieces of cut tiles, their arrival words): one buffer per device and stream, kept and
-# grown as needed.  Products on one stream run one after the other, and each leaves the arrival words ready for the
-# next one; products on different streams may overlap in time and must not share a buffer.
-_workspaces = {}
-
-
-def _gemm_workspace(device, nbytes):
-    """Called with `device` current."""
-    key = (device.index, _stream())
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() * 4 < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20) // 4 + 64, dtype=torch.float32, device=device)
-        _workspaces[key] = ws
-    return ws
-
 
 def _stream():
     """The current device's current stream as a hipStream_t value."""
@@ -315,57 +318,33 @@ class HipKernels:
 
     # ---------------------------------------------------------------- matrix products
     @staticmethod
-    def _mat(t, batched):
-        s = t.stride()
-        return (t.data_ptr(), s[0], s[1], s[2]) if batched else (t.data_ptr(), s[0], s[1])
-
-    @classmethod
-    def _product(cls, name, batched, L, R, Mop, extra, offset):
-        ops = (L, R) if Mop is None else (L, R, Mop)
+    def _product(kind, batched, L, R, M, delta_L, offset):
+        """kind: 0 PAM products, 1 ordinary ones, 2 those of the exact gradient for M."""
+        ops = (L, R) if M is None else (L, R, M)
         _check(*ops)
         nd = 3 if batched else 2
         if any(t.dim() != nd for t in ops):
-            raise ValueError(f"{name}: expected {nd}-D operands")
-        if L.shape[-1] != R.shape[-2] or (batched and L.shape[0] != R.shape[0]):
-            raise ValueError(f"{name}: shapes {tuple(L.shape)} and {tuple(R.shape)} do not multiply")
-        batch = L.shape[0] if batched else 1
-        m, k, n = L.shape[-2], L.shape[-1], R.shape[-1]
-        if Mop is not None and tuple(Mop.shape[-2:]) != (m, n):
-            raise ValueError(f"{name}: third operand must have the shape of the result")
-        out = torch.empty((batch, m, n) if batched else (m, n), dtype=torch.float32, device=L.device)
-        if out.numel() == 0:
-            return out
-        with _on(L.device):
-            lib = load_library()
-            ws_bytes = lib.pam_hip_gemm_workspace_bytes(batch, m, n, k)
-            ws = _gemm_workspace(L.device, ws_bytes) if ws_bytes else None
-            args = []
-            for t in ops:
-                args += cls._mat(t, batched)
-            args += cls._mat(out, batched)
-            args += ([batch] if batched else []) + [m, n, k] + extra + [float(offset)]
-            args += [ws.data_ptr() if ws is not None else None, ws_bytes, _stream()]
-            _call(f"pam_hip_{name}", *args)
-        return out
+            raise ValueError(f"matrix product: expected {nd}-D operands")
+        return host().product(kind, L, R, M, delta_L, None, float(offset))
 
     def pam_matmul_fwd(self, A, B, A_row_major, B_row_major, offset):
         # the layout flags of the reference select a kernel instance there; here the strides do
-        return self._product("pam_matmul_fwd", False, A, B, None, [], offset)
+        return self._product(0, False, A, B, None, False, offset)
 
     def pam_bmm_fwd(self, A, B, A_row_major, B_row_major, offset):
-        return self._product("pam_bmm_fwd", True, A, B, None, [], offset)
+        return self._product(0, True, A, B, None, False, offset)
 
     def standard_matmul(self, A, B, A_row_major, B_row_major, offset):
-        return self._product("standard_matmul", False, A, B, None, [], offset)
+        return self._product(1, False, A, B, None, False, offset)
 
     def standard_bmm(self, A, B, A_row_major, B_row_major, offset):
-        return self._product("standard_bmm", True, A, B, None, [], offset)
+        return self._product(1, True, A, B, None, False, offset)
 
     def pam_matmul_bwd(self, L, R, M, L_row_major, R_row_major, delta_L, offset):
-        return self._product("pam_matmul_bwd", False, L, R, M, [int(bool(delta_L))], offset)
+        return self._product(2, False, L, R, M, bool(delta_L), offset)
 
     def pam_bmm_bwd(self, L, R, M, L_row_major, R_row_major, delta_L, offset):
-        return self._product("pam_bmm_bwd", True, L, R, M, [int(bool(delta_L))], offset)
+        return self._product(2, True, L, R, M, bool(delta_L), offset)
 
 
 class HipRowKernels:
@@ -542,28 +521,19 @@ def adam_step(p, g, m, v, beta1, one_minus_beta1, beta2, one_minus_beta2, eps, d
 
 
 def adam_step_many(table, device, beta1, one_minus_beta1, beta2, one_minus_beta2, eps, decay, step_size, offset):
-    """adam_step for many tensors on `device` with the same scalars.  table: a flat list of p, g, m, v addresses and
-    element count per tensor; the caller has checked what adam_step checks."""
+    """adam_step for many tensors on `device` with the same scalars.  table: p, g, m, v addresses and element count per
+    tensor, as 64-bit words (bytes) or a flat list of numbers; the caller has checked what adam_step checks."""
     if table:
-        words = array.array("Q", table)
+        words = table if isinstance(table, bytes) else array.array("Q", table).tobytes()
         with _on(device):
-            _call("pam_hip_adam_step_many", words.buffer_info()[0], len(table) // 5, float(beta1), float(one_minus_beta1),
+            _call("pam_hip_adam_step_many", words, len(words) // 40, float(beta1), float(one_minus_beta1),
                   float(beta2), float(one_minus_beta2), float(eps), float(decay or 0.0), int(bool(decay)), float(step_size),
                   float(offset), _stream())
 
 
 def column_sums(A, B=None):
     """A.sum(0), or (A.sum(0), B.sum(0)) of two matrices of one shape: fp32 GPU matrices whose rows are contiguous."""
-    rows, n = A.shape
-    a_sums = torch.empty(n, dtype=torch.float32, device=A.device)
-    b_sums = None if B is None else torch.empty(n, dtype=torch.float32, device=A.device)
-    with _on(A.device):
-        nbytes = load_library().pam_hip_column_sums_workspace_bytes(rows, n, 1 if B is None else 2)
-        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=A.device) if nbytes else None
-        _call("pam_hip_column_sums", A.data_ptr(), A.stride(0), a_sums.data_ptr(), None if B is None else B.data_ptr(),
-              0 if B is None else B.stride(0), None if B is None else b_sums.data_ptr(), rows, n,
-              None if ws is None else ws.data_ptr(), nbytes, _stream())
-    return a_sums if B is None else (a_sums, b_sums)
+    return host().column_sums(A, B)
 
 
 def _conv_geometry(X, W, stride, padding, groups=1):
@@ -622,23 +592,3 @@ def conv2d_bwd_input(dY, W, X, padding, exact, offset, groups=1):
             _call("pam_hip_conv2d_bwd_input", dY.data_ptr(), W.data_ptr(), X.data_ptr(), dX.data_ptr(), *geo,
                   int(bool(exact)), float(offset), ws.data_ptr(), nbytes, _stream())
     return dX
-
-
-def linear_fwd(X, Wt, bias, offset):
-    """X[m, k] (x) Wt[k, n] + bias[n] in one pass (any strides for X and Wt; bias contiguous or None)."""
-    _check(X, Wt) if bias is None else _check(X, Wt, bias)
-    if X.dim() != 2 or Wt.dim() != 2 or X.shape[1] != Wt.shape[0]:
-        raise ValueError(f"linear_fwd: shapes {tuple(X.shape)} and {tuple(Wt.shape)} do not multiply")
-    m, k = X.shape
-    n = Wt.shape[1]
-    if bias is not None and (bias.numel() != n or not bias.is_contiguous()):
-        raise ValueError("linear_fwd: bias must be contiguous with one value per output column")
-    out = torch.empty((m, n), dtype=torch.float32, device=X.device)
-    if out.numel():
-        with _on(X.device):
-            ws_bytes = load_library().pam_hip_gemm_workspace_bytes(1, m, n, k)
-            ws = _gemm_workspace(X.device, ws_bytes) if ws_bytes else None
-            _call("pam_hip_pam_linear_fwd", X.data_ptr(), X.stride(0), X.stride(1), Wt.data_ptr(), Wt.stride(0), Wt.stride(1),
-                  None if bias is None else bias.data_ptr(), out.data_ptr(), out.stride(0), out.stride(1), m, n, k,
-                  float(offset), ws.data_ptr() if ws is not None else None, ws_bytes, _stream())
-    return out

@@ -1,4 +1,5 @@
-"""Compiles the HIP sources of this package into pam_amd/lib/libpam_hip.so for gfx950.
+"""Compiles the HIP sources of this package into pam_amd/lib/libpam_hip.so for gfx950, and the ops' host path into the
+Python module pam_amd/lib/_pam_host.so on top of it.
 
 hipcc cross-compiles without a GPU, so this runs anywhere the ROCm toolchain is installed.
 Packed-fp32 instruction selection is switched off and floating-point contraction is off:
@@ -19,7 +20,9 @@ SOURCES = [CSRC / "pam_rowops_plain.hip", CSRC / "pam_rowops_offset.hip"] + sort
     CSRC / "pam_gemm.hip", CSRC / "pam_elementwise.hip", CSRC / "pam_rowops.hip", CSRC / "pam_colsum.hip", CSRC / "pam_probe.hip"]   # slowest first
 JOBS = 8
 STAMP_SOURCE = CSRC / "pam_stamp.cpp"
+HOST_SOURCE = CSRC / "pam_host.cpp"
 LIB = HERE / "lib" / "libpam_hip.so"
+HOST = HERE / "lib" / "_pam_host.so"
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -27,6 +30,19 @@ FLAGS = [
 ]
 _NOISE = "is not a recognized feature for this target"      # the host pass does not know the device feature
 _TAG = b"pam_hip_source_hash="
+
+
+def _host_flags():
+    import sysconfig
+
+    import torch
+    root = pathlib.Path(torch.__file__).resolve().parent
+    flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DTORCH_EXTENSION_NAME=_pam_host",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + sysconfig.get_paths()["include"],
+             f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include"]
+    link = [f"-L{root}/lib", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", f"-L{LIB.parent}",
+            "-l:libpam_hip.so", "-Wl,-rpath,$ORIGIN"]
+    return flags, link
 
 
 def _run(cmd, verbose):
@@ -69,13 +85,14 @@ def source_hash():
 
 
 def built_hash():
-    """The hash the built library carries, or None if there is no library (or one without a stamp).  Read from the
-    file's bytes: loading a possibly stale library into this process, which may go on to load its replacement,
-    would register two copies of the code objects."""
-    if not LIB.exists():
-        return None
-    m = re.search(re.escape(_TAG) + rb"([0-9a-f]{16})\0", LIB.read_bytes())
-    return m.group(1).decode() if m else None
+    """The hash the built library and host module carry, or None if one is missing, without a stamp or not built with
+    the other.  Read from the files' bytes: loading a possibly stale library into this process, which may go on to load
+    its replacement, would register two copies of the code objects."""
+    found = set()
+    for lib in (LIB, HOST):
+        m = re.search(re.escape(_TAG) + rb"([0-9a-f]{16})\0", lib.read_bytes()) if lib.exists() else None
+        found.add(m.group(1).decode() if m else None)
+    return found.pop() if len(found) == 1 else None
 
 
 def ensure_built(verbose=False):
@@ -104,21 +121,24 @@ def build(verbose=False, object_dir=None):
         out.mkdir(parents=True, exist_ok=True)
         jobs, objects = [], []
         with concurrent.futures.ThreadPoolExecutor(JOBS) as pool:
-            for src in SOURCES + [STAMP_SOURCE]:
+            host_flags, host_link = _host_flags()
+            for src in SOURCES + [HOST_SOURCE, STAMP_SOURCE]:
                 obj = out / (src.stem + ".o")
-                objects.append(str(obj))
-                flags = FLAGS + ([stamp] if src == STAMP_SOURCE else [])
+                compiler, flags = ("g++", host_flags) if src == HOST_SOURCE else ("hipcc", FLAGS + ([stamp] if src == STAMP_SOURCE else []))
+                if src != HOST_SOURCE:
+                    objects.append(str(obj))
                 key = hashlib.sha256(" ".join(flags).encode() + b"".join(f.read_bytes() for f in _with_includes(src))).hexdigest()
                 keyfile = out / (src.stem + ".key")
                 if object_dir and obj.exists() and keyfile.exists() and keyfile.read_text() == key:
                     continue
                 keyfile.unlink(missing_ok=True)
-                jobs.append((pool.submit(_run, ["hipcc", *flags, "-c", str(src), "-o", str(obj)], verbose), keyfile, key))
+                jobs.append((pool.submit(_run, [compiler, *flags, "-c", str(src), "-o", str(obj)], verbose), keyfile, key))
             for job, keyfile, key in jobs:
                 job.result()
                 if object_dir:
                     keyfile.write_text(key)
         _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objects, "-o", str(LIB)], verbose)
+        _run(["g++", "-shared", str(out / "pam_host.o"), str(out / "pam_stamp.o"), "-o", str(HOST), *host_link], verbose)
     return LIB
 
 

@@ -12,7 +12,7 @@ import math
 import torch
 
 from . import utils
-from ._abi import HipKernels
+from ._abi import HipKernels, host
 
 cuda_kernels = HipKernels()
 
@@ -166,12 +166,33 @@ class pam_matmul_autograd(torch.autograd.Function):
         return delta_A, delta_B, None, None, None
 
 
+def approx_codes(approx_bwd):
+    """(first operands, second operands, exp / log) as numbers for the nodes in C++; -1 where it is neither a flag nor a
+    pair, which only a backward pass minds.  The last is the flag's truth value, so a pair counts as set
+    (pam/cuda_bindings.py:227, 267)."""
+    if isinstance(approx_bwd, bool):
+        return approx_bwd, approx_bwd, approx_bwd
+    try:
+        a, b = approx_bwd
+    except (TypeError, ValueError):
+        return -1, -1, -1
+    return bool(a), bool(b), bool(approx_bwd)
+
+
+def _product_node(A, B, offset, approx_bwd, BMM):
+    if type(cuda_kernels) is HipKernels and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
+        # the node in C++: the same checks, products and formulas
+        a, b, _ = approx_codes(approx_bwd)
+        return host().matmul(A, B, 3 if BMM else 2, _offset_value(offset), a, b)
+    return pam_matmul_autograd.apply(A, B, offset, approx_bwd, BMM)
+
+
 def pam_matmul(A, B, *, offset=None, approx_bwd=False):
-    return pam_matmul_autograd.apply(A, B, offset, approx_bwd, False)
+    return _product_node(A, B, offset, approx_bwd, False)
 
 
 def pam_bmm(A, B, *, offset=None, approx_bwd=False):
-    return pam_matmul_autograd.apply(A, B, offset, approx_bwd, True)
+    return _product_node(A, B, offset, approx_bwd, True)
 
 
 class standard_matmul_autograd(torch.autograd.Function):

@@ -15,7 +15,7 @@ import torch
 from . import _abi
 from . import cuda_bindings
 from ._abi import HipRowKernels
-from .cuda_bindings import _both, _offset_value
+from .cuda_bindings import _both, _offset_value, approx_codes
 
 row_kernels = HipRowKernels()
 
@@ -36,29 +36,10 @@ def _wants_grad(*tensors):
     return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
 
 
-class softmax_autograd(torch.autograd.Function):
-    """softmax over the last dimension; the gradient is the chain of the primitives'
-    gradients (pam/cuda_bindings.py:43-57, 78-97, 224-239) in one kernel."""
-
-    @staticmethod
-    def forward(ctx, x, offset=None, approx_bwd=False):
-        ctx.offset = _offset_value(offset)
-        ctx.approx_bwd = approx_bwd
-        rows = x.reshape(-1, x.shape[-1])
-        y, row_sum, shift = row_kernels.softmax_fwd(rows, ctx.offset)
-        ctx.save_for_backward(rows, row_sum, shift)
-        return y.view(x.shape)
-
-    @staticmethod
-    def backward(ctx, grad):
-        rows, row_sum, shift = ctx.saved_tensors
-        g = grad.contiguous().view(rows.shape)
-        dx = row_kernels.softmax_bwd(rows, g, row_sum, shift, ctx.offset, *_flags(ctx.approx_bwd))
-        return dx.view(grad.shape), None, None
-
-
 def softmax(x, offset=None, approx_bwd=False):
-    return softmax_autograd.apply(x, offset, approx_bwd)
+    """softmax over the last dimension; the gradient is the chain of the primitives' gradients
+    (pam/cuda_bindings.py:43-57, 78-97, 224-239) in one kernel."""
+    return _abi.host().softmax(x, _offset_value(offset), *approx_codes(approx_bwd))
 
 
 def _flags(approx_bwd):
@@ -138,51 +119,9 @@ def mean_last(x, keepdim, offset=None):
     return y.view(x.shape[:-1] + ((1,) if keepdim else ()))
 
 
-def _summable(t):
-    """Whether the sum over the rows of t runs on the kernel: not where autograd is to record it (a gradient's gradient)."""
-    return (t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.stride(1) == 1 and t.numel() > 0
-            and not (t.requires_grad and torch.is_grad_enabled()))
-
-
-def _sum_rows(t):
-    return _abi.column_sums(t) if _summable(t) else t.sum(0)
-
-
-class layer_norm_autograd(torch.autograd.Function):
-    """layer_norm over the last n values of each row; weight and bias of n values or None."""
-
-    @staticmethod
-    def forward(ctx, rows, weight, bias, eps, offset, approx_bwd):
-        ctx.offset = _offset_value(offset)
-        ctx.approx_bwd = approx_bwd
-        ctx.eps = eps
-        ctx.has_bias = bias is not None
-        w = None if weight is None else weight.contiguous().view(-1)
-        b = None if bias is None else bias.contiguous().view(-1)
-        ctx.save_for_backward(rows, w)
-        return row_kernels.layer_norm_fwd(rows, w, b, eps, ctx.offset)
-
-    @staticmethod
-    def backward(ctx, grad):
-        rows, w = ctx.saved_tensors
-        g = grad.contiguous()
-        want_w = w is not None and ctx.needs_input_grad[1]
-        dx, terms = row_kernels.layer_norm_bwd(rows, w, g, ctx.eps, ctx.offset, *_flags(ctx.approx_bwd), want_w)
-        # the broadcast weight and bias collect their gradients by a sum over the rows, as autograd's expand does
-        want_b = ctx.has_bias and ctx.needs_input_grad[2]
-        if want_w and want_b and _summable(g):
-            dw, db = _abi.column_sums(terms, g)
-        else:
-            dw = _sum_rows(terms) if want_w else None
-            db = _sum_rows(g) if want_b else None
-        return dx, dw, db, None, None, None
-
-
 def layer_norm(x, n, weight, bias, eps, offset=None, approx_bwd=False):
-    w = None if weight is None else weight.reshape(-1)
-    b = None if bias is None else bias.reshape(-1)
-    out = layer_norm_autograd.apply(x.reshape(-1, n), w, b, eps, offset, approx_bwd)
-    return out.view(x.shape)
+    """layer_norm over the last n values of each row; weight and bias of n values or None."""
+    return _abi.host().layer_norm(x, n, weight, bias, eps, _offset_value(offset), *approx_codes(approx_bwd))
 
 
 # ---------------------------------------------------------------- power with a scalar exponent
@@ -283,41 +222,8 @@ def conv2d(X, W, stride, padding, offset=None, approx_bwd=False, groups=1):
 
 # ---------------------------------------------------------------- linear with the bias added in the product's epilogue
 
-class linear_autograd(torch.autograd.Function):
-    """X W^T + bias in one kernel; the gradients are those of the product
-    (pam/cuda_bindings.py:132-166) and, for the bias, the sum of the upstream gradient over the rows."""
-
-    @staticmethod
-    def forward(ctx, X, W, bias, offset, approx_bwd):
-        ctx.offset = _offset_value(offset)
-        ctx.approx_bwd = approx_bwd
-        X2, _ = cuda_bindings.check_row_major(X, 2)
-        Wt, _ = cuda_bindings.check_row_major(W.t(), 2)
-        ctx.save_for_backward(X2, Wt)
-        return _abi.linear_fwd(X2, Wt, bias.contiguous(), ctx.offset)
-
-    @staticmethod
-    def backward(ctx, dY):
-        A, B = ctx.saved_tensors                      # A = X, B = W^T as the product saw them
-        k, off = cuda_bindings.cuda_kernels, ctx.offset
-        approx_a, approx_b = _both(ctx.approx_bwd)
-        crm = cuda_bindings.check_row_major
-        dY2, dY_rm = crm(dY, 2)
-        At, At_rm = crm(A.mT, 2)
-        Bt, Bt_rm = crm(B.mT, 2)
-        dX = dW = db = None
-        if ctx.needs_input_grad[0]:
-            dX = k.pam_matmul_fwd(dY2, Bt, dY_rm, Bt_rm, off) if approx_a else k.pam_matmul_bwd(dY2, Bt, A, dY_rm, Bt_rm, True, off)
-        if ctx.needs_input_grad[1]:
-            dB = k.pam_matmul_fwd(At, dY2, At_rm, dY_rm, off) if approx_b else k.pam_matmul_bwd(At, dY2, B, At_rm, dY_rm, False, off)
-            dW = dB.t()
-        if ctx.needs_input_grad[2]:
-            db = _sum_rows(dY2)
-        return dX, dW, db, None, None
-
-
 class add_bias_autograd(torch.autograd.Function):
-    """rows + bias, with the bias gradient that linear_autograd forms."""
+    """rows + bias, with the bias gradient that the linear node forms."""
 
     @staticmethod
     def forward(ctx, rows, bias):
@@ -325,7 +231,10 @@ class add_bias_autograd(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        return g, _sum_rows(g) if ctx.needs_input_grad[1] else None
+        if not ctx.needs_input_grad[1]:
+            return g, None
+        recorded = g.requires_grad and torch.is_grad_enabled()           # a gradient's gradient: autograd sees the sum
+        return g, g.sum(0) if recorded or g.stride(1) != 1 or g.numel() == 0 else _abi.column_sums(g)
 
 
 def add_bias(rows, bias):
@@ -333,4 +242,7 @@ def add_bias(rows, bias):
 
 
 def linear_with_bias(X2d, W, bias, offset=None, approx_bwd=False):
-    return linear_autograd.apply(X2d, W, bias, offset, approx_bwd)
+    """X W^T + bias in one kernel; the gradients are those of the product
+    (pam/cuda_bindings.py:132-166) and, for the bias, the sum of the upstream gradient over the rows."""
+    a, b, _ = approx_codes(approx_bwd)
+    return _abi.host().linear(X2d, W, bias, _offset_value(offset), a, b)

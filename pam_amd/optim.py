@@ -66,32 +66,28 @@ class Adam(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        batch = _Batch(1.0 if self.offset is None else self.offset)
-        try:
-            for group in self.param_groups:
-                for p in group["params"]:
-                    if p.grad is not None and not (self.fused and self._add_to(batch, group, p)):
-                        batch.flush()                  # parameters are updated in their order
-                        self._update(group, p)
-        finally:
-            batch.flush()                              # also those before one that raised
+        for group in self.param_groups:
+            self._step_group(group)
         return loss
 
-    def _add_to(self, batch, group, p):
-        """Enters a parameter with moments into the batch that one kernel updates, if p, its gradient and moments are
-        contiguous fp32 tensors of one shape on one GPU; else returns False and changes nothing."""
-        state = self.state.get(p)
-        if not state or group.get("amsgrad", False):
-            return False
-        grad, exp_avg, exp_avg_sq, shape, device = p.grad, state["exp_avg"], state["exp_avg_sq"], p.shape, p.device
-        if device.type != "cuda":
-            return False
-        for t in (p, grad, exp_avg, exp_avg_sq):
-            if t.dtype is not torch.float32 or t.device != device or t.shape != shape or t.is_sparse or not t.is_contiguous():
-                return False
-        state["step"] += 1
-        batch.add(group, state["step"], device, (p.data_ptr(), grad.data_ptr(), exp_avg.data_ptr(), exp_avg_sq.data_ptr(), p.numel()))
-        return True
+    def _step_group(self, group):
+        """The group's parameters in their order: runs of contiguous fp32 GPU tensors with moments and one step count by
+        one launch each, others by themselves."""
+        params, at = group["params"], 0
+        together = self.fused and type(params) is list and not group.get("amsgrad", False)
+        while at < len(params):
+            if together:
+                at, step, device, table = _abi.host().adam_collect(params, at, self.state)
+                if table:
+                    beta1, beta2 = group["betas"]
+                    decay, step_size = _step_scalars(group, step)
+                    _abi.adam_step_many(table, torch.device("cuda", device), beta1, 1 - beta1, beta2, 1 - beta2, group["eps"], decay,
+                                        step_size, 1.0 if self.offset is None else self.offset)
+                    continue
+            if at < len(params):
+                if params[at].grad is not None:
+                    self._update(group, params[at])
+                at += 1
 
     def _update(self, group, p):
         """One parameter by itself, by the single-tensor kernel or op by op."""
@@ -141,28 +137,6 @@ def _step_scalars(group, step):
     correction2 = 1 - beta2 ** step
     decay = group["weight_decay"] * group["lr"] if group["weight_decay"] != 0 else None
     return decay, group["lr"] * math.sqrt(correction2) / correction1
-
-
-class _Batch:
-    """The tensors of a step that one call updates: consecutive parameters of one group, step count and device."""
-
-    def __init__(self, offset):
-        self.offset, self.key, self.table = offset, None, []
-
-    def add(self, group, step, device, entry):
-        key = (id(group), step, device)
-        if key != self.key:
-            self.flush()
-            self.key, self.group = key, group
-        self.table.extend(entry)
-
-    def flush(self):
-        table, self.table = self.table, []
-        if table:
-            group, (_, step, device) = self.group, self.key
-            beta1, beta2 = group["betas"]
-            decay, step_size = _step_scalars(group, step)
-            _abi.adam_step_many(table, device, beta1, 1 - beta1, beta2, 1 - beta2, group["eps"], decay, step_size, self.offset)
 
 
 def multiply_grads(params, c, op_dict):

@@ -286,3 +286,79 @@ def test_bench_refuses_more_than_one_gpu():
     root = pathlib.Path(__file__).resolve().parents[1]
     res = subprocess.run([sys.executable, str(root / "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert res.returncode != 0 and "one GPU" in res.stderr and res.stdout.strip() == ""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["linear", "matmul", "bmm", "softmax", "layer_norm"])
+def test_nodes_keep_autograds_rules(op):
+    """The ops whose autograd nodes are in C++: saved-tensor hooks see their tensors, a tensor changed in place after the
+    forward pass is an error, gradients come only for what asks for one, a gradient that is differentiated again keeps
+    the graph of its ordinary sums, and a flag that is none only fails a backward pass."""
+    torch.manual_seed(0)
+    new = lambda *shape: torch.randn(*shape, device="cuda")
+    inputs = {"linear": [new(33, 20), new(24, 20), new(24)], "matmul": [new(33, 20), new(20, 24)], "bmm": [new(3, 9, 20), new(3, 20, 8)],
+              "softmax": [new(5, 37)], "layer_norm": [new(5, 6, 40), new(40), new(40)]}[op]
+    call = {"linear": pam_amd.linear, "matmul": pam_amd.matmul, "bmm": pam_amd.bmm,
+            "softmax": lambda x, **kw: pam_amd.softmax(x, dim=-1, **kw),
+            "layer_norm": lambda x, w, b, **kw: pam_amd.layer_norm(x, 40, w, b, **kw)}[op]
+    leaves = [t.clone().requires_grad_() for t in inputs]
+    y = call(*leaves, approx_bwd=True)
+    dy = torch.randn_like(y)
+    want = torch.autograd.grad(y, leaves, dy)
+    assert all(g.shape == t.shape for g, t in zip(want, leaves)) and not call(*inputs).requires_grad
+
+    seen = []
+    def pack(t):
+        seen.append(t.shape)
+        return t.cpu()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        y = call(*leaves, approx_bwd=True)
+    assert seen and all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, leaves, dy), want))
+
+    for i in range(len(inputs)):                                        # one gradient at a time
+        some = [t.clone().requires_grad_(j == i) for j, t in enumerate(inputs)]
+        g, = torch.autograd.grad(call(*some, approx_bwd=True), [some[i]], dy)
+        assert torch.equal(g, want[i])
+
+    y = call(*leaves, approx_bwd=True)
+    with torch.no_grad():
+        leaves[0].mul_(1.0)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        torch.autograd.grad(y, leaves, dy)
+
+    if op in ("linear", "layer_norm"):                                    # the bias gradient is a plain sum of dy
+        dyr = dy.clone().requires_grad_()
+        grads = torch.autograd.grad(call(*leaves, approx_bwd=True), leaves, dyr, create_graph=True)
+        again, = torch.autograd.grad(grads[2].sum(), dyr)
+        assert torch.equal(again, torch.ones_like(dy))
+
+    y = call(*leaves, approx_bwd=None)
+    with pytest.raises(TypeError):
+        torch.autograd.grad(y, leaves, dy)
+    if op in ("matmul", "bmm"):
+        with pytest.raises(TypeError):
+            call(*[t.double() for t in inputs])
+
+
+@pytest.mark.gpu
+def test_nodes_on_threads_and_streams():
+    """Products that cut their tiles, from several threads on streams of their own at once: each as alone (every stream has
+    its own scratch)."""
+    import threading
+    torch.manual_seed(1)
+    data = [[torch.randn(300, 4096, device="cuda"), torch.randn(4096, 100 + 30 * i, device="cuda")] for i in range(4)]
+    want = [pam_amd.matmul(a, b) for a, b in data]
+    torch.cuda.synchronize()
+    bad = []
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(10):
+                if not torch.equal(pam_amd.matmul(*data[i]), want[i]):
+                    bad.append(i)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
