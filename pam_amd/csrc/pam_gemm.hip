@@ -375,7 +375,7 @@ int conv_prepare(const char* what, const ConvShape& s, const ConvSpace& sp, void
     hipLaunchKernelGGL(conv_tables_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, ktab, ltab, (int)s.K(), (int)s.L(),
                        (int)s.kh, (int)s.kw, (int)s.h, (int)s.w, (int)s.wo, (int)s.sh, (int)s.sw, (int)s.ph, (int)s.pw);
     const bool quads = s.ph == 0 && s.pw == 0 && s.kw % 4 == 0 && s.w % 4 == 0 && s.sw % 4 == 0;
-    const bool row_quads = s.sw == 1 && s.wo % 4 == 0;
+    const bool row_quads = s.sw == 1 && s.wo % 4 == 0 && s.w >= 4;
     cv = ConvGeom{ktab, ltab, (int)s.h, (int)s.w, transposed ? 1 : 0, quads ? 1 : 0, row_quads ? 1 : 0};
     return PAM_HIP_OK;
 }

@@ -285,3 +285,16 @@ def test_grouped_module_matches_unfolded_composition(approx, stride):
             composites.implicit_conv = True
     for a, c in zip(res[True], res[False]):
         assert a.shape == c.shape and _close(a, c)
+
+
+@pytest.mark.parametrize("case", [
+    (1, 3, 6, 4, 5, 3, 7, (1, 1), (1, 3)),              # rows of four values: quads up to three places over either end
+    (1, 2, 5, 4, 3, 1, 9, (1, 1), (0, 4)),              # ... and wholly outside
+    (2, 3, 6, 7, 5, 3, 4, (1, 1), (1, 2)),              # odd width, even kernel: ends of different reach
+    (1, 3, 6, 2, 4, 1, 3, (1, 1), (0, 2)),              # rows shorter than a quad
+])
+def test_position_quads_over_the_row_ends(oracle, case):
+    """Four output positions per load where the patches reach over the ends of the image's rows, by every number of places."""
+    test_forward_against_oracle(oracle, case, None)
+    test_weight_gradient_against_oracle(oracle, case, None)
+    test_input_gradient_against_oracle(oracle, case, None)
