@@ -176,6 +176,66 @@ __global__ __launch_bounds__(128) void fold_kernel(pamgemm::GemmArgs g)
         if (c + j < g.N) dst[(long)j * g.y_sc] = g.bias ? sums[j] + g.bias[c + j] : sums[j];
 }
 
+// Products of at most kFewRows rows and short sums (one decoding step of attention: a query against the keys and values of
+// every head).  The matrix kernel's 64 x 64 tiles leave 63 of 64 rows empty there and run a k-tile at a time, each a round
+// trip to memory; here a work-group takes 64 columns of one matrix, a k-tile is 64 deep with all of a lane's loads in flight and the
+// next tile's loads run under the sums of this one.  Wavefront r sums row r, one column per lane, k ascending from +0: the
+// order of whole tiles.  Bound by the latency of two to three rounds of loads.  256 products of 1 x 120, k = 64: 8.6 -> 4.4 us,
+// of 1 x 64, k = 120: 13.8 -> 5.9; 512 of 4 x 512, k = 64: 35 -> 21 (1.6 to 2.8 times faster at all of 1 ... 4 rows, k 64 ... 300).
+constexpr int kFewRows = 4, kFewDepth = 64;
+constexpr long kFewLongest = 512;         // longer sums: the tiles' k ranges in pieces have more loads in flight
+template <bool ALONG_K>                   // which index of the right operand is contiguous (or nearer to it)
+__global__ __launch_bounds__(256) void few_rows_kernel(pamgemm::GemmArgs g)
+{
+    using namespace pamgemm;
+    constexpr int kEach = kFewDepth * 64 / 256, kPitch = 64 + 1;
+    __shared__ uint32_t right[kFewDepth * kPitch];
+    __shared__ __attribute__((aligned(16))) uint32_t left[kFewRows][kFewDepth];
+    const int zb = blockIdx.x / g.ntn, col0 = (blockIdx.x - zb * g.ntn) * 64;
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const float* lbase = g.L.p + (long)zb * g.L.sb + (long)min(wave, g.M - 1) * g.L.sr;
+    const float* rbase = g.R.p + (long)zb * g.R.sb;
+    uint32_t rv[kEach], lv;
+    // (indexes past the end repeat the last one: their values are not summed)
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        lv = f2u(lbase[(long)min(k0 + lane, g.K - 1) * g.L.sk]);
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+            const int k = ALONG_K ? lane : wave + 4 * i, n = ALONG_K ? wave + 4 * i : lane;
+            rv[i] = f2u(rbase[(long)min(col0 + n, g.N - 1) * g.R.sr + (long)min(k0 + k, g.K - 1) * g.R.sk]);
+        }
+    };
+    float acc = 0.0f;
+    load(0);
+    for (int k0 = 0; k0 < g.K; k0 += kFewDepth) {
+        uint32_t seen = window(lv);
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+            const int k = ALONG_K ? lane : wave + 4 * i, n = ALONG_K ? wave + 4 * i : lane;
+            right[k * kPitch + n] = rv[i];
+            seen = max(seen, window(rv[i]));
+        }
+        left[wave][lane] = lv;
+        const bool plain = __syncthreads_or(seen >= kWindowSpan ? 1 : 0) == 0;
+        const int depth = min(kFewDepth, g.K - k0);
+        if (k0 + kFewDepth < g.K) load(k0 + kFewDepth);
+        if (wave < g.M) {
+            const uint32_t* lrow = left[wave];
+            if (plain) {
+#pragma unroll 16
+                for (int k = 0; k < depth; ++k) acc = acc + u2f(lrow[k] + (right[k * kPitch + lane] - kBias));
+            } else {
+#pragma unroll 1
+                for (int k = 0; k < depth; ++k) acc = acc + pam_mul(u2f(lrow[k]), u2f(right[k * kPitch + lane]));
+            }
+        }
+        __syncthreads();
+    }
+    const int c = col0 + lane;
+    if (wave < g.M && c < g.N)
+        g.Y[(long)zb * g.y_sb + (long)wave * g.y_sr + (long)c * g.y_sc] = g.bias ? acc + g.bias[c] : acc;
+}
+
 int load_kind(long s_row, long s_k, long s_batch, const float* p, long rows, long K)
 {
     bool aligned = ((reinterpret_cast<uintptr_t>(p) & 15u) == 0) && (s_batch % 4 == 0);
@@ -248,6 +308,12 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
 
     g.cv = conv ? *conv : ConvGeom{nullptr, nullptr, 0, 0, 0, 0, 0};
 
+    if (mode == MODE_PAM && !conv && M <= kFewRows && K <= kFewLongest && p.pieces == 1 && g.has_off == 0 && g_force_bk == 0 && g_force_pieces == 0) {
+        const unsigned groups = (unsigned)(batch * g.ntn);
+        if (g.R.sk <= g.R.sr) hipLaunchKernelGGL(few_rows_kernel<true>, dim3(groups), dim3(256), 0, st, g);
+        else hipLaunchKernelGGL(few_rows_kernel<false>, dim3(groups), dim3(256), 0, st, g);
+        return pamhost::check_launch(what);
+    }
     int lk = load_kind(l_sr, l_sc, l_sb, l, M, K);
     int rk = conv ? LOAD_CONV : load_kind(r_sc, r_sr, r_sb, r, N, K);
     if (conv && conv->quads && !conv->transposed && mode == MODE_PAM && lk == LOAD_KVEC && K % 4 == 0 && (reinterpret_cast<uintptr_t>(r) & 15u) == 0 && r_sb % 4 == 0)

@@ -716,3 +716,49 @@ def test_more_than_two_to_the_31_elements(K, oracle):
     Y = K.pam_matmul_fwd(L, Rm, True, True, 1.0)
     for lo, hi in ((0, 70), (m - 70, m)):
         assert_same_bits(host(Y[lo:hi]), ogemm(oracle, host(L[lo:hi]), host(Rm), plan_shape=(1, m, 64, 16)), f"product rows [{lo}:{hi}]")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,n,k", [(1, 1, 1, 1), (3, 1, 120, 64), (3, 1, 64, 120), (2, 2, 65, 63), (2, 3, 63, 65), (5, 4, 197, 129), (700, 4, 130, 512)])
+def test_few_rows_equal_the_matrix_kernel(oracle, batch, m, n, k):
+    """Products of up to four rows take a kernel of their own; the matrix kernel with whole tiles sums in the same order: bit
+    for bit the same for every order and stride of the operands and every class of values."""
+    from pam_amd import _abi
+    lib, H = _abi.load_library(), _abi.host()
+    rng = np.random.RandomState(batch + m + n + k)
+    def operand(rows, cols, specials):
+        a = rng.standard_normal((batch, rows, cols)).astype(np.float32)
+        if specials:
+            flat = a.reshape(-1)
+            some = rng.choice(flat.size, min(flat.size, 7), replace=False)
+            flat[some] = np.array([0.0, -0.0, 1e-40, -3e38, np.inf, np.nan, 1e-30], np.float32)[:some.size]
+        return a
+    def views(a):
+        t = torch.from_numpy(a).cuda()
+        b, r, c = a.shape
+        apart = torch.zeros(b, r + 1, c + 3, device="cuda")[:, 1:, 2:c + 2]
+        apart.copy_(t)
+        wide = torch.zeros(b, r, 2 * c, device="cuda")[:, :, ::2]
+        wide.copy_(t)
+        heads = torch.zeros(r, b, c, device="cuda").transpose(0, 1)           # (batch stride below the row stride)
+        heads.copy_(t)
+        return [t, t.transpose(1, 2).contiguous().transpose(1, 2), apart, wide, heads]
+    for specials in (False, True):
+        A, B = operand(m, k, specials), operand(k, n, specials)
+        want = None
+        for a in views(A):
+            for b in views(B):
+                got = H.product(0, a, b, None, False, None, 1.0)
+                if want is None:
+                    lib.pam_hip_set_tuning(16, 1)
+                    try:
+                        want = H.product(0, a, b, None, False, None, 1.0).cpu().numpy()
+                    finally:
+                        lib.pam_hip_set_tuning(0, 0)
+                    if batch <= 5:
+                        assert_same_bits(want, oracle.gemm(A, B, kchunk=0), "whole tiles")
+                if _abi.gemm_plan(batch, m, n, k) in (0,) or _abi.gemm_plan(batch, m, n, k) >= k:
+                    assert_same_bits(got.cpu().numpy(), want, f"{batch} x {m}x{k}x{n} specials={specials}")
+    bias = torch.randn(n, device="cuda")
+    a, b = (torch.from_numpy(t[0]).cuda() for t in (operand(m, k, False), operand(k, n, False)))
+    assert torch.equal(H.product(0, a, b, None, False, bias, 1.0), H.product(0, a, b, None, False, None, 1.0) + bias)
