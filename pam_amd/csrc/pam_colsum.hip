@@ -6,8 +6,8 @@
 // the rows are cut into ranges of at least kLeastRows, whose sums go to the workspace and are added by the same kernel in
 // a second launch.  No step adds more than a few dozen values one after the other, so the rounding error stays below that
 // of longer chains.  Two matrices of one shape can be summed in one launch.
-// Measured against torch's sum over dim 0 (which also clears a buffer first): 12608 x 768 values 26 -> 14 us, 50432 x 192
-// twice 48 -> 22 us.
+// Measured against torch's sum over dim 0 (which also clears a buffer first, 5 us): a linear layer of 12608 x 192 -> 768 with
+// its gradients 277 -> 266 us, 4096 x 512 -> 1024 375 -> 361.
 #include <algorithm>
 #include <cstdint>
 

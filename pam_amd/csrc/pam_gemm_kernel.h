@@ -180,7 +180,7 @@ __device__ __forceinline__ int swizzled(int row, int k) { return BK == 32 ? row 
 // one 128-bit load from where the quad lies inside the row, in image_quad, and `settle`, which moves it to its place by
 // selects when the values are staged (done at once they would wait for the load there) -- a quad reaches at most a kernel's
 // width over the row's ends, almost always by one.  (Four loads, each with its own test, address and execution mask, were
-// a quarter of the vector instructions of a 3 x 3 convolution: 1442 -> 1401 us, forward and both gradients of 128 images of
+// a quarter of the vector instructions of a 3 x 3 convolution: 1442 -> 1390 us, forward and both gradients of 128 images of
 // 64 x 32 x 32 to 128 channels.)  W is at least 4.
 typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));      // at any float's address
 __device__ __forceinline__ float4 image_quad(const float* base, const ConvGeom& cv, const int2 ke, const int2 le, int& over)
@@ -216,12 +216,12 @@ struct TileLoader {
     int patch_at[kVecs > 0 ? kVecs : 1];          // LOAD_CONVQ: where the patches of the lane's rows begin in the image
     int2 row_entry[KIND == LOAD_CONVK && kVecs > 0 ? kVecs : 1];      // LOAD_CONVK: the k table's entries of the lane's rows
 
-    int over[(KIND == LOAD_CONVR || KIND == LOAD_CONVK) && kVecs > 0 ? kVecs : 1];      // ... how far their quads reach over the row's ends
+    int over[KIND == LOAD_CONVR && kVecs > 0 ? kVecs : 1];      // LOAD_CONVR: how far the quads reach over the row's ends
 
     // before the loaded values are looked at
     __device__ __forceinline__ void arrive()
     {
-        if (KIND == LOAD_CONVR || KIND == LOAD_CONVK) {
+        if (KIND == LOAD_CONVR) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) v[i] = settle(v[i], over[i]);
         }
@@ -271,7 +271,17 @@ struct TileLoader {
                 have_fixed = true;
             }
 #pragma unroll
-            for (int i = 0; i < kVecs; ++i) v[i] = image_quad(base, cv, row_entry[i], cv.ltab[min(k0 + ((tid + i * NT) % (BK / 4)) * 4, kend - 4)], over[i]);
+            for (int i = 0; i < kVecs; ++i) {
+                // (value by value: with one load per quad as in LOAD_CONVR the 3 x 3 weight gradient took 542 us instead of 527)
+                const int2 le = cv.ltab[min(k0 + ((tid + i * NT) % (BK / 4)) * 4, kend - 4)], ke = row_entry[i];
+                const int h = (le.y >> 16) + (ke.y >> 16), w = (int)(short)(le.y & 0xffff) + (ke.y & 0xffff);
+                const bool row_inside = (unsigned)h < (unsigned)cv.H;
+                const float* at = base + (ke.x + le.x);
+                v[i].x = row_inside && (unsigned)w < (unsigned)cv.W ? at[0] : 0.0f;
+                v[i].y = row_inside && (unsigned)(w + 1) < (unsigned)cv.W ? at[1] : 0.0f;
+                v[i].z = row_inside && (unsigned)(w + 2) < (unsigned)cv.W ? at[2] : 0.0f;
+                v[i].w = row_inside && (unsigned)(w + 3) < (unsigned)cv.W ? at[3] : 0.0f;
+            }
         } else if (KIND == LOAD_CONVQ) {
             // as LOAD_KVEC, the address from the two tables: the rows' entries once per work-group, k's per k-tile
             typedef const __attribute__((address_space(4))) int* ConstTable;

@@ -6,9 +6,9 @@ from the primitive kernels (the reference's pam/pam_ops.py:288-378), in one swee
 rows instead of five to fifteen elementwise launches.  The only difference is the order of
 the row sums, which the reference leaves to torch.sum and the kernels fix.
 
-`row_kernels` is the kernel object; tests may swap it for another object with the same
-five methods.  `fusable` says whether a call can take this path: float32 GPU tensor,
-contiguous, reduced dimension last, not empty.
+softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp).  `row_kernels` is the kernel
+object of the others.  `fusable` says whether a call can take this path: float32 GPU tensor, contiguous, reduced dimension
+last, not empty.
 """
 import torch
 
