@@ -185,7 +185,7 @@ class _FiniteWord(threading.local):
     def get(self, device):
         entry = self.by_device.get(device.index)
         if entry is None:
-            word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            word = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)      # (a default device does not apply)
             event = torch.cuda.Event()
             event.record()                            # (creates it)
             entry = self.by_device[device.index] = (word, ctypes.c_int.from_address(word.data_ptr()), event)

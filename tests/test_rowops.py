@@ -661,6 +661,26 @@ def test_nonfinite_input_is_refused_and_the_largest_finite_one_is_not(rows, n):
 
 
 @pytest.mark.gpu
+def test_finite_check_under_a_default_device():
+    """The word that the check reports to is host memory whatever the default device is: the first call of a thread comes
+    under one here."""
+    import threading
+    x = torch.randn(5, 37, device="cuda")
+    want, answers = pam_amd.log_softmax(x, dim=-1), []
+    def work():
+        try:
+            with torch.device("cuda"):
+                answers.append(pam_amd.log_softmax(x, dim=-1))
+                answers.append(pam_amd.logsumexp(x, dim=-1))
+        except Exception as e:
+            answers.append(e)
+    thread = threading.Thread(target=work)
+    thread.start()
+    thread.join()
+    assert len(answers) == 2 and torch.equal(answers[0], want) and torch.equal(answers[1], pam_amd.logsumexp(x, dim=-1)), answers
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,n", [(1, 1), (2, 4), (127, 64), (128, 68), (257, 63), (300, 192), (4097, 20), (12608, 768), (70001, 3), (3, 30011)])
 def test_column_sums(rows, n):
     """Sums over the rows against 64-bit ones, on both load widths, on rows apart from each other and for two matrices in
