@@ -684,15 +684,35 @@ def test_finite_check_under_a_default_device():
 @pytest.mark.parametrize("rows,n", [(1, 1), (2, 4), (127, 64), (128, 68), (257, 63), (300, 192), (4097, 20), (12608, 768), (70001, 3), (3, 30011)])
 def test_column_sums(rows, n):
     """Sums over the rows against 64-bit ones, on both load widths, on rows apart from each other and for two matrices in
-    one call.  A value takes part in at most 64 + 4 + 128 + 4 rounded additions at these sizes (a lane's chain and the tree,
-    twice), each off by 2^-24 of a partial sum that is at most the sum of magnitudes."""
+    one call.  A value takes part in fewer than 64 rounded additions at these sizes (per pass a tree of eight or a rest of
+    up to seven, chains of sixteen, a tree over the lanes), each off by 2^-24 of a partial sum that is at most the sum of
+    magnitudes.  The bits depend on the sizes alone."""
     from pam_amd import _abi
     g = torch.Generator().manual_seed(rows + n)
     a, b = (torch.randn(rows, n, generator=g).cuda() for _ in range(2))
     apart = torch.randn(rows, n + 5, generator=g).cuda()[:, 1:n + 1]
-    sums = [_abi.column_sums(a), *_abi.column_sums(b, a), _abi.column_sums(apart), *_abi.column_sums(a, apart)]
+    copy = torch.zeros(rows, n + 3, device="cuda")[:, 2:n + 2]
+    copy.copy_(a)
+    sums = [_abi.column_sums(a), *_abi.column_sums(b, a), _abi.column_sums(apart), *_abi.column_sums(copy, apart)]
     for got, t in zip(sums, (a, b, a, apart, a, apart)):
         t64 = t.cpu().double()
-        bound = 200 * 2.0 ** -24 * t64.abs().sum(0)
+        bound = 64 * 2.0 ** -24 * t64.abs().sum(0)
         assert ((got.cpu().double() - t64.sum(0)).abs() <= bound).all()
-    assert torch.equal(sums[0], sums[2]) or rows > 128          # cut alike where nothing is cut
+    assert torch.equal(sums[0], sums[2]) and torch.equal(sums[0], sums[4]) and torch.equal(sums[3], sums[5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n", [(1 << 20, 63), (65536, 609), (16384, 4095), (65536, 2048), (8192, 32001), (4096, 131073)])
+def test_column_sums_of_long_shares(rows, n):
+    """Sizes at which a lane's share of a column is long (many rows, or so many columns that the rows are not cut).  Equal
+    values whose last bits every addition to a long partial sum loses the same way: a single chain is off by up to a
+    quarter of its length times 2^-24.  A value takes part in fewer than 64 rounded additions (see above)."""
+    from pam_amd import _abi
+    value = 1.0 + torch.arange(n, device="cuda", dtype=torch.float64) / n * 2.0 ** -10
+    row = value.float()
+    a = row.expand(rows, n).contiguous()
+    alone = _abi.column_sums(a)
+    exact = row.double() * rows
+    assert ((alone.double() - exact).abs() <= 64 * 2.0 ** -24 * exact).all()
+    first, second = _abi.column_sums(a, a)
+    assert torch.equal(first, alone) and torch.equal(second, alone)
