@@ -130,6 +130,13 @@ bool summable(const Tensor& t)
 // the sums over the rows of one matrix, or of two of one shape
 std::pair<Tensor, Tensor> column_sums(const Tensor& a, const Tensor& b)
 {
+    check_tensor(a);
+    TORCH_CHECK_VALUE(a.dim() == 2 && (a.stride(1) == 1 || a.size(1) <= 1), "column_sums: expected a matrix whose rows are contiguous");
+    if (b.defined()) {
+        check_tensor(b);
+        TORCH_CHECK_VALUE(b.sizes() == a.sizes() && b.device() == a.device() && (b.stride(1) == 1 || b.size(1) <= 1),
+                          "column_sums: the second matrix must have the first one's shape and device, and contiguous rows");
+    }
     const OnDevice on(a);
     const int64_t rows = a.size(0), n = a.size(1);
     Tensor a_sums = new_floats({n}, a), b_sums, ws;

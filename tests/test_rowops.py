@@ -716,3 +716,20 @@ def test_column_sums_of_long_shares(rows, n):
     assert ((alone.double() - exact).abs() <= 64 * 2.0 ** -24 * exact).all()
     first, second = _abi.column_sums(a, a)
     assert torch.equal(first, alone) and torch.equal(second, alone)
+
+
+@pytest.mark.gpu
+def test_column_sums_refuses_what_its_kernel_does_not_take():
+    """Checked on the host before a pointer is passed on: the device, the type, the rank, the order, and the second matrix's
+    shape, device and order.  No rows give zeros, no columns an empty result."""
+    from pam_amd import _abi
+    a = torch.randn(8, 12, device="cuda")
+    for bad in (a.cpu(), a[0], a.t(), a.view(2, 4, 12)):
+        with pytest.raises((RuntimeError, ValueError)):
+            _abi.column_sums(bad)
+    with pytest.raises(TypeError):
+        _abi.column_sums(a.double())
+    for other in (a.cpu(), a[:4], torch.randn(12, 8, device="cuda"), torch.randn(12, 8, device="cuda").t(), a[0]):
+        with pytest.raises((RuntimeError, ValueError)):
+            _abi.column_sums(a, other)
+    assert torch.equal(_abi.column_sums(a[:0]), torch.zeros(12, device="cuda")) and _abi.column_sums(a[:, :0]).shape == (0,)
