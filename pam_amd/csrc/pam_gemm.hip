@@ -177,20 +177,30 @@ __global__ __launch_bounds__(128) void fold_kernel(pamgemm::GemmArgs g)
 }
 
 // Products of at most kFewRows rows and short sums (one decoding step of attention: a query against the keys and values of
-// every head).  The matrix kernel's 64 x 64 tiles leave 63 of 64 rows empty there and run a k-tile at a time, each a round
-// trip to memory; here a work-group takes 64 columns of one matrix, a k-tile is 64 deep with all of a lane's loads in flight and the
+// every head).  The matrix kernel's 64 x 64 tiles leave 60 or more of 64 rows empty there and run a k-tile at a time, each a
+// round trip to memory; here a work-group takes 64 columns of one matrix, a k-tile is 64 deep with all of a lane's loads in flight and the
 // next tile's loads run under the sums of this one.  Wavefront r sums row r, one column per lane, k ascending from +0: the
 // order of whole tiles.  Bound by the latency of two to three rounds of loads.  256 products of 1 x 120, k = 64: 8.6 -> 4.4 us,
-// of 1 x 64, k = 120: 13.8 -> 5.9; 512 of 4 x 512, k = 64: 35 -> 21 (1.6 to 2.8 times faster at all of 1 ... 4 rows, k 64 ... 300).
+// of 1 x 64, k = 120: 13.8 -> 5.9; 512 of 4 x 512, k = 64: 35 -> 18; 1600 of 4 x 64, k = 512: 90 -> 49.
+// Zeros (masked keys, padded caches, activations behind a ReLU) contribute nothing: where a tile's only values outside the
+// plain window are zeros, a product is selected away by one test of both operands, since no sum that starts from +0 becomes -0.
+// (The general definition for such tiles was up to 45 % slower than the matrix kernel with its paths for zeros: 256 of 1 x 120,
+// k = 64, a third of the right operand zeros 12.2 us, matrix kernel 10.2, now 5.3; 1600 of 4 x 64, k = 512 156, 121, 74.)
+// Other values outside the window (subnormal, infinite, huge, tiny) take the general definition: 100 us at the latter, 207
+// in the matrix kernel.  With up to four rows this kernel was the faster one in every class of values at thirteen shapes, 1.4 to
+// 4.5 times.  A plan that cuts k (k of 256 and more on fewer than 1536 tiles) goes to the matrix kernel, whose pieces the
+// sums follow; beyond kFewLongest nothing was measured.
 constexpr int kFewRows = 4, kFewDepth = 64;
-constexpr long kFewLongest = 512;         // longer sums: the tiles' k ranges in pieces have more loads in flight
+constexpr long kFewLongest = 512;
 template <bool ALONG_K>                   // which index of the right operand is contiguous (or nearer to it)
 __global__ __launch_bounds__(256) void few_rows_kernel(pamgemm::GemmArgs g)
 {
     using namespace pamgemm;
     constexpr int kEach = kFewDepth * 64 / 256, kPitch = 64 + 1;
+    enum { kPlain = 0, kZeros = 1, kOdd = 2 };
     __shared__ uint32_t right[kFewDepth * kPitch];
     __shared__ __attribute__((aligned(16))) uint32_t left[kFewRows][kFewDepth];
+    __shared__ int classes[kFewRows];
     const int zb = blockIdx.x / g.ntn, col0 = (blockIdx.x - zb * g.ntn) * 64;
     const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
     const float* lbase = g.L.p + (long)zb * g.L.sb + (long)min(wave, g.M - 1) * g.L.sr;
@@ -216,16 +226,31 @@ __global__ __launch_bounds__(256) void few_rows_kernel(pamgemm::GemmArgs g)
             seen = max(seen, window(rv[i]));
         }
         left[wave][lane] = lv;
-        const bool plain = __syncthreads_or(seen >= kWindowSpan ? 1 : 0) == 0;
+        int mine = kPlain;
+        if (__ballot(seen >= kWindowSpan) != 0ull) {
+            uint32_t odd = (lv << 1) != 0u ? window(lv) : 0u;
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) odd = max(odd, (rv[i] << 1) != 0u ? window(rv[i]) : 0u);
+            mine = __ballot(odd >= kWindowSpan) != 0ull ? kOdd : kZeros;
+        }
+        if (lane == 0) classes[wave] = mine;
+        __syncthreads();
+        const int cls = max(max(classes[0], classes[1]), max(classes[2], classes[3]));
         const int depth = min(kFewDepth, g.K - k0);
         if (k0 + kFewDepth < g.K) load(k0 + kFewDepth);
         if (wave < g.M) {
             const uint32_t* lrow = left[wave];
-            if (plain) {
+            if (cls == kPlain) {
 #pragma unroll 16
                 for (int k = 0; k < depth; ++k) acc = acc + u2f(lrow[k] + (right[k * kPitch + lane] - kBias));
+            } else if (cls == kZeros) {
+#pragma unroll 16
+                for (int k = 0; k < depth; ++k) {
+                    const uint32_t l = lrow[k], r = right[k * kPitch + lane];
+                    acc = acc + (min(l << 1, r << 1) != 0u ? u2f(l + (r - kBias)) : 0.0f);
+                }
             } else {
-#pragma unroll 1
+#pragma unroll 4
                 for (int k = 0; k < depth; ++k) acc = acc + pam_mul(u2f(lrow[k]), u2f(right[k * kPitch + lane]));
             }
         }

@@ -762,3 +762,36 @@ def test_few_rows_equal_the_matrix_kernel(oracle, batch, m, n, k):
     bias = torch.randn(n, device="cuda")
     a, b = (torch.from_numpy(t[0]).cuda() for t in (operand(m, k, False), operand(k, n, False)))
     assert torch.equal(H.product(0, a, b, None, False, bias, 1.0), H.product(0, a, b, None, False, None, 1.0) + bias)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["left", "right", "both", "all left", "all right", "one, and one inf"])
+@pytest.mark.parametrize("batch,m,n,k", [(2, 1, 70, 64), (3, 4, 64, 130), (700, 2, 190, 512)])
+def test_few_rows_with_zeros(oracle, batch, m, n, k, where):
+    """Zeros of either sign among ordinary values, in one k-tile and not in the next, whole operands of them, and next to
+    an infinity (whose product with a zero is what the definition says): the bits of whole tiles and of the oracle."""
+    from pam_amd import _abi
+    lib, H = _abi.load_library(), _abi.host()
+    rng = np.random.RandomState(batch + m + n + k)
+    A, B = rng.standard_normal((batch, m, k)).astype(np.float32), rng.standard_normal((batch, k, n)).astype(np.float32)
+    def zeros(a, share):
+        at = rng.random_sample(a.shape) < share
+        a[at] = np.where(rng.random_sample(a.shape) < 0.5, 0.0, -0.0).astype(np.float32)[at]
+    if where in ("left", "both"): zeros(A[..., :64], 0.5)
+    if where in ("right", "both"): zeros(B[:, -64:], 0.5)
+    if where == "all left": zeros(A, 1.0)
+    if where == "all right": zeros(B, 1.0)
+    if where == "one, and one inf":
+        A[0, 0, 0], B[0, 0, 0], B[-1, -1, -1] = 0.0, np.inf, 0.0
+    a, b = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
+    lib.pam_hip_set_tuning(16, 1)
+    try:
+        want = H.product(0, a, b, None, False, None, 1.0).cpu().numpy()
+    finally:
+        lib.pam_hip_set_tuning(0, 0)
+    if batch <= 3:
+        assert_same_bits(want, oracle.gemm(A, B, kchunk=0), "whole tiles")
+    plan = _abi.gemm_plan(batch, m, n, k)
+    assert plan == 0 or plan >= k
+    for right in (b, b.transpose(1, 2).contiguous().transpose(1, 2)):
+        assert_same_bits(H.product(0, a, right, None, False, None, 1.0).cpu().numpy(), want, where)
