@@ -31,6 +31,10 @@ size_t pam_hip_column_sums_workspace_bytes(long rows, long n, int matrices);
 int pam_hip_column_sums(const float *a, long a_row_stride, float *a_sums, const float *b, long b_row_stride, float *b_sums,
                         long rows, long n, void *workspace, size_t workspace_bytes, void *stream);
 
+/* Beside pam_hip_gemm_plan: whether the work-groups of that product (exact: of the exact gradient's products) lower their
+ * priority as they proceed. */
+int pam_hip_gemm_priority_steps(long batch, long m, long n, long k, int exact);
+
 #ifdef __cplusplus
 }
 #endif

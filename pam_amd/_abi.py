@@ -74,6 +74,7 @@ _SIGNATURES = {
 # include/pam_hip_extra.h
 _EXTRA_SIGNATURES = {
     "pam_hip_logsumexp_fwd_finite": ([_p, _p, _p, _p, _l, _l, _f, _p, _p, _p, _z, _p], _i),
+    "pam_hip_gemm_priority_steps": ([_l, _l, _l, _l, _i], _i),
     "pam_hip_column_sums_workspace_bytes": ([_l, _l, _i], _z),
     "pam_hip_column_sums": ([_p, _l, _p, _p, _l, _p, _l, _l, _p, _z, _p], _i),
     "pam_hip_adam_step_many": ([_p, _l, _f, _f, _f, _f, _f, _f, _i, _f, _f, _p], _i),

@@ -101,6 +101,7 @@ struct GemmArgs {
     int pieces, piece_kt;        // k ranges a tile is cut into (1: whole tiles) and their length in k-tiles
     int units;                   // tiles of all matrices x pieces: one work-group each
     int xcd_chunk;               // > 0: work-group x takes unit (x % XCDS) * xcd_chunk + x / XCDS, else unit x
+    int steps;                   // work-groups lower their priority by quarters of their k-tiles (priority_steps)
     int fold_here;               // cut tiles are added up by the work-group that arrives last (else by a second kernel)
     unsigned long long* arrive;  // cut tiles: one arrival word per tile
     unsigned long long tag;      // cut tiles: this launch's tag in the arrival words (40 bits)
@@ -938,12 +939,15 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
         // Among wavefronts of one priority the scheduler serves the oldest first: of four work-groups on a compute unit two
         // finished at half the time the others took, and those then ran at fewer wavefronts than hide each other's waits
         // (4096 x 1024, k = 512: wavefronts resident for 64 % of the launch on average).  So a work-group's priority falls
-        // by quarters of its k-tiles: the ones behind catch up, and all are there until the end.  Forward and gradients of
-        // 4096 x 1024 x 512 with a ReLU's zeros 309 -> 277 us, exact gradients 352 -> 330, 12608 x 192 x 768 260 -> 257.
-        if (t == 0) __builtin_amdgcn_s_setprio(3);
-        else if (t == q1) __builtin_amdgcn_s_setprio(2);
-        else if (t == q2) __builtin_amdgcn_s_setprio(1);
-        else if (t == q3) __builtin_amdgcn_s_setprio(0);
+        // by quarters of its k-tiles: the ones behind catch up, and all are there until the end -- in the launches where
+        // that pays (priority_steps in pam_gemm.hip).  Forward and gradients of 4096 x 1024 x 512 with a ReLU's zeros
+        // 309 -> 277 us, exact gradients 352 -> 330.
+        if (g.steps) {
+            if (t == 0) __builtin_amdgcn_s_setprio(3);
+            else if (t == q1) __builtin_amdgcn_s_setprio(2);
+            else if (t == q2) __builtin_amdgcn_s_setprio(1);
+            else if (t == q3) __builtin_amdgcn_s_setprio(0);
+        }
         if (MODE != MODE_STD) {
             uint32_t f = 0;
 #pragma unroll

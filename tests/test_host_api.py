@@ -362,3 +362,17 @@ def test_nodes_on_threads_and_streams():
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("shape,exact,want", [
+    # (1024 work-groups are resident: four on each of 256 compute units)
+    ((1, 96, 128, 64), 0, 0), ((1, 512, 4096, 64), 0, 0),                       # a round of at most two per compute unit: nothing to even out
+    ((1, 2112, 1024, 96), 0, 1), ((1, 4096, 1024, 512), 0, 1), ((192, 197, 64, 197), 0, 1),     # more than half a round
+    ((1, 4352, 1024, 96), 0, 0), ((128, 128, 576, 1024), 0, 0), ((128, 128, 576, 1024), 1, 0),  # one more per compute unit behind a full round or two
+    ((1, 12608, 768, 192), 0, 1), ((1, 12608, 768, 192), 1, 0),                 # two more behind: whole tiles, and deep enough
+    ((1, 12544 + 63, 768, 192), 0, 0), ((192, 197, 133, 64), 0, 0),             # ragged ones, shallow ones
+    ((128, 64, 1024, 1152), 0, 1), ((128, 64, 1024, 1152), 1, 1),               # two full rounds
+    ((1, 192, 768, 12608), 0, 1), ((1, 192, 768, 12608), 1, 1),                 # 57 pieces of 36 tiles: two rounds and four units
+    ((512, 128, 128, 64), 0, 0), ((1, 8192, 1024, 128), 1, 0), ((1, 8192, 1024, 256), 1, 1), ((1, 16384, 1024, 256), 1, 0), ((1, 16384, 1024, 320), 1, 1)])
+def test_priorities_fall_only_where_the_last_round_fills_the_chip(shape, exact, want):
+    assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, exact) == want
