@@ -128,8 +128,10 @@ bool priority_steps(const Plan& p, long M, long N, bool exact)
 {
     const long cus = cu_count(), resident = (long)kResidentPerCu * cus;
     if (p.units <= resident) return p.units > resident / 2;
-    // (2 % over whole rounds count as those where many pieces are added by a second kernel: 2052 units of 224 k 0.95)
-    const long counted = p.pieces > pamgemm::kFoldInKernel ? p.units - p.units / 50 : p.units;
+    // (piece-major launches end with the tiles' last pieces, which may be short: a few of at most a third of the length behind
+    // full rounds do not count, 2052 units of 224 k of which the last 36 have 64: 0.95; from half the length on they do, 1.02 to 1.10)
+    const long tiles = p.units / p.pieces, extra = p.units % resident, tail = p.kt - (long)(p.pieces - 1) * p.piece_kt;
+    const long counted = p.pieces > pamgemm::kFoldInKernel && extra <= tiles && 3 * tail <= p.piece_kt ? p.units - extra : p.units;
     const long rounds = (counted + resident - 1) / resident, last = (counted - 1) % resident + 1;
     const bool most = last > resident / 2;
     if (p.piece_kt < (!exact || (most && rounds <= 2) ? 6 : most && rounds <= 3 ? 8 : 10)) return false;

@@ -372,7 +372,8 @@ def test_nodes_on_threads_and_streams():
     ((1, 12608, 768, 192), 0, 1), ((1, 12608, 768, 192), 1, 0),                 # two more behind: whole tiles, and deep enough
     ((1, 12544 + 63, 768, 192), 0, 0), ((192, 197, 133, 64), 0, 0),             # ragged ones, shallow ones
     ((128, 64, 1024, 1152), 0, 1), ((128, 64, 1024, 1152), 1, 1),               # two full rounds
-    ((1, 192, 768, 12608), 0, 1), ((1, 192, 768, 12608), 1, 1),                 # 57 pieces of 36 tiles: two rounds and four units
+    ((1, 192, 768, 12608), 0, 1), ((1, 192, 768, 12608), 1, 1),                 # 57 pieces of 36 tiles: two rounds and four short units
+    ((1, 364, 233, 13642), 0, 0),                                               # 43 pieces of 24 tiles: a round and eight units of 0.7 the length
     ((512, 128, 128, 64), 0, 0), ((1, 8192, 1024, 128), 1, 0), ((1, 8192, 1024, 256), 1, 1), ((1, 16384, 1024, 256), 1, 0), ((1, 16384, 1024, 320), 1, 1)])
 def test_priorities_fall_only_where_the_last_round_fills_the_chip(shape, exact, want):
     assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, exact) == want
