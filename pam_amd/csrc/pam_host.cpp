@@ -52,16 +52,25 @@ Tensor new_floats(at::IntArrayRef shape, const Tensor& like) { return at::empty(
 
 // The matrix products' scratch (pieces of cut tiles, their arrival words): one buffer per device and stream, kept and
 // grown as needed.  Products on one stream run one after the other, and each leaves the arrival words ready for the
-// next one; products on different streams may overlap in time and must not share a buffer.
+// next one; products on different streams may overlap in time and must not share a buffer.  The lock covers the table
+// only: buffers are allocated and given back outside it, since the allocator may wait for the driver or for the
+// interpreter (its hooks), which another thread that waits for the lock might hold.
 Tensor gemm_workspace(const Tensor& like, void* stream, size_t bytes)
 {
     static std::mutex lock;
     static auto* kept = new std::map<std::pair<int, void*>, Tensor>;           // (not destroyed after the allocator at exit)
+    const std::pair<int, void*> key{like.device().index(), stream};
+    const auto fits = [&](const Tensor& t) { return t.defined() && (size_t)t.numel() * 4 >= bytes; };
+    {
+        std::lock_guard<std::mutex> hold(lock);
+        const auto at = kept->find(key);
+        if (at != kept->end() && fits(at->second)) return at->second;
+    }
+    Tensor ws = new_floats({(int64_t)(std::max(bytes, (size_t)1 << 20) / 4 + 64)}, like);
     std::lock_guard<std::mutex> hold(lock);
-    Tensor& ws = (*kept)[{like.device().index(), stream}];
-    if (!ws.defined() || (size_t)ws.numel() * 4 < bytes)
-        ws = new_floats({(int64_t)(std::max(bytes, (size_t)1 << 20) / 4 + 64)}, like);
-    return ws;
+    Tensor& entry = (*kept)[key];
+    if (!fits(entry)) std::swap(entry, ws);          // (ws, the smaller one or a second one, goes after the lock has)
+    return entry;
 }
 
 // ---------------------------------------------------------------- products
@@ -370,26 +379,33 @@ py::tuple adam_collect(py::list params, size_t start, py::dict state)
 
 }  // namespace
 
+// The interpreter is free for other threads while an op checks, allocates and launches, each of which may wait (a full
+// launch queue, the driver, the table of workspaces); only adam_collect reads Python objects.
 PYBIND11_MODULE(_pam_host, module)
 {
+    const py::call_guard<py::gil_scoped_release> unlocked;
     module.def("product", [](int kind, const Tensor& L, const Tensor& R, const std::optional<Tensor>& other, bool delta_left,
                              const std::optional<Tensor>& bias, double offset) {
         return product(kind, L, R, other.value_or(Tensor()), delta_left, bias.value_or(Tensor()), offset);
-    });
+    }, unlocked);
     module.def("column_sums", [](const Tensor& a, const std::optional<Tensor>& b) {
-        const auto sums = column_sums(a, b.value_or(Tensor()));
+        std::pair<Tensor, Tensor> sums;
+        {
+            const py::gil_scoped_release release;
+            sums = column_sums(a, b.value_or(Tensor()));
+        }
         return b ? py::cast(sums) : py::cast(sums.first);
     });
     module.def("matmul", [](const Tensor& A, const Tensor& B, int64_t dims, double offset, int64_t a, int64_t b) {
         return MatmulNode::apply(A, B, dims, offset, a, b);
-    });
+    }, unlocked);
     module.def("linear", [](const Tensor& X, const Tensor& W, const Tensor& bias, double offset, int64_t a, int64_t b) {
         return LinearNode::apply(X, W, bias, offset, a, b);
-    });
-    module.def("softmax", [](const Tensor& x, double offset, int64_t a, int64_t b, int64_t e) { return SoftmaxNode::apply(x, offset, a, b, e); });
+    }, unlocked);
+    module.def("softmax", [](const Tensor& x, double offset, int64_t a, int64_t b, int64_t e) { return SoftmaxNode::apply(x, offset, a, b, e); }, unlocked);
     module.def("layer_norm", [](const Tensor& x, int64_t n, const std::optional<Tensor>& weight, const std::optional<Tensor>& bias, double eps,
                                 double offset, int64_t a, int64_t b, int64_t e) {
         return LayerNormNode::apply(x, n, weight, bias, eps, offset, a, b, e);
-    });
+    }, unlocked);
     module.def("adam_collect", &adam_collect);
 }

@@ -377,3 +377,36 @@ def test_nodes_on_threads_and_streams():
     ((512, 128, 128, 64), 0, 0), ((1, 8192, 1024, 128), 1, 0), ((1, 8192, 1024, 256), 1, 1), ((1, 16384, 1024, 256), 1, 0), ((1, 16384, 1024, 320), 1, 1)])
 def test_priorities_fall_only_where_the_last_round_fills_the_chip(shape, exact, want):
     assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, exact) == want
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_launch_waits():
+    """Behind one long product thousands of small ones fill the launch queue, and the next call waits for it: other
+    Python threads go on meanwhile."""
+    import threading
+    import time
+    a, b = torch.ones(16384, 65536, device="cuda"), torch.ones(65536, 16384, device="cuda")
+    small = torch.ones(1, 1, device="cuda")
+    pam_amd.matmul(a[:64], b[:, :64])
+    pam_amd.matmul(small, small)
+    torch.cuda.synchronize()
+    gaps, stop = [0.0], threading.Event()
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(1e-3)
+            now = time.perf_counter()
+            gaps.append(now - last)
+            last = now
+    thread = threading.Thread(target=tick)
+    thread.start()
+    began = time.perf_counter()
+    pam_amd.matmul(a, b)
+    for _ in range(25000):
+        pam_amd.matmul(small, small)
+    queued = time.perf_counter() - began
+    torch.cuda.synchronize()
+    stop.set()
+    thread.join()
+    print(f"queued in {queued:.2f} s, longest gap {max(gaps):.3f} s")
+    assert max(gaps) < 0.2, (queued, max(gaps))
