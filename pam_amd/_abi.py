@@ -537,6 +537,19 @@ def column_sums(A, B=None):
     return host().column_sums(A, B)
 
 
+def sum_rows(A):
+    """A.sum(0) by the kernel where it takes A; by torch where it does not or where autograd is to record the sum."""
+    return host().sum_rows(A)
+
+
+def linear_fwd(X, Wt, bias, offset):
+    """X[m, k] (x) Wt[k, n] + bias[n] in one pass (any strides for X and Wt; bias contiguous or None)."""
+    _check(X, Wt) if bias is None else _check(X, Wt, bias)
+    if X.dim() != 2 or Wt.dim() != 2:
+        raise ValueError(f"linear_fwd: shapes {tuple(X.shape)} and {tuple(Wt.shape)} do not multiply")
+    return host().product(0, X, Wt, None, False, bias, float(offset))
+
+
 def _conv_geometry(X, W, stride, padding, groups=1):
     if X.dim() != 4 or W.dim() != 4 or groups < 1 or X.shape[1] != W.shape[1] * groups or W.shape[0] % groups:
         raise ValueError("conv2d: expected X[batch, c, h, w] and W[co, c / groups, kh, kw]")

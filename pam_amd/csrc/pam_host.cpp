@@ -396,6 +396,7 @@ PYBIND11_MODULE(_pam_host, module)
         }
         return b ? py::cast(sums) : py::cast(sums.first);
     });
+    module.def("sum_rows", &sum_rows, unlocked);
     module.def("matmul", [](const Tensor& A, const Tensor& B, int64_t dims, double offset, int64_t a, int64_t b) {
         return MatmulNode::apply(A, B, dims, offset, a, b);
     }, unlocked);

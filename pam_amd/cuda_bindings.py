@@ -179,8 +179,14 @@ def approx_codes(approx_bwd):
     return bool(a), bool(b), bool(approx_bwd)
 
 
+def own_kernels(kernels, cls):
+    """Whether a kernel object is the package's own with no method replaced, so that a node in C++ may stand for it; any
+    other object's methods are called, by the autograd functions in Python."""
+    return type(kernels) is cls and not vars(kernels)
+
+
 def _product_node(A, B, offset, approx_bwd, BMM):
-    if type(cuda_kernels) is HipKernels and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
+    if own_kernels(cuda_kernels, HipKernels) and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
         # the node in C++: the same checks, products and formulas
         a, b, _ = approx_codes(approx_bwd)
         return host().matmul(A, B, 3 if BMM else 2, _offset_value(offset), a, b)

@@ -6,16 +6,16 @@ from the primitive kernels (the reference's pam/pam_ops.py:288-378), in one swee
 rows instead of five to fifteen elementwise launches.  The only difference is the order of
 the row sums, which the reference leaves to torch.sum and the kernels fix.
 
-softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp).  `row_kernels` is the kernel
-object of the others.  `fusable` says whether a call can take this path: float32 GPU tensor, contiguous, reduced dimension
-last, not empty.
+`row_kernels` is the kernel object; it may be swapped for another one with the same methods.  With the package's own,
+softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp) that make the same calls.
+`fusable` says whether a call can take this path: float32 GPU tensor, contiguous, reduced dimension last, not empty.
 """
 import torch
 
 from . import _abi
 from . import cuda_bindings
-from ._abi import HipRowKernels
-from .cuda_bindings import _both, _offset_value, approx_codes
+from ._abi import HipKernels, HipRowKernels
+from .cuda_bindings import _both, _offset_value, approx_codes, own_kernels
 
 row_kernels = HipRowKernels()
 
@@ -36,9 +36,30 @@ def _wants_grad(*tensors):
     return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
 
 
+class softmax_autograd(torch.autograd.Function):
+    """softmax over the last dimension on a swapped kernel object."""
+
+    @staticmethod
+    def forward(ctx, x, offset=None, approx_bwd=False):
+        ctx.offset, ctx.approx_bwd = _offset_value(offset), approx_bwd
+        rows = x.reshape(-1, x.shape[-1])
+        y, row_sum, shift = row_kernels.softmax_fwd(rows, ctx.offset)
+        ctx.save_for_backward(rows, row_sum, shift)
+        return y.view(x.shape)
+
+    @staticmethod
+    def backward(ctx, grad):
+        rows, row_sum, shift = ctx.saved_tensors
+        g = grad.contiguous().view(rows.shape)
+        dx = row_kernels.softmax_bwd(rows, g, row_sum, shift, ctx.offset, *_flags(ctx.approx_bwd))
+        return dx.view(grad.shape), None, None
+
+
 def softmax(x, offset=None, approx_bwd=False):
     """softmax over the last dimension; the gradient is the chain of the primitives' gradients
     (pam/cuda_bindings.py:43-57, 78-97, 224-239) in one kernel."""
+    if not own_kernels(row_kernels, HipRowKernels):
+        return softmax_autograd.apply(x, offset, approx_bwd)
     return _abi.host().softmax(x, _offset_value(offset), *approx_codes(approx_bwd))
 
 
@@ -62,7 +83,8 @@ class logsumexp_autograd(torch.autograd.Function):
         ctx.approx_bwd = approx_bwd
         ctx.as_log_softmax = as_log_softmax
         rows = x.reshape(-1, x.shape[-1])
-        lse, y, shift = row_kernels.logsumexp_fwd(rows, ctx.offset, not as_log_softmax, as_log_softmax, check_finite)
+        lse, y, shift = row_kernels.logsumexp_fwd(rows, ctx.offset, not as_log_softmax, as_log_softmax,
+                                                  *([True] if check_finite else []))
         ctx.save_for_backward(rows, shift)
         if as_log_softmax:
             return y.view(x.shape)
@@ -86,8 +108,9 @@ def log_softmax(x, offset=None, approx_bwd=False, check_finite=False):
 
 
 def finite_in_kernel():
-    """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded."""
-    return not torch.cuda.is_current_stream_capturing()
+    """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded, and not
+    asked of a swapped kernel object."""
+    return own_kernels(row_kernels, HipRowKernels) and not torch.cuda.is_current_stream_capturing()
 
 
 class mean_autograd(torch.autograd.Function):
@@ -119,8 +142,34 @@ def mean_last(x, keepdim, offset=None):
     return y.view(x.shape[:-1] + ((1,) if keepdim else ()))
 
 
+class layer_norm_autograd(torch.autograd.Function):
+    """layer_norm over the last n values of each row on a swapped kernel object; weight and bias of n values or None."""
+
+    @staticmethod
+    def forward(ctx, rows, weight, bias, eps, offset, approx_bwd):
+        ctx.offset, ctx.approx_bwd, ctx.eps = _offset_value(offset), approx_bwd, eps
+        ctx.has_bias = bias is not None
+        w = None if weight is None else weight.contiguous()
+        ctx.save_for_backward(rows, w)
+        return row_kernels.layer_norm_fwd(rows, w, None if bias is None else bias.contiguous(), eps, ctx.offset)
+
+    @staticmethod
+    def backward(ctx, grad):
+        rows, w = ctx.saved_tensors
+        g = grad.contiguous()
+        want_w = w is not None and ctx.needs_input_grad[1]
+        dx, terms = row_kernels.layer_norm_bwd(rows, w, g, ctx.eps, ctx.offset, *_flags(ctx.approx_bwd), want_w)
+        # the broadcast weight and bias collect their gradients by a sum over the rows, as autograd's expand does
+        dw = _abi.sum_rows(terms) if want_w else None
+        db = _abi.sum_rows(g) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
+        return dx, dw, db, None, None, None
+
+
 def layer_norm(x, n, weight, bias, eps, offset=None, approx_bwd=False):
     """layer_norm over the last n values of each row; weight and bias of n values or None."""
+    if not own_kernels(row_kernels, HipRowKernels):
+        w, b = (None if t is None else t.reshape(-1) for t in (weight, bias))
+        return layer_norm_autograd.apply(x.reshape(-1, n), w, b, eps, offset, approx_bwd).view(x.shape)
     return _abi.host().layer_norm(x, n, weight, bias, eps, _offset_value(offset), *approx_codes(approx_bwd))
 
 
@@ -241,8 +290,40 @@ def add_bias(rows, bias):
     return add_bias_autograd.apply(rows, bias)
 
 
+class linear_autograd(torch.autograd.Function):
+    """X W^T + bias in one kernel, with the gradients' products on a swapped kernel object."""
+
+    @staticmethod
+    def forward(ctx, X, W, bias, offset, approx_bwd):
+        ctx.offset, ctx.approx_bwd = _offset_value(offset), approx_bwd
+        X2, _ = cuda_bindings.check_row_major(X, 2)
+        Wt, _ = cuda_bindings.check_row_major(W.t(), 2)
+        ctx.save_for_backward(X2, Wt)
+        return _abi.linear_fwd(X2, Wt, bias.contiguous(), ctx.offset)
+
+    @staticmethod
+    def backward(ctx, dY):
+        A, B = ctx.saved_tensors                      # A = X, B = W^T as the product saw them
+        k, off, crm = cuda_bindings.cuda_kernels, ctx.offset, cuda_bindings.check_row_major
+        approx_a, approx_b = _both(ctx.approx_bwd)
+        dY2, dY_rm = crm(dY, 2)
+        At, At_rm = crm(A.mT, 2)
+        Bt, Bt_rm = crm(B.mT, 2)
+        dX = dW = db = None
+        if ctx.needs_input_grad[0]:
+            dX = k.pam_matmul_fwd(dY2, Bt, dY_rm, Bt_rm, off) if approx_a else k.pam_matmul_bwd(dY2, Bt, A, dY_rm, Bt_rm, True, off)
+        if ctx.needs_input_grad[1]:
+            dB = k.pam_matmul_fwd(At, dY2, At_rm, dY_rm, off) if approx_b else k.pam_matmul_bwd(At, dY2, B, At_rm, dY_rm, False, off)
+            dW = dB.t()
+        if ctx.needs_input_grad[2]:
+            db = _abi.sum_rows(dY2)
+        return dX, dW, db, None, None
+
+
 def linear_with_bias(X2d, W, bias, offset=None, approx_bwd=False):
     """X W^T + bias in one kernel; the gradients are those of the product
     (pam/cuda_bindings.py:132-166) and, for the bias, the sum of the upstream gradient over the rows."""
+    if not own_kernels(cuda_bindings.cuda_kernels, HipKernels):
+        return linear_autograd.apply(X2d, W, bias, offset, approx_bwd)
     a, b, _ = approx_codes(approx_bwd)
     return _abi.host().linear(X2d, W, bias, _offset_value(offset), a, b)

@@ -410,3 +410,59 @@ def test_other_threads_run_while_a_launch_waits():
     thread.join()
     print(f"queued in {queued:.2f} s, longest gap {max(gaps):.3f} s")
     assert max(gaps) < 0.2, (queued, max(gaps))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["object", "method"])
+@pytest.mark.parametrize("approx", [True, False, (True, False)])
+def test_swapped_kernel_objects_are_called(monkeypatch, how, approx):
+    """Another object in place of `fused.row_kernels` or `cuda_bindings.cuda_kernels`, or a method replaced on the one that is
+    there, computes the ops that go through it, forward and backward; one that passes the calls on gives the same bits."""
+    from pam_amd import fused
+    torch.manual_seed(2)
+    calls = []
+
+    class Recorder:                        # the methods as callers know them, without optional arguments of the package's own
+        def __init__(self, kernels):
+            self.kernels = kernels
+        def __getattr__(self, name):
+            method = getattr(self.kernels, name)
+            def call(*args):
+                assert name != "logsumexp_fwd" or len(args) == 4
+                calls.append(name)
+                return method(*args)
+            return call
+
+    x, w, b = (torch.randn(*s, device="cuda") for s in ((6, 37, 40), (40,), (40,)))
+    wl, bl = torch.randn(24, 40, device="cuda"), torch.randn(24, device="cuda")
+    ops = {
+        "softmax": (lambda x: pam_amd.softmax(x, dim=-1, approx_bwd=approx), (x,), fused, ["softmax_fwd", "softmax_bwd"]),
+        "log_softmax": (lambda x: pam_amd.log_softmax(x, dim=-1, approx_bwd=approx), (x,), fused, ["logsumexp_fwd", "logsumexp_bwd"]),
+        "layer_norm": (lambda x, w, b: pam_amd.layer_norm(x, 40, w, b, approx_bwd=approx), (x, w, b), fused, ["layer_norm_fwd", "layer_norm_bwd"]),
+        "linear": (lambda x, w, b: pam_amd.linear(x, w, b, approx_bwd=approx), (x, wl, bl), cuda_bindings, ["pam_matmul_fwd", "pam_matmul_bwd"]),
+        "matmul": (lambda x, w: pam_amd.matmul(x, w, approx_bwd=approx), (x[0], wl.t()), cuda_bindings, ["pam_matmul_fwd", "pam_matmul_bwd"]),
+    }
+    for op, (f, inputs, module, names) in ops.items():
+        def run():
+            leaves = [t.detach().clone().requires_grad_() for t in inputs]
+            y = f(*leaves)
+            return [y, *torch.autograd.grad(y, leaves, torch.linspace(-1, 1, y.numel(), device="cuda").view(y.shape))]
+        want = run()
+        assert not calls
+        holder = "row_kernels" if module is fused else "cuda_kernels"
+        with monkeypatch.context() as m:
+            recorder = Recorder(type(getattr(module, holder))())
+            if how == "object":
+                m.setattr(module, holder, recorder)
+            else:
+                for name in names:
+                    m.setattr(getattr(module, holder), name, getattr(recorder, name), raising=False)
+            got = run()
+        expected = set(names)
+        if op in ("linear", "matmul"):
+            expected = {"pam_matmul_fwd"} if approx is True else {"pam_matmul_bwd"} if approx is False and op == "linear" else set(names)
+        assert set(calls) == expected, (op, calls)
+        calls.clear()
+        for a, c in zip(got, want):
+            assert torch.equal(a, c), op
+    assert not calls and run() is not None and not calls
