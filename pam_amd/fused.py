@@ -271,25 +271,6 @@ def conv2d(X, W, stride, padding, offset=None, approx_bwd=False, groups=1):
 
 # ---------------------------------------------------------------- linear with the bias added in the product's epilogue
 
-class add_bias_autograd(torch.autograd.Function):
-    """rows + bias, with the bias gradient that the linear node forms."""
-
-    @staticmethod
-    def forward(ctx, rows, bias):
-        return rows + bias
-
-    @staticmethod
-    def backward(ctx, g):
-        if not ctx.needs_input_grad[1]:
-            return g, None
-        recorded = g.requires_grad and torch.is_grad_enabled()           # a gradient's gradient: autograd sees the sum
-        return g, g.sum(0) if recorded or g.stride(1) != 1 or g.numel() == 0 else _abi.column_sums(g)
-
-
-def add_bias(rows, bias):
-    return add_bias_autograd.apply(rows, bias)
-
-
 class linear_autograd(torch.autograd.Function):
     """X W^T + bias in one kernel, with the gradients' products on a swapped kernel object."""
 

@@ -105,15 +105,12 @@ def linear(X, W, bias=None, *, offset=None, approx_bwd=False, use_kernel=True):
     (pam/pam_ops.py:107-115).  W.T is passed as a view: the kernel reads W in place."""
     lead = X.shape[:-1]
     rows = X.reshape(-1, X.shape[-1])
-    in_kernel = (bias is not None and use_kernel and rows.is_cuda and rows.numel() and bias.dim() == 1
-                 and all(t.dtype == torch.float32 for t in (rows, W, bias)))
-    if fused_bias and in_kernel:
+    if (fused_bias and bias is not None and use_kernel and rows.is_cuda and rows.numel() and bias.dim() == 1
+            and all(t.dtype == torch.float32 for t in (rows, W, bias))):
         # the bias is added to the finished sums inside the product kernel: the same add, one pass less
         out = fused.linear_with_bias(rows, W, bias, offset, approx_bwd)
         return out.reshape(*lead, out.shape[-1])
     out = matmul(rows, W.T, offset=offset, approx_bwd=approx_bwd, use_kernel=use_kernel)
-    if in_kernel:
-        return fused.add_bias(out, bias).reshape(*lead, out.shape[-1])      # (the bias gradient is the same sum either way)
     out = out.reshape(*lead, out.shape[-1])
     return out if bias is None else out + bias
 

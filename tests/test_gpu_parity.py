@@ -565,7 +565,9 @@ def test_reference_vectors_on_device(K):
 @pytest.mark.gpu
 def test_linear_with_bias_in_the_epilogue(oracle):
     """pam.linear with a bias: added inside the product kernel (after the chunk sums when k is split),
-    bit-identical to the product followed by a separate add; gradients as without the fusion."""
+    bit-identical to the product followed by a separate add; gradients of the input and the weight as without the
+    fusion, the bias's within the rounding of its sum of the 64-bit one, on both sides (fewer than 64 additions per
+    value in this package's sum, see test_column_sums, and no more in autograd's at these sizes)."""
     import pam_amd
     from pam_amd import pam_ops, _abi
     rng = np.random.RandomState(11)
@@ -585,8 +587,11 @@ def test_linear_with_bias_in_the_epilogue(oracle):
             finally:
                 pam_ops.fused_bias = True
         assert_same_bits(res[True][0], want, f"linear+bias {m}x{k}x{n}")
-        for a, c, name in zip(res[True], res[False], ("y", "dX", "dW", "db")):
+        for a, c, name in zip(res[True], res[False], ("y", "dX", "dW")):
             assert_same_bits(a, c, f"{name} fused vs separate add, {m}x{k}x{n}")
+        for side in res.values():
+            d64 = dY.astype(np.float64)
+            assert (np.abs(side[3] - d64.sum(0)) <= 64 * 2.0 ** -24 * np.abs(d64).sum(0)).all(), f"db, {m}x{k}x{n}"
     # leading dimensions and the module
     lin = pam_amd.Linear(192, 96, approx_bwd=True).cuda()
     x3 = torch.randn(4, 197, 192, device="cuda")
