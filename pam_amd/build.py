@@ -30,6 +30,7 @@ FLAGS = [
 ]
 _NOISE = "is not a recognized feature for this target"      # the host pass does not know the device feature
 _TAG = b"pam_hip_source_hash="
+_HOST_TAG = b"pam_host_build="
 
 
 def _host_flags():
@@ -45,13 +46,25 @@ def _host_flags():
     return flags, link
 
 
+def host_hash():
+    """Hash of what the host module depends on beside the library's sources: its flags and link line, the torch whose
+    headers and libraries it is built on, and the Python it is a module of.  It is compiled into the module."""
+    import sysconfig
+
+    import torch
+    flags, link = _host_flags()
+    parts = [part for part in flags + link if "/" not in part]           # (not where this tree or torch lie)
+    parts += [torch.__version__, str(torch.version.git_version), str(sysconfig.get_config_var("SOABI"))]
+    return hashlib.sha256("\0".join(parts).encode()).hexdigest()[:16]
+
+
 def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     err = "\n".join(l for l in res.stderr.splitlines() if _NOISE not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + err)
+        raise RuntimeError(f"{cmd[0]} failed:\n" + err)
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
@@ -84,15 +97,18 @@ def source_hash():
     return h.hexdigest()[:16]
 
 
+def _stamped(path, tag):
+    m = re.search(re.escape(tag) + rb"([0-9a-f]{16})\0", path.read_bytes()) if path.exists() else None
+    return m.group(1).decode() if m else None
+
+
 def built_hash():
     """The hash the built library and host module carry, or None if one is missing, without a stamp or not built with
-    the other.  Read from the files' bytes: loading a possibly stale library into this process, which may go on to load
-    its replacement, would register two copies of the code objects."""
-    found = set()
-    for lib in (LIB, HOST):
-        m = re.search(re.escape(_TAG) + rb"([0-9a-f]{16})\0", lib.read_bytes()) if lib.exists() else None
-        found.add(m.group(1).decode() if m else None)
-    return found.pop() if len(found) == 1 else None
+    the other, or if the module was built on another torch or Python or with other flags.  Read from the files' bytes:
+    loading a possibly stale library into this process, which may go on to load its replacement, would register two
+    copies of the code objects."""
+    found = {_stamped(lib, _TAG) for lib in (LIB, HOST)}
+    return found.pop() if len(found) == 1 and _stamped(HOST, _HOST_TAG) == host_hash() else None
 
 
 def ensure_built(verbose=False):
@@ -111,7 +127,8 @@ def ensure_built(verbose=False):
 
 
 def build(verbose=False, object_dir=None):
-    """Compiles the sources side by side (the matrix kernel's many instances dominate), then links.
+    """Compiles the sources side by side (the matrix kernel's many instances dominate), then links: the library, which
+    needs hipcc alone, and then the host module on top of it, which needs g++ and torch's and Python's headers too.
     object_dir: keep the objects there and recompile only the sources that changed since (for development;
     the default compiles everything)."""
     LIB.parent.mkdir(exist_ok=True)
@@ -119,26 +136,29 @@ def build(verbose=False, object_dir=None):
     with tempfile.TemporaryDirectory() as tmp:
         out = pathlib.Path(object_dir) if object_dir else pathlib.Path(tmp)
         out.mkdir(parents=True, exist_ok=True)
-        jobs, objects = [], []
-        with concurrent.futures.ThreadPoolExecutor(JOBS) as pool:
-            host_flags, host_link = _host_flags()
-            for src in SOURCES + [HOST_SOURCE, STAMP_SOURCE]:
-                obj = out / (src.stem + ".o")
-                compiler, flags = ("g++", host_flags) if src == HOST_SOURCE else ("hipcc", FLAGS + ([stamp] if src == STAMP_SOURCE else []))
-                if src != HOST_SOURCE:
-                    objects.append(str(obj))
-                key = hashlib.sha256(" ".join(flags).encode() + b"".join(f.read_bytes() for f in _with_includes(src))).hexdigest()
-                keyfile = out / (src.stem + ".key")
-                if object_dir and obj.exists() and keyfile.exists() and keyfile.read_text() == key:
-                    continue
+
+        def compile_one(src, compiler, flags):
+            obj, keyfile = out / (src.stem + ".o"), out / (src.stem + ".key")
+            key = hashlib.sha256(" ".join(flags).encode() + b"".join(f.read_bytes() for f in _with_includes(src))).hexdigest()
+            if not (object_dir and obj.exists() and keyfile.exists() and keyfile.read_text() == key):
                 keyfile.unlink(missing_ok=True)
-                jobs.append((pool.submit(_run, [compiler, *flags, "-c", str(src), "-o", str(obj)], verbose), keyfile, key))
-            for job, keyfile, key in jobs:
-                job.result()
+                _run([compiler, *flags, "-c", str(src), "-o", str(obj)], verbose)
                 if object_dir:
                     keyfile.write_text(key)
-        _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objects, "-o", str(LIB)], verbose)
-        _run(["g++", "-shared", str(out / "pam_host.o"), str(out / "pam_stamp.o"), "-o", str(HOST), *host_link], verbose)
+            return str(obj)
+
+        def compile_host():
+            flags, link = _host_flags()
+            return compile_one(HOST_SOURCE, "g++", flags + [f'-DPAM_HOST_BUILD="{host_hash()}"']), link
+
+        with concurrent.futures.ThreadPoolExecutor(JOBS) as pool:
+            jobs = [pool.submit(compile_one, src, "hipcc", FLAGS + ([stamp] if src == STAMP_SOURCE else [])) for src in SOURCES + [STAMP_SOURCE]]
+            host_job = pool.submit(compile_host)
+            objects = [job.result() for job in jobs]
+            _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objects, "-o", str(LIB)], verbose)
+            HOST.unlink(missing_ok=True)             # (never beside a library it was not built with)
+            host_object, host_link = host_job.result()
+        _run(["g++", "-shared", host_object, objects[-1], "-o", str(HOST), *host_link], verbose)
     return LIB
 
 

@@ -18,6 +18,9 @@
 #include "../../include/pam_hip.h"
 #include "../../include/pam_hip_extra.h"
 
+// what this module was built on (pam_amd/build.py reads it from the file's bytes)
+extern "C" __attribute__((used, visibility("default"))) const char pam_host_build[] = "pam_host_build=" PAM_HOST_BUILD;
+
 namespace {
 
 using at::Tensor;

@@ -466,3 +466,39 @@ def test_swapped_kernel_objects_are_called(monkeypatch, how, approx):
         for a, c in zip(got, want):
             assert torch.equal(a, c), op
     assert not calls and run() is not None and not calls
+
+
+def test_build_stamp_covers_what_the_host_module_is_built_on(monkeypatch, tmp_path):
+    """The built files count as current for this torch and these flags, wherever the tree lies, and for no others."""
+    from pam_amd import build as builder
+    assert builder.built_hash() == builder.source_hash()
+    host_hash, flags = builder.host_hash(), builder._host_flags()
+    with monkeypatch.context() as m:
+        m.setattr(builder, "LIB", tmp_path / "elsewhere" / "libpam_hip.so")
+        assert builder.host_hash() == host_hash
+    for what in ("torch", "flags", "link"):
+        with monkeypatch.context() as m:
+            if what == "torch":
+                m.setattr(torch, "__version__", "0.0")
+            else:
+                m.setattr(builder, "_host_flags", lambda: (flags[0] + ["-O1"], flags[1]) if what == "flags" else (flags[0], flags[1] + ["-lm"]))
+            assert builder.built_hash() is None
+    assert builder.built_hash() == builder.source_hash()
+
+
+def test_build_links_the_library_without_the_host_modules_needs(monkeypatch, tmp_path):
+    """Where g++ or torch's headers are missing the library is still linked (a program in C needs no more), the failure
+    is reported, and no host module of another build stays beside it."""
+    from pam_amd import build as builder
+    ran = []
+    def run(cmd, verbose):
+        ran.append(cmd)
+        if cmd[0] == "g++":
+            raise RuntimeError("g++ failed")
+    monkeypatch.setattr(builder, "_run", run)
+    monkeypatch.setattr(builder, "LIB", tmp_path / "libpam_hip.so")
+    monkeypatch.setattr(builder, "HOST", tmp_path / "_pam_host.so")
+    builder.HOST.write_text("an older one")
+    with pytest.raises(RuntimeError, match="g\\+\\+"):
+        builder.build()
+    assert any("-shared" in cmd and str(builder.LIB) in cmd for cmd in ran) and not builder.HOST.exists()
