@@ -119,7 +119,8 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 // has at most one work-group per compute unit they lose 2 to 11 %: units that would have ended apart and let the rest
 // begin early all end at once, and the rest runs alone (on 1024 resident ones: 1328 work-groups 0.97 of the time
 // without steps where the tiles are whole, 1088 1.08, 2304 1.04, 2049 1.05, 2048 0.95, 1024 0.93, 640 0.88, 512 and less 1.00 to
-// 1.03).  Between the two they gain 2 to 3 % on whole tiles that are not cut and nothing elsewhere.  In a launch of several
+// 1.03).  Between the two, in the second and third round, they gain 2 to 3 % in units of twenty and more k-tiles, and in
+// shorter ones that are whole tiles of whole 64 x 64 outputs; elsewhere between -4 and +6 %.  In a launch of several
 // rounds each step must cover more than one k-tile of its unit: units of four or five k-tiles lose 2 to 6 % there, and the
 // exact gradients', with three operations per product, those of up to seven (beyond three rounds nine) 2 to 10 %.
 // On 4151 products of drawn shapes, geometric mean of the time over that without steps: always 0.989, this rule 0.980, the
@@ -135,7 +136,7 @@ bool priority_steps(const Plan& p, long M, long N, bool exact)
     const long rounds = (counted + resident - 1) / resident, last = (counted - 1) % resident + 1;
     const bool most = last > resident / 2;
     if (p.piece_kt < (!exact || (most && rounds <= 2) ? 6 : most && rounds <= 3 ? 8 : 10)) return false;
-    return most || (last > cus && rounds <= 3 && p.pieces == 1 && M % 64 == 0 && N % 64 == 0);
+    return most || (last > cus && rounds <= 3 && (p.piece_kt >= 20 || (p.pieces == 1 && M % 64 == 0 && N % 64 == 0)));
 }
 
 // workspace of a plan that cuts tiles: [arrival words, one per tile][one piece per unit].  The words' part has one size

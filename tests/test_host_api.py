@@ -371,6 +371,7 @@ def test_nodes_on_threads_and_streams():
     ((1, 4352, 1024, 96), 0, 0), ((128, 128, 576, 1024), 0, 0), ((128, 128, 576, 1024), 1, 0),  # one more per compute unit behind a full round or two
     ((1, 12608, 768, 192), 0, 1), ((1, 12608, 768, 192), 1, 0),                 # two more behind: whole tiles, and deep enough
     ((1, 12544 + 63, 768, 192), 0, 0), ((192, 197, 133, 64), 0, 0),             # ragged ones, shallow ones
+    ((51, 128, 900, 864), 0, 1), ((704, 64, 130, 224), 0, 0),                   # ragged, but deep; ragged and not deep
     ((128, 64, 1024, 1152), 0, 1), ((128, 64, 1024, 1152), 1, 1),               # two full rounds
     ((1, 192, 768, 12608), 0, 1), ((1, 192, 768, 12608), 1, 1),                 # 57 pieces of 36 tiles: two rounds and four short units
     ((1, 364, 233, 13642), 0, 0),                                               # 43 pieces of 24 tiles: a round and eight units of 0.7 the length
