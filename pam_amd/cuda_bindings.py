@@ -180,9 +180,11 @@ def approx_codes(approx_bwd):
 
 
 def own_kernels(kernels, cls):
-    """Whether a kernel object is the package's own with no method replaced, so that a node in C++ may stand for it; any
-    other object's methods are called, by the autograd functions in Python."""
-    return type(kernels) is cls and not vars(kernels)
+    """Whether a node in C++ may stand for a kernel object's methods: the object is the package's own with no method
+    replaced, and the call is not being traced (torch.jit.trace records an autograd function in Python as an operation
+    of its own, but of a node in C++ only the allocation of its output).  Any other call goes to the methods, by the
+    autograd functions in Python."""
+    return type(kernels) is cls and not vars(kernels) and not torch.jit.is_tracing()
 
 
 def _product_node(A, B, offset, approx_bwd, BMM):

@@ -7,7 +7,8 @@ rows instead of five to fifteen elementwise launches.  The only difference is th
 the row sums, which the reference leaves to torch.sum and the kernels fix.
 
 `row_kernels` is the kernel object; it may be swapped for another one with the same methods.  With the package's own,
-softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp) that make the same calls.
+softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp) that make the same calls; the
+autograd functions here are for other objects and for calls that are traced.
 `fusable` says whether a call can take this path: float32 GPU tensor, contiguous, reduced dimension last, not empty.
 """
 import torch
@@ -37,7 +38,7 @@ def _wants_grad(*tensors):
 
 
 class softmax_autograd(torch.autograd.Function):
-    """softmax over the last dimension on a swapped kernel object."""
+    """softmax over the last dimension by the kernel object's methods."""
 
     @staticmethod
     def forward(ctx, x, offset=None, approx_bwd=False):
@@ -108,8 +109,8 @@ def log_softmax(x, offset=None, approx_bwd=False, check_finite=False):
 
 
 def finite_in_kernel():
-    """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded, and not
-    asked of a swapped kernel object."""
+    """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded or the
+    call is traced, and not asked of a swapped kernel object."""
     return own_kernels(row_kernels, HipRowKernels) and not torch.cuda.is_current_stream_capturing()
 
 
@@ -143,7 +144,7 @@ def mean_last(x, keepdim, offset=None):
 
 
 class layer_norm_autograd(torch.autograd.Function):
-    """layer_norm over the last n values of each row on a swapped kernel object; weight and bias of n values or None."""
+    """layer_norm over the last n values of each row by the kernel object's methods; weight and bias of n values or None."""
 
     @staticmethod
     def forward(ctx, rows, weight, bias, eps, offset, approx_bwd):
@@ -272,7 +273,7 @@ def conv2d(X, W, stride, padding, offset=None, approx_bwd=False, groups=1):
 # ---------------------------------------------------------------- linear with the bias added in the product's epilogue
 
 class linear_autograd(torch.autograd.Function):
-    """X W^T + bias in one kernel, with the gradients' products on a swapped kernel object."""
+    """X W^T + bias in one kernel, with the gradients' products by the kernel object's methods."""
 
     @staticmethod
     def forward(ctx, X, W, bias, offset, approx_bwd):

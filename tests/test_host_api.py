@@ -503,3 +503,25 @@ def test_build_links_the_library_without_the_host_modules_needs(monkeypatch, tmp
     with pytest.raises(RuntimeError, match="g\\+\\+"):
         builder.build()
     assert any("-shared" in cmd and str(builder.LIB) in cmd for cmd in ran) and not builder.HOST.exists()
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+@pytest.mark.parametrize("op", ["linear", "matmul", "bmm", "softmax", "log_softmax", "layer_norm"])
+def test_traced_functions_compute_on_new_inputs(op):
+    """torch.jit.trace records the ops: a traced function gives on other inputs, forward and backward, what the ops give."""
+    torch.manual_seed(4)
+    new = lambda *shape: torch.randn(*shape, device="cuda")
+    w, b, right = new(24, 40), new(24), new(3, 40, 7)
+    f = {"linear": lambda x: pam_amd.linear(x, w, b, approx_bwd=True), "matmul": lambda x: pam_amd.matmul(x[0], w.t(), approx_bwd=True),
+         "bmm": lambda x: pam_amd.bmm(x, right, approx_bwd=True), "softmax": lambda x: pam_amd.softmax(x, dim=-1, approx_bwd=True),
+         "log_softmax": lambda x: pam_amd.log_softmax(x, dim=-1, approx_bwd=True),
+         "layer_norm": lambda x: pam_amd.layer_norm(x, 40, w[0], w[1], approx_bwd=True)}[op]
+    for grad in (False, True):
+        traced = torch.jit.trace(f, (new(3, 6, 40).requires_grad_(grad),), check_trace=False)
+        x = new(3, 6, 40)
+        assert torch.equal(traced(x), f(x))
+        if grad:
+            x = x.requires_grad_()
+            dy = torch.randn_like(f(x))
+            assert torch.equal(torch.autograd.grad(traced(x), x, dy)[0], torch.autograd.grad(f(x), x, dy)[0])
