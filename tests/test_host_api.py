@@ -525,3 +525,15 @@ def test_traced_functions_compute_on_new_inputs(op):
             x = x.requires_grad_()
             dy = torch.randn_like(f(x))
             assert torch.equal(torch.autograd.grad(traced(x), x, dy)[0], torch.autograd.grad(f(x), x, dy)[0])
+
+
+@pytest.mark.gpu
+def test_rows_of_a_tensor_subclass_keep_their_class():
+    """softmax, log_softmax and layer_norm of a subclass are of that class, of a Parameter ordinary tensors."""
+    class Marked(torch.Tensor):
+        pass
+    x, w = torch.randn(6, 40, device="cuda"), torch.randn(40, device="cuda")
+    for f in (lambda t: pam_amd.softmax(t, dim=-1), lambda t: pam_amd.log_softmax(t, dim=-1), lambda t: pam_amd.layer_norm(t, 40, w, w)):
+        got = f(x.as_subclass(Marked))
+        assert type(got) is Marked and torch.equal(got.as_subclass(torch.Tensor), f(x))
+        assert type(f(torch.nn.Parameter(x))) is torch.Tensor
