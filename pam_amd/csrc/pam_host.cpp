@@ -162,17 +162,14 @@ std::pair<Tensor, Tensor> column_sums(const Tensor& a, const Tensor& b)
 
 Tensor sum_rows(const Tensor& t) { return summable(t) ? column_sums(t, Tensor()).first : t.sum(0); }
 
-// What `approx_bwd` asks for, per operand of the products (first, second) and for exp and log: 0 the exact gradient, 1 the
-// approximate one, negative neither a flag nor a pair of them, which only a backward pass minds.
+// What `approx_bwd` asks for, per operand of the products (first, second) and for exp and log: the approximate gradient or
+// the exact one.
 struct Approx {
-    int64_t a, b, e;
-    void check() const { TORCH_CHECK_TYPE(a >= 0 && b >= 0 && e >= 0, "approx_bwd must be a bool or a pair of them"); }
+    bool a, b, e;
     void save(AutogradContext* ctx) const { ctx->saved_data["a"] = a; ctx->saved_data["b"] = b; ctx->saved_data["e"] = e; }
     static Approx saved(AutogradContext* ctx)
     {
-        const Approx f{ctx->saved_data["a"].toInt(), ctx->saved_data["b"].toInt(), ctx->saved_data["e"].toInt()};
-        f.check();
-        return f;
+        return Approx{ctx->saved_data["a"].toBool(), ctx->saved_data["b"].toBool(), ctx->saved_data["e"].toBool()};
     }
 };
 
@@ -194,11 +191,11 @@ ProductGrads product_grads(const Tensor& A, const Tensor& B, const Tensor& dY, i
 }
 
 struct MatmulNode : torch::autograd::Function<MatmulNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& A_in, const Tensor& B_in, int64_t dims, double offset, int64_t a, int64_t b)
+    static Tensor forward(AutogradContext* ctx, const Tensor& A_in, const Tensor& B_in, int64_t dims, double offset, bool a, bool b)
     {
         const Tensor A = row_major(A_in, dims), B = row_major(B_in, dims);
         ctx->saved_data["dims"] = dims; ctx->saved_data["offset"] = offset;
-        Approx{a, b, 0}.save(ctx);
+        Approx{a, b, false}.save(ctx);
         ctx->save_for_backward({A, B});
         return product(kPam, A, B, Tensor(), false, Tensor(), offset);
     }
@@ -216,11 +213,11 @@ struct MatmulNode : torch::autograd::Function<MatmulNode> {
 
 // X W^T + bias in one kernel; the gradient of the bias is the sum of the upstream gradient over the rows
 struct LinearNode : torch::autograd::Function<LinearNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& X_in, const Tensor& W, const Tensor& bias, double offset, int64_t a, int64_t b)
+    static Tensor forward(AutogradContext* ctx, const Tensor& X_in, const Tensor& W, const Tensor& bias, double offset, bool a, bool b)
     {
         const Tensor X = row_major(X_in, 2), Wt = row_major(W.t(), 2);
         ctx->saved_data["offset"] = offset;
-        Approx{a, b, 0}.save(ctx);
+        Approx{a, b, false}.save(ctx);
         ctx->save_for_backward({X, Wt});
         return product(kPam, X, Wt, Tensor(), false, bias.contiguous(), offset);
     }
@@ -244,7 +241,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
 // softmax over the last dimension of a contiguous tensor; the gradient is the chain of the primitives' gradients
 // (pam/cuda_bindings.py:43-57, 78-97, 224-239)
 struct SoftmaxNode : torch::autograd::Function<SoftmaxNode> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& x, double offset, int64_t a, int64_t b, int64_t e)
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, double offset, bool a, bool b, bool e)
     {
         check_tensor(x);
         TORCH_CHECK_VALUE(x.dim() >= 1 && x.is_contiguous(), "softmax: expected a contiguous tensor");
@@ -273,7 +270,7 @@ struct SoftmaxNode : torch::autograd::Function<SoftmaxNode> {
         const Tensor dx = new_floats(x.sizes(), x);
         if (x.numel())
             check_call(pam_hip_softmax_bwd(data(x), data(g), data(row_sum), data(shift), data(dx), row_sum.numel(), x.size(-1),
-                                           (float)ctx->saved_data["offset"].toDouble(), f.a != 0, f.b != 0, f.e != 0, on.stream), "softmax_bwd");
+                                           (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, f.e, on.stream), "softmax_bwd");
         return {dx, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
@@ -281,7 +278,7 @@ struct SoftmaxNode : torch::autograd::Function<SoftmaxNode> {
 // layer_norm over the last n values; weight and bias of n values, or undefined
 struct LayerNormNode : torch::autograd::Function<LayerNormNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, int64_t n, const std::optional<Tensor>& weight, const std::optional<Tensor>& bias,
-                          double eps, double offset, int64_t a, int64_t b, int64_t e)
+                          double eps, double offset, bool a, bool b, bool e)
     {
         const Tensor w = weight ? weight->contiguous() : Tensor(), c = bias ? bias->contiguous() : Tensor();
         check_tensor(x);
@@ -317,7 +314,7 @@ struct LayerNormNode : torch::autograd::Function<LayerNormNode> {
         if (x.numel())
             check_call(pam_hip_layer_norm_bwd(data(x), data_or_null(w), data(g), data(dx), data_or_null(terms), rows, n,
                                               (float)ctx->saved_data["eps"].toDouble(), (float)ctx->saved_data["offset"].toDouble(),
-                                              f.a != 0, f.b != 0, f.e != 0, on.stream), "layer_norm_bwd");
+                                              f.a, f.b, f.e, on.stream), "layer_norm_bwd");
         // the broadcast weight and bias collect their gradients by a sum over the rows, as autograd's expand does
         Tensor dw, db;
         const Tensor g_rows = want_b ? g.view({rows, n}) : Tensor();
@@ -400,15 +397,15 @@ PYBIND11_MODULE(_pam_host, module)
         return b ? py::cast(sums) : py::cast(sums.first);
     });
     module.def("sum_rows", &sum_rows, unlocked);
-    module.def("matmul", [](const Tensor& A, const Tensor& B, int64_t dims, double offset, int64_t a, int64_t b) {
+    module.def("matmul", [](const Tensor& A, const Tensor& B, int64_t dims, double offset, bool a, bool b) {
         return MatmulNode::apply(A, B, dims, offset, a, b);
     }, unlocked);
-    module.def("linear", [](const Tensor& X, const Tensor& W, const Tensor& bias, double offset, int64_t a, int64_t b) {
+    module.def("linear", [](const Tensor& X, const Tensor& W, const Tensor& bias, double offset, bool a, bool b) {
         return LinearNode::apply(X, W, bias, offset, a, b);
     }, unlocked);
-    module.def("softmax", [](const Tensor& x, double offset, int64_t a, int64_t b, int64_t e) { return SoftmaxNode::apply(x, offset, a, b, e); }, unlocked);
+    module.def("softmax", [](const Tensor& x, double offset, bool a, bool b, bool e) { return SoftmaxNode::apply(x, offset, a, b, e); }, unlocked);
     module.def("layer_norm", [](const Tensor& x, int64_t n, const std::optional<Tensor>& weight, const std::optional<Tensor>& bias, double eps,
-                                double offset, int64_t a, int64_t b, int64_t e) {
+                                double offset, bool a, bool b, bool e) {
         return LayerNormNode::apply(x, n, weight, bias, eps, offset, a, b, e);
     }, unlocked);
     module.def("adam_collect", &adam_collect);

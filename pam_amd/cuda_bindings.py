@@ -166,32 +166,33 @@ class pam_matmul_autograd(torch.autograd.Function):
         return delta_A, delta_B, None, None, None
 
 
-def approx_codes(approx_bwd):
-    """(first operands, second operands, exp / log) as numbers for the nodes in C++; -1 where it is neither a flag nor a
-    pair, which only a backward pass minds.  The last is the flag's truth value, so a pair counts as set
+_is_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)      # (a call less per op)
+
+
+def node_arguments(kernels, cls, offset, approx_bwd):
+    """What a node in C++ takes of a call: (offset, approximate for the first operands, for the second, for exp and log),
+    or None where the autograd function in Python is to be called: the kernel object is not the package's own or has a
+    method replaced; the call is traced (torch.jit.trace records an autograd function in Python as an operation of its
+    own, but of a node in C++ only the allocation of its output); or an argument is not of the ordinary types, so that it
+    is accepted or refused where and as that function does it.  A pair counts as set for exp and log
     (pam/cuda_bindings.py:227, 267)."""
-    if isinstance(approx_bwd, bool):
-        return approx_bwd, approx_bwd, approx_bwd
-    try:
-        a, b = approx_bwd
-    except (TypeError, ValueError):
-        return -1, -1, -1
-    return bool(a), bool(b), bool(approx_bwd)
-
-
-def own_kernels(kernels, cls):
-    """Whether a node in C++ may stand for a kernel object's methods: the object is the package's own with no method
-    replaced, and the call is not being traced (torch.jit.trace records an autograd function in Python as an operation
-    of its own, but of a node in C++ only the allocation of its output).  Any other call goes to the methods, by the
-    autograd functions in Python."""
-    return type(kernels) is cls and not vars(kernels) and not torch.jit.is_tracing()
+    if type(kernels) is not cls or kernels.__dict__ or _is_tracing():
+        return None
+    if offset is None:
+        offset = 1.0
+    elif not isinstance(offset, (float, int)):
+        return None
+    if type(approx_bwd) is bool:
+        return offset, approx_bwd, approx_bwd, approx_bwd
+    if type(approx_bwd) is tuple and len(approx_bwd) == 2 and type(approx_bwd[0]) is bool and type(approx_bwd[1]) is bool:
+        return offset, *approx_bwd, True
+    return None
 
 
 def _product_node(A, B, offset, approx_bwd, BMM):
-    if own_kernels(cuda_kernels, HipKernels) and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
-        # the node in C++: the same checks, products and formulas
-        a, b, _ = approx_codes(approx_bwd)
-        return host().matmul(A, B, 3 if BMM else 2, _offset_value(offset), a, b)
+    node = node_arguments(cuda_kernels, HipKernels, offset, approx_bwd)
+    if node is not None and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
+        return host().matmul(A, B, 3 if BMM else 2, *node[:3])        # the same checks, products and formulas
     return pam_matmul_autograd.apply(A, B, offset, approx_bwd, BMM)
 
 

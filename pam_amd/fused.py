@@ -16,7 +16,7 @@ import torch
 from . import _abi
 from . import cuda_bindings
 from ._abi import HipKernels, HipRowKernels
-from .cuda_bindings import _both, _offset_value, approx_codes, own_kernels
+from .cuda_bindings import _both, _offset_value, node_arguments
 
 row_kernels = HipRowKernels()
 
@@ -65,9 +65,10 @@ def _ordinary(x):
 def softmax(x, offset=None, approx_bwd=False):
     """softmax over the last dimension; the gradient is the chain of the primitives' gradients
     (pam/cuda_bindings.py:43-57, 78-97, 224-239) in one kernel."""
-    if not (own_kernels(row_kernels, HipRowKernels) and _ordinary(x)):
+    node = node_arguments(row_kernels, HipRowKernels, offset, approx_bwd)
+    if node is None or not _ordinary(x):
         return softmax_autograd.apply(x, offset, approx_bwd)
-    return _abi.host().softmax(x, _offset_value(offset), *approx_codes(approx_bwd))
+    return _abi.host().softmax(x, *node)
 
 
 def _flags(approx_bwd):
@@ -117,7 +118,7 @@ def log_softmax(x, offset=None, approx_bwd=False, check_finite=False):
 def finite_in_kernel():
     """Whether the kernel can report to the host that its input is not finite: not while a graph is recorded or the
     call is traced, and not asked of a swapped kernel object."""
-    return own_kernels(row_kernels, HipRowKernels) and not torch.cuda.is_current_stream_capturing()
+    return node_arguments(row_kernels, HipRowKernels, None, False) is not None and not torch.cuda.is_current_stream_capturing()
 
 
 class mean_autograd(torch.autograd.Function):
@@ -174,10 +175,11 @@ class layer_norm_autograd(torch.autograd.Function):
 
 def layer_norm(x, n, weight, bias, eps, offset=None, approx_bwd=False):
     """layer_norm over the last n values of each row; weight and bias of n values or None."""
-    if not (own_kernels(row_kernels, HipRowKernels) and _ordinary(x)):
+    node = node_arguments(row_kernels, HipRowKernels, offset, approx_bwd)
+    if node is None or not _ordinary(x):
         w, b = (None if t is None else t.reshape(-1) for t in (weight, bias))
         return layer_norm_autograd.apply(x.reshape(-1, n), w, b, eps, offset, approx_bwd).view(x.shape)
-    return _abi.host().layer_norm(x, n, weight, bias, eps, _offset_value(offset), *approx_codes(approx_bwd))
+    return _abi.host().layer_norm(x, n, weight, bias, eps, *node)
 
 
 # ---------------------------------------------------------------- power with a scalar exponent
@@ -311,7 +313,7 @@ class linear_autograd(torch.autograd.Function):
 def linear_with_bias(X2d, W, bias, offset=None, approx_bwd=False):
     """X W^T + bias in one kernel; the gradients are those of the product
     (pam/cuda_bindings.py:132-166) and, for the bias, the sum of the upstream gradient over the rows."""
-    if not own_kernels(cuda_bindings.cuda_kernels, HipKernels):
+    node = node_arguments(cuda_bindings.cuda_kernels, HipKernels, offset, approx_bwd)
+    if node is None:
         return linear_autograd.apply(X2d, W, bias, offset, approx_bwd)
-    a, b, _ = approx_codes(approx_bwd)
-    return _abi.host().linear(X2d, W, bias, _offset_value(offset), a, b)
+    return _abi.host().linear(X2d, W, bias, *node[:3])

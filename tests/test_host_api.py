@@ -537,3 +537,31 @@ def test_rows_of_a_tensor_subclass_keep_their_class():
         got = f(x.as_subclass(Marked))
         assert type(got) is Marked and torch.equal(got.as_subclass(torch.Tensor), f(x))
         assert type(f(torch.nn.Parameter(x))) is torch.Tensor
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["linear", "matmul", "softmax", "layer_norm"])
+def test_unusual_flags_and_offsets_are_taken_or_refused_where_they_were(op):
+    """approx_bwd is unpacked in the backward pass only: a list or a tensor of two is a pair, anything else that is no flag
+    fails there, with the error of the unpacking, and not in a forward pass.  An offset is whatever float() takes."""
+    torch.manual_seed(6)
+    x, w, b = (torch.randn(*s, device="cuda") for s in ((6, 40), (24, 40), (24,)))
+    f = {"linear": lambda x, **kw: pam_amd.linear(x, w, b, **kw), "matmul": lambda x, **kw: pam_amd.matmul(x, w.t(), **kw),
+         "softmax": lambda x, **kw: pam_amd.softmax(x, dim=-1, **kw), "layer_norm": lambda x, **kw: pam_amd.layer_norm(x, 40, w[0], w[1], **kw)}[op]
+    def gradient(**kw):
+        leaf = x.clone().requires_grad_()
+        y = f(leaf, **kw)
+        return torch.autograd.grad(y, leaf, torch.linspace(-1, 1, y.numel(), device="cuda").view(y.shape))[0]
+    pair = gradient(approx_bwd=(True, False))
+    assert torch.equal(gradient(approx_bwd=[True, False]), pair)
+    if op in ("linear", "matmul"):
+        assert torch.equal(gradient(approx_bwd=torch.tensor([True, False])), pair)
+    for flag, error in ((None, TypeError), (1, TypeError), (np.bool_(True), TypeError), ((True,), ValueError), ((True,) * 3, ValueError)):
+        assert torch.equal(f(x, approx_bwd=flag), f(x))
+        with pytest.raises(error):
+            gradient(approx_bwd=flag)
+    want = f(x, offset=1.0552)
+    for offset in (np.float64(1.0552), np.float32(1.0552), torch.tensor(1.0552)):
+        assert torch.equal(f(x, offset=offset), want)
+    with pytest.raises(ValueError):
+        f(x, offset="x")
