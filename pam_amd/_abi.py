@@ -325,7 +325,8 @@ class HipKernels:
         _check(*ops)
         nd = 3 if batched else 2
         if any(t.dim() != nd for t in ops):
-            raise ValueError(f"matrix product: expected {nd}-D operands")
+            name = ("pam_{}_fwd", "standard_{}", "pam_{}_bwd")[kind].format("bmm" if batched else "matmul")
+            raise ValueError(f"{name}: expected {nd}-D operands")
         return host().product(kind, L, R, M, delta_L, None, float(offset))
 
     def pam_matmul_fwd(self, A, B, A_row_major, B_row_major, offset):

@@ -13,6 +13,8 @@
 
 #include <map>
 #include <mutex>
+#include <sstream>
+#include <string>
 #include <utility>
 
 #include "../../include/pam_hip.h"
@@ -32,7 +34,17 @@ using torch::autograd::variable_list;
 void check_tensor(const Tensor& t)
 {
     TORCH_CHECK(t.is_cuda(), "argument must be a CUDA tensor");                 // CHECK_CUDA, pam/cuda_kernels.cu:8
-    TORCH_CHECK_TYPE(t.scalar_type() == at::kFloat, "PAM kernels compute in float32, got ", c10::toString(t.scalar_type()));
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kFloat, "PAM kernels compute in float32, got torch.", c10::getDtypeNames(t.scalar_type()).first);
+}
+
+// a tensor's shape as Python prints it
+std::string shape(const Tensor& t)
+{
+    std::ostringstream text;
+    text << '(';
+    for (int64_t i = 0; i < t.dim(); ++i) text << (i ? ", " : "") << t.size(i);
+    text << (t.dim() == 1 ? ",)" : ")");
+    return text.str();
 }
 
 void check_call(int rc, const char* name)
@@ -96,11 +108,12 @@ Tensor product(int kind, const Tensor& L, const Tensor& R, const Tensor& other, 
     if (bias.defined()) check_tensor(bias);
     const bool batched = L.dim() == 3;
     static const char* const names[2][3] = {{"pam_matmul_fwd", "standard_matmul", "pam_matmul_bwd"}, {"pam_bmm_fwd", "standard_bmm", "pam_bmm_bwd"}};
-    const char* name = names[batched][kind];
+    const char* name = bias.defined() ? "linear_fwd" : names[batched][kind];
+    TORCH_CHECK_TYPE(kind != kSlope || other.defined(), name, ": the forward operand is missing");
     const int64_t nd = batched ? 3 : 2;
     TORCH_CHECK_VALUE(L.dim() == nd && R.dim() == nd && (!other.defined() || other.dim() == nd), name, ": expected ", nd, "-D operands");
     const int64_t batch = batched ? L.size(0) : 1, m = L.size(-2), k = L.size(-1), n = R.size(-1);
-    TORCH_CHECK_VALUE(k == R.size(-2) && (!batched || batch == R.size(0)), name, ": shapes ", L.sizes(), " and ", R.sizes(), " do not multiply");
+    TORCH_CHECK_VALUE(k == R.size(-2) && (!batched || batch == R.size(0)), name, ": shapes ", shape(L), " and ", shape(R), " do not multiply");
     TORCH_CHECK_VALUE(!other.defined() || (other.size(-2) == m && other.size(-1) == n), name, ": third operand must have the shape of the result");
     TORCH_CHECK_VALUE(!bias.defined() || (bias.numel() == n && bias.is_contiguous()), "linear_fwd: bias must be contiguous with one value per output column");
     const OnDevice on(L);
@@ -126,7 +139,7 @@ Tensor product(int kind, const Tensor& L, const Tensor& R, const Tensor& other, 
         else rc = pam_hip_pam_matmul_bwd(PAM_MAT(L), PAM_MAT(R), PAM_MAT(other), PAM_MAT(out), m, n, k, delta_left, off, scratch, bytes, on.stream);
 #undef PAM_MAT
     }
-    check_call(rc, name);
+    check_call(rc, bias.defined() ? "pam_linear_fwd" : name);
     return out;
 }
 

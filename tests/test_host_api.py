@@ -565,3 +565,23 @@ def test_unusual_flags_and_offsets_are_taken_or_refused_where_they_were(op):
         assert torch.equal(f(x, offset=offset), want)
     with pytest.raises(ValueError):
         f(x, offset="x")
+
+
+@pytest.mark.gpu
+def test_refusals_say_what_they_said():
+    """The checks of the products in C++: kinds of error, names, types and shapes as Python prints them."""
+    K, x, w = _abi.HipKernels(), torch.randn(6, 40, device="cuda"), torch.randn(24, 40, device="cuda")
+    b = torch.randn(24, device="cuda")
+    for call, error, text in (
+            (lambda: K.pam_matmul_fwd(x, w, True, True, 1.0), ValueError, r"pam_matmul_fwd: shapes \(6, 40\) and \(24, 40\) do not multiply"),
+            (lambda: K.pam_bmm_fwd(x, w.t(), True, True, 1.0), ValueError, "pam_bmm_fwd: expected 3-D operands"),
+            (lambda: K.standard_matmul(x[None], w.t(), True, True, 1.0), ValueError, "standard_matmul: expected 2-D operands"),
+            (lambda: K.pam_bmm_fwd(x.expand(2, 6, 40), w.t().expand(3, 40, 24), True, True, 1.0), ValueError, r"shapes \(2, 6, 40\) and \(3, 40, 24\) do not"),
+            (lambda: K.pam_matmul_bwd(x, w.t(), None, True, True, True, 1.0), TypeError, "the forward operand is missing"),
+            (lambda: K.pam_matmul_bwd(x, w.t(), x, True, True, True, 1.0), ValueError, "third operand must have the shape of the result"),
+            (lambda: pam_amd.matmul(x.half(), w.t()), TypeError, "PAM kernels compute in float32, got torch.float16"),
+            (lambda: pam_amd.linear(x, w[:, :39], b), ValueError, r"linear_fwd: shapes \(6, 40\) and \(39, 24\) do not multiply"),
+            (lambda: pam_amd.linear(x, w, b[:23]), ValueError, "linear_fwd: bias must be contiguous with one value per output column"),
+            (lambda: pam_amd.matmul(x, w.t().cpu()), RuntimeError, "argument must be a CUDA tensor")):
+        with pytest.raises(error, match=text):
+            call()
