@@ -121,8 +121,8 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 // without steps where the tiles are whole, 1088 1.08, 2304 1.04, 2049 1.05, 2048 0.95, 1024 0.93, 640 0.88, 512 and less 1.00 to
 // 1.03).  Between the two, in the second and third round, they gain 2 to 3 % in units of twenty and more k-tiles, and in
 // shorter ones that are whole tiles of whole 64 x 64 outputs; elsewhere between -4 and +6 %.  In a launch of several
-// rounds each step must cover more than one k-tile of its unit: units of four or five k-tiles lose 2 to 6 % there, and the
-// exact gradients', with three operations per product, those of up to seven (beyond three rounds nine) 2 to 10 %.
+// rounds each step must cover more than one k-tile of its unit: units of four or five k-tiles lose 2 to 6 % there, and of the
+// exact gradients', with three operations per product, those of up to seven in the third round and up to nine beyond, 2 to 10 %.
 // On 4151 products of drawn shapes, geometric mean of the time over that without steps: always 0.989, this rule 0.980, the
 // better of the two each time 0.979.
 bool priority_steps(const Plan& p, long M, long N, bool exact)

@@ -86,8 +86,9 @@ struct Operand { const float* p; long sb, sr, sk; };    // batch, row (the non-k
 // consecutive, 16-byte aligned values of an image row and always inside the image, and the loader fetches them as one.
 // `row_quads`: horizontal stride 1 and an output width that is a multiple of four: four consecutive output positions are
 // then four consecutive pixels of one image row under every k, and the loader works out one address and one row test per
-// four values and hands the staging 128-bit vectors along the positions (padding allowed: the ends of a row are tested
-// per value).
+// four values and hands the staging 128-bit vectors along the positions.  Padding is allowed: the forward product and the
+// input gradient move a quad that reaches over a row's end to its place (image_quad, settle), the weight gradient tests
+// the values one by one.  Image rows of fewer than four values take the loader value by value.
 struct ConvGeom { const int2* ktab; const int2* ltab; int H, W; int transposed; int quads; int row_quads; };
 
 struct GemmArgs {
