@@ -214,8 +214,8 @@ __global__ __launch_bounds__(128) void fold_kernel(pamgemm::GemmArgs g)
 // (The general definition for such tiles was up to 45 % slower than the matrix kernel with its paths for zeros: 256 of 1 x 120,
 // k = 64, a third of the right operand zeros 12.2 us, matrix kernel 10.2, now 5.3; 1600 of 4 x 64, k = 512 156, 121, 74.)
 // Other values outside the window (subnormal, infinite, huge, tiny) take the general definition: 100 us at the latter, 207
-// in the matrix kernel.  With up to four rows this kernel was the faster one in every class of values at thirteen shapes, 1.4 to
-// 4.5 times.  A plan that cuts k (k of 256 and more on fewer than 1536 tiles) goes to the matrix kernel, whose pieces the
+// in the matrix kernel.  With up to four rows this kernel was the faster one in every class of values at eleven shapes, 1.6 to
+// 4 times.  A plan that cuts k (k of 256 and more on fewer than 1536 tiles) goes to the matrix kernel, whose pieces the
 // sums follow; beyond kFewLongest nothing was measured.
 constexpr int kFewRows = 4, kFewDepth = 64;
 constexpr long kFewLongest = 512;
