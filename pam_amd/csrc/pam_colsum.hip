@@ -1,18 +1,22 @@
 // Sums over the rows of a matrix (the gradients of biases and of layer_norm's parameters): ordinary float32 additions.
 //
-// Bound by memory, one read of the matrix.  A work-group of 256 lanes takes 64 columns of a range of rows: 16 lanes with
-// 128-bit loads side by side (256 contiguous bytes of a row) and 16 rows at a time, eight loads in flight per lane, the
-// sixteen lanes of a column added through LDS in a tree.  Where one range of rows would leave compute units without work
-// the rows are cut into ranges of at least kLeastRows, whose sums go to the workspace and are added by the same kernel in
-// a second launch.  Two matrices of one shape can be summed in one launch.
+// Bound by memory, one read of the matrix.  A work-group of 256 lanes takes up to 64 columns of a range of rows: WIDE lanes with
+// 128-bit loads side by side (at most 256 contiguous bytes of a row; as few as cover the matrix) and 256 / WIDE rows at a time,
+// eight loads in flight per lane, the lanes of a column added through LDS in a tree.  Where the rows keep a lane busy for more
+// than four such rounds they are cut into ranges of at least one round, whose sums go to the workspace and are added by the
+// same kernel in a second launch (2 us: one launch of four rounds is no slower).  Two matrices of one shape can be summed in
+// one launch.
 // Rounding: the eight loaded values are added as a tree and the trees' sums in a cascade, kChain at a time on each of
 // kLevels levels, so that a value passes through fewer than 64 rounded additions at the sizes of a model's gradients and
 // fewer than 100 in any matrix of up to 2^31 values, however long a lane's share of the rows is (many columns leave no
 // work-groups to cut the rows for: 4096 rows of 131073 equal values near 1 in one chain per lane were off by 1.5e-5, now by
 // less than 4e-6).  The order depends on the two sizes alone: not on a second matrix beside, nor on strides or alignment
-// (128-bit loads at any float's address; n that are no multiple of four take one value per load).
-// Measured against torch's sum over dim 0 (which also clears a buffer first, 5 us): a linear layer of 12608 x 192 -> 768 with
-// its gradients 277 -> 266 us, 4096 x 512 -> 1024 375 -> 361.
+// (128-bit loads at any float's address; where a row's last loads would pass its end they start earlier and some columns are
+// summed twice alike).
+// Measured against torch's sum over dim 0 (which clears a buffer first where it cuts the rows), us: 96 x 128 3.3 (torch 4.2),
+// 256 x 64 3.5 (5.0), 4096 x 1024 5.7 (20), 12608 x 768 12.6 (26), 65536 x 1024 twice 94, 4096 x 10000 34 (181), 10^6 x 1
+// 5.8 (10.7), 10^6 x 10 14 (22); with sixteen lanes across whatever the width, and cut from 256 rows on, the last two took
+// 35 and 39 and 256 x 64 5.2.  A linear layer of 12608 x 192 -> 768 with its gradients 277 -> 266 us with these sums, 4096 x 512 -> 1024 375 -> 361.
 #include <algorithm>
 #include <cstdint>
 
@@ -22,28 +26,25 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kColumns = 64;            // per work-group
-constexpr long kLeastRows = 128;        // per range
+constexpr int kFlight = 8;              // loads in flight per lane: a round
 constexpr long kMostGroups = 2048;      // work-groups per matrix of a launch that cuts the rows: eight per compute unit
 constexpr int kChain = 16, kLevels = 4;
 
 struct Sums { const float* in[2]; float* out[2]; long row_stride[2]; };
 
-// VEC: values per lane and load.  Work-group (x, y, z): columns x * 64 ..., range y of the rows, matrix z; the sums of
-// range y go to out[z] + y * n.
-template <int VEC>
+// VEC: values per lane and load, WIDE: lanes per row.  Work-group (x, y, z): the x-th VEC * WIDE columns, range y of the rows,
+// matrix z; the sums of range y go to out[z] + y * n.  n is at least VEC.
+template <int VEC, int WIDE>
 __global__ __launch_bounds__(kThreads) void column_sums_kernel(Sums s, long rows, long n, long range)
 {
-    constexpr int kWide = kColumns / VEC, kDeep = kThreads / kWide;
-    constexpr int kFlight = 8;
+    constexpr int kColumns = VEC * WIDE, kDeep = kThreads / WIDE;
     typedef float vec __attribute__((ext_vector_type(VEC)));
     typedef float vec_any __attribute__((ext_vector_type(VEC), aligned(4)));
-    __shared__ __attribute__((aligned(16))) float part[kDeep][kColumns];
-    const int tx = threadIdx.x % kWide, ty = threadIdx.x / kWide;
-    const long column = (long)blockIdx.x * kColumns + tx * VEC;
+    __shared__ float part[kDeep][kColumns];
+    const int tx = threadIdx.x % WIDE, ty = threadIdx.x / WIDE;
+    const long base = (long)blockIdx.x * kColumns, column = min(base + tx * VEC, n - VEC);
     const long first = (long)blockIdx.y * range, last = min(rows, first + range);
-    const bool inside = column + VEC <= n;          // (VEC = 4 takes only n that are multiples of four)
-    const float* at = s.in[blockIdx.z] + (inside ? column : 0);
+    const float* at = s.in[blockIdx.z] + column;
     const long stride = s.row_stride[blockIdx.z];
     vec level[kLevels] = {};
     unsigned trees = 0;
@@ -63,33 +64,49 @@ __global__ __launch_bounds__(kThreads) void column_sums_kernel(Sums s, long rows
     for (; r < last; r += kDeep) total += *reinterpret_cast<const vec_any*>(at + r * stride);
 #pragma unroll
     for (int l = 0; l < kLevels; ++l) total += level[l];
-    *reinterpret_cast<vec*>(&part[ty][tx * VEC]) = total;
+    union { vec v; float f[VEC]; } sums;
+    sums.v = total;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)                   // (a lane that starts earlier writes what its neighbour does)
+        if (column + e >= base) part[ty][column + e - base] = sums.f[e];
     for (int half = kDeep / 2; half >= 1; half /= 2) {
         __syncthreads();
         for (int i = threadIdx.x; i < half * kColumns; i += kThreads) part[i / kColumns][i % kColumns] += part[i / kColumns + half][i % kColumns];
     }
     __syncthreads();
-    if (threadIdx.x < kColumns) {
-        const long c = (long)blockIdx.x * kColumns + threadIdx.x;
-        if (c < n) s.out[blockIdx.z][(long)blockIdx.y * n + c] = part[0][threadIdx.x];
-    }
+    if (threadIdx.x < kColumns && base + threadIdx.x < n) s.out[blockIdx.z][(long)blockIdx.y * n + base + threadIdx.x] = part[0][threadIdx.x];
+}
+
+// values per load and lanes per row for n columns: the narrowest that covers them, up to 64 columns
+struct Lanes { int vec, wide; int columns() const { return vec * wide; } };
+Lanes lanes_for(long n)
+{
+    const int vec = n < 4 ? 1 : 4;
+    int wide = 1;
+    while (wide < 16 && (long)vec * wide < n) wide *= 2;
+    return Lanes{vec, wide};
 }
 
 // rows per range and number of ranges
 struct Cut { long range, ranges; };
 Cut cut_rows(long rows, long n)
 {
-    const long groups = (n + kColumns - 1) / kColumns;
-    const long most = std::max(1L, std::min({rows / kLeastRows, kMostGroups / groups, 65535L}));
+    const Lanes l = lanes_for(n);
+    const long round = (long)kFlight * (kThreads / l.wide), groups = (n + l.columns() - 1) / l.columns();
+    if (rows <= 4 * round) return Cut{rows, 1};
+    const long most = std::max(1L, std::min({rows / round, kMostGroups / groups, 65535L}));
     const long range = (rows + most - 1) / most;
     return Cut{range, (rows + range - 1) / range};
 }
 
 void launch(const Sums& s, int matrices, long rows, long n, const Cut& cut, hipStream_t st)
 {
-    const dim3 grid((unsigned)((n + kColumns - 1) / kColumns), (unsigned)cut.ranges, (unsigned)matrices);
-    if (n % 4 == 0) hipLaunchKernelGGL(column_sums_kernel<4>, grid, dim3(kThreads), 0, st, s, rows, n, cut.range);
-    else hipLaunchKernelGGL(column_sums_kernel<1>, grid, dim3(kThreads), 0, st, s, rows, n, cut.range);
+    const Lanes l = lanes_for(n);
+    const dim3 grid((unsigned)((n + l.columns() - 1) / l.columns()), (unsigned)cut.ranges, (unsigned)matrices);
+#define PAM_COLUMN_SUMS(V, W) if (l.vec == V && l.wide == W) { hipLaunchKernelGGL((column_sums_kernel<V, W>), grid, dim3(kThreads), 0, st, s, rows, n, cut.range); return; }
+    PAM_COLUMN_SUMS(4, 16) PAM_COLUMN_SUMS(4, 8) PAM_COLUMN_SUMS(4, 4) PAM_COLUMN_SUMS(4, 2) PAM_COLUMN_SUMS(4, 1)
+    PAM_COLUMN_SUMS(1, 4) PAM_COLUMN_SUMS(1, 2) PAM_COLUMN_SUMS(1, 1)
+#undef PAM_COLUMN_SUMS
 }
 
 }  // namespace

@@ -681,7 +681,9 @@ def test_finite_check_under_a_default_device():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,n", [(1, 1), (2, 4), (127, 64), (128, 68), (257, 63), (300, 192), (4097, 20), (12608, 768), (70001, 3), (3, 30011)])
+@pytest.mark.parametrize("rows,n", [(1, 1), (2, 4), (127, 64), (128, 68), (257, 63), (300, 192), (4097, 20), (12608, 768), (70001, 3), (3, 30011),
+                                    (9, 2), (8192, 1), (8193, 1), (200001, 2), (4, 4), (8193, 4), (5000, 5), (4097, 6), (2049, 9), (2048, 16), (1025, 31), (1024, 33),
+                                    (512, 65), (513, 66), (511, 67), (1000, 129)])
 def test_column_sums(rows, n):
     """Sums over the rows against 64-bit ones, on both load widths, on rows apart from each other and for two matrices in
     one call.  A value takes part in fewer than 64 rounded additions at these sizes (per pass a tree of eight or a rest of
