@@ -56,17 +56,16 @@ class softmax_autograd(torch.autograd.Function):
         return dx.view(grad.shape), None, None
 
 
-def _ordinary(x):
-    """Whether the result of an op on x is an ordinary tensor: one of a subclass has a result of that class, which the
-    autograd functions in Python make (torch.empty_like keeps the class)."""
-    return type(x) is torch.Tensor or type(x) is torch.nn.Parameter
+# The classes whose results are ordinary tensors: an op on a tensor of another class has a result of that class, which the
+# autograd functions in Python make (torch.empty_like keeps the class).
+_ORDINARY = (torch.Tensor, torch.nn.Parameter)
 
 
 def softmax(x, offset=None, approx_bwd=False):
     """softmax over the last dimension; the gradient is the chain of the primitives' gradients
     (pam/cuda_bindings.py:43-57, 78-97, 224-239) in one kernel."""
     node = node_arguments(row_kernels, HipRowKernels, offset, approx_bwd)
-    if node is None or not _ordinary(x):
+    if node is None or type(x) not in _ORDINARY:
         return softmax_autograd.apply(x, offset, approx_bwd)
     return _abi.host().softmax(x, *node)
 
@@ -176,7 +175,7 @@ class layer_norm_autograd(torch.autograd.Function):
 def layer_norm(x, n, weight, bias, eps, offset=None, approx_bwd=False):
     """layer_norm over the last n values of each row; weight and bias of n values or None."""
     node = node_arguments(row_kernels, HipRowKernels, offset, approx_bwd)
-    if node is None or not _ordinary(x):
+    if node is None or type(x) not in _ORDINARY:
         w, b = (None if t is None else t.reshape(-1) for t in (weight, bias))
         return layer_norm_autograd.apply(x.reshape(-1, n), w, b, eps, offset, approx_bwd).view(x.shape)
     return _abi.host().layer_norm(x, n, weight, bias, eps, *node)

@@ -93,9 +93,10 @@ def matmul(A, B, *, offset=None, approx_bwd=False, use_kernel=True):
 
 def bmm(A, B, *, offset=None, approx_bwd=False, use_kernel=True):
     """pam/pam_ops.py:89-104"""
-    assert A.dim() == B.dim() == 3
-    assert A.shape[0] == B.shape[0]
-    assert A.shape[2] == B.shape[1]
+    a, b = A.shape, B.shape
+    assert len(a) == len(b) == 3
+    assert a[0] == b[0]
+    assert a[2] == b[1]
     _require_kernel(A, use_kernel)
     return cuda_bindings.pam_bmm(A, B, offset=offset, approx_bwd=approx_bwd)
 
@@ -106,7 +107,7 @@ def linear(X, W, bias=None, *, offset=None, approx_bwd=False, use_kernel=True):
     lead = X.shape[:-1]
     rows = X.reshape(-1, X.shape[-1])
     if (fused_bias and bias is not None and use_kernel and rows.is_cuda and rows.numel() and bias.dim() == 1
-            and all(t.dtype == torch.float32 for t in (rows, W, bias))):
+            and rows.dtype is torch.float32 and W.dtype is torch.float32 and bias.dtype is torch.float32):
         # the bias is added to the finished sums inside the product kernel: the same add, one pass less
         out = fused.linear_with_bias(rows, W, bias, offset, approx_bwd)
         return out.reshape(*lead, out.shape[-1])
