@@ -3,9 +3,9 @@
 // Bound by memory, one read of the matrix.  A work-group of 256 lanes takes up to 64 columns of a range of rows: WIDE lanes with
 // 128-bit loads side by side (at most 256 contiguous bytes of a row; as few as cover the matrix) and 256 / WIDE rows at a time,
 // eight loads in flight per lane, the lanes of a column added through LDS in a tree.  Where the rows keep a lane busy for more
-// than four such rounds they are cut into ranges of at least one round, whose sums go to the workspace and are added by the
-// same kernel in a second launch (2 us: one launch of four rounds is no slower).  Two matrices of one shape can be summed in
-// one launch.
+// than eight such rounds they are cut into ranges of about one round, whose sums go to the workspace and are added by the
+// same kernel in a second launch (which costs what eight rounds do: 1000 x 197 5.3 us in one launch, 6.1 in two).  Two
+// matrices of one shape can be summed in one launch.
 // Rounding: the eight loaded values are added as a tree and the trees' sums in a cascade, kChain at a time on each of
 // kLevels levels, so that a value passes through fewer than 64 rounded additions at the sizes of a model's gradients and
 // fewer than 100 in any matrix of up to 2^31 values, however long a lane's share of the rows is (many columns leave no
@@ -13,10 +13,11 @@
 // less than 4e-6).  The order depends on the two sizes alone: not on a second matrix beside, nor on strides or alignment
 // (128-bit loads at any float's address; where a row's last loads would pass its end they start earlier and some columns are
 // summed twice alike).
-// Measured against torch's sum over dim 0 (which clears a buffer first where it cuts the rows), us: 96 x 128 3.3 (torch 4.2),
-// 256 x 64 3.5 (5.0), 4096 x 1024 5.7 (20), 12608 x 768 12.6 (26), 65536 x 1024 twice 94, 4096 x 10000 34 (181), 10^6 x 1
-// 5.8 (10.7), 10^6 x 10 14 (22); with sixteen lanes across whatever the width, and cut from 256 rows on, the last two took
-// 35 and 39 and 256 x 64 5.2.  A linear layer of 12608 x 192 -> 768 with its gradients 277 -> 266 us with these sums, 4096 x 512 -> 1024 375 -> 361.
+// Measured against torch's sum over dim 0 (which clears a buffer first where it cuts the rows), us: 96 x 128 3.2 (torch 4.2),
+// 256 x 64 3.4 (5.0), 4096 x 1024 5.9 (20), 12608 x 768 10.8 (26), 65536 x 1024 twice 93, 4096 x 10000 34 (181), 10^6 x 1
+// 5.8 (10.7), 10^6 x 10 14 (22).  With sixteen lanes across whatever the width, cut from 256 rows on and a range's odd rows one by
+// one: 256 x 64 5.2, 12608 x 768 12.6 and the last two 35 and 39.  A linear layer of 12608 x 192 -> 768 with its gradients
+// 277 -> 266 us with these sums, 4096 x 512 -> 1024 375 -> 361.
 #include <algorithm>
 #include <cstdint>
 
@@ -28,6 +29,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kFlight = 8;              // loads in flight per lane: a round
 constexpr long kMostGroups = 2048;      // work-groups per matrix of a launch that cuts the rows: eight per compute unit
+constexpr long kRoundsAlone = 8;        // rounds of a lane up to which the rows are not cut
 constexpr int kChain = 16, kLevels = 4;
 
 struct Sums { const float* in[2]; float* out[2]; long row_stride[2]; };
@@ -44,24 +46,32 @@ __global__ __launch_bounds__(kThreads) void column_sums_kernel(Sums s, long rows
     const int tx = threadIdx.x % WIDE, ty = threadIdx.x / WIDE;
     const long base = (long)blockIdx.x * kColumns, column = min(base + tx * VEC, n - VEC);
     const long first = (long)blockIdx.y * range, last = min(rows, first + range);
-    const float* at = s.in[blockIdx.z] + column;
-    const long stride = s.row_stride[blockIdx.z];
-    vec level[kLevels] = {};
+    const long stride = s.row_stride[blockIdx.z], step = stride * kDeep;
+    const float* at = s.in[blockIdx.z] + column + (first + ty) * stride;
+    long left = last - first - ty;                  // rows from the lane's next one to the range's end
+    vec level[kLevels] = {}, v[kFlight];
+    auto tree = [&]() __attribute__((always_inline)) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
     unsigned trees = 0;
-    long r = first + ty;
-    for (; r + (kFlight - 1) * kDeep < last; r += kFlight * kDeep) {
-        vec v[kFlight];
+    for (; left > (kFlight - 1) * kDeep; left -= kFlight * kDeep) {
 #pragma unroll
-        for (int u = 0; u < kFlight; ++u) v[u] = *reinterpret_cast<const vec_any*>(at + (r + u * kDeep) * stride);
-        level[0] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        for (int u = 0; u < kFlight; ++u, at += step) v[u] = *reinterpret_cast<const vec_any*>(at);
+        level[0] += tree();
         ++trees;
-        unsigned whole = kChain;
+        if (trees % kChain == 0) {
+            unsigned whole = kChain;
 #pragma unroll
-        for (int l = 0; l + 1 < kLevels; ++l, whole *= kChain)
-            if (trees % whole == 0) { level[l + 1] += level[l]; level[l] = 0.0f; }
+            for (int l = 0; l + 1 < kLevels; ++l, whole *= kChain)
+                if (trees % whole == 0) { level[l + 1] += level[l]; level[l] = 0.0f; }
+        }
     }
     vec total = 0.0f;
-    for (; r < last; r += kDeep) total += *reinterpret_cast<const vec_any*>(at + r * stride);
+    if (left > 0) {                                 // the rest, all in flight too: rows past the end are the first one again and count as zeros
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) v[u] = *reinterpret_cast<const vec_any*>(at + (u * kDeep < left ? u * step : 0));
+#pragma unroll
+        for (int u = 1; u < kFlight; ++u) if (u * kDeep >= left) v[u] = 0.0f;
+        total = tree();
+    }
 #pragma unroll
     for (int l = 0; l < kLevels; ++l) total += level[l];
     union { vec v; float f[VEC]; } sums;
@@ -93,8 +103,8 @@ Cut cut_rows(long rows, long n)
 {
     const Lanes l = lanes_for(n);
     const long round = (long)kFlight * (kThreads / l.wide), groups = (n + l.columns() - 1) / l.columns();
-    if (rows <= 4 * round) return Cut{rows, 1};
-    const long most = std::max(1L, std::min({rows / round, kMostGroups / groups, 65535L}));
+    if (rows <= kRoundsAlone * round) return Cut{rows, 1};
+    const long most = std::max(1L, std::min({(rows + round - 1) / round, kMostGroups / groups, 65535L}));
     const long range = (rows + most - 1) / most;
     return Cut{range, (rows + range - 1) / range};
 }

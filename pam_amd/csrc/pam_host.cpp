@@ -68,7 +68,7 @@ Tensor new_floats(at::IntArrayRef shape, const Tensor& like) { return at::empty(
 // The matrix products' scratch (pieces of cut tiles, their arrival words): one buffer per device and stream, kept and
 // grown as needed.  Products on one stream run one after the other, and each leaves the arrival words ready for the
 // next one; products on different streams may overlap in time and must not share a buffer.  The lock covers the table
-// only: buffers are allocated and given back outside it, since the allocator may wait for the driver or for the
+// only: buffers are allocated and given back outside it, since the allocator may wait for the device or for the
 // interpreter (its hooks), which another thread that waits for the lock might hold.
 Tensor gemm_workspace(const Tensor& like, void* stream, size_t bytes)
 {
@@ -393,7 +393,7 @@ py::tuple adam_collect(py::list params, size_t start, py::dict state)
 }  // namespace
 
 // The interpreter is free for other threads while an op checks, allocates and launches, each of which may wait (a full
-// launch queue, the driver, the table of workspaces); only adam_collect reads Python objects.
+// launch queue, device memory, the table of workspaces); only adam_collect reads Python objects.
 PYBIND11_MODULE(_pam_host, module)
 {
     const py::call_guard<py::gil_scoped_release> unlocked;

@@ -686,8 +686,8 @@ def test_finite_check_under_a_default_device():
                                     (512, 65), (513, 66), (511, 67), (1000, 129)])
 def test_column_sums(rows, n):
     """Sums over the rows against 64-bit ones, on both load widths, on rows apart from each other and for two matrices in
-    one call.  A value takes part in fewer than 64 rounded additions at these sizes (per pass a tree of eight or a rest of
-    up to seven, chains of sixteen, a tree over the lanes), each off by 2^-24 of a partial sum that is at most the sum of
+    one call.  A value takes part in fewer than 64 rounded additions at these sizes (per pass a tree of eight, chains of
+    sixteen, a tree over the lanes), each off by 2^-24 of a partial sum that is at most the sum of
     magnitudes.  The bits depend on the sizes alone."""
     from pam_amd import _abi
     g = torch.Generator().manual_seed(rows + n)
