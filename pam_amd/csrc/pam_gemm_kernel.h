@@ -65,7 +65,9 @@ namespace pamgemm {
 using namespace pamdev;
 
 enum { MODE_PAM = 0, MODE_STD = 1, MODE_BWD_DL = 2, MODE_BWD_DR = 3 };
-enum { LOAD_KVEC = 0, LOAD_RVEC = 1, LOAD_ANY = 2, LOAD_CONV = 3, LOAD_CONVQ = 4, LOAD_CONVR = 5, LOAD_CONVK = 6 };   // k contiguous / row contiguous / any strides / image patches / ... in quads along k / ... in quads of output positions / the same, transposed
+enum { LOAD_KVEC = 0, LOAD_RVEC = 1, LOAD_ANY = 2, LOAD_CONV = 3, LOAD_CONVQ = 4, LOAD_CONVR = 5, LOAD_CONVK = 6, LOAD_KODD = 7, LOAD_RODD = 8 };
+// k contiguous / row contiguous (lines of whole, aligned quads) / any strides / image patches / ... in quads along k / ... in quads of
+// output positions / the same, transposed / k contiguous / row contiguous, lines of any length from four on, at any float's address
 
 constexpr int KGRAN = 32;         // k ranges handed to work-groups are multiples of this
 constexpr int PAD = 4;
@@ -178,13 +180,19 @@ constexpr uint32_t kStandInR = 64u << 23;
 template <int BK>
 __device__ __forceinline__ int swizzled(int row, int k) { return BK == 32 ? row ^ ((k & 16) >> 1) : row; }
 
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));      // at any float's address
+__device__ __forceinline__ float4 any_quad(const float* p)
+{
+    const v4f_any q = *reinterpret_cast<const v4f_any*>(p);
+    return make_float4(q.x, q.y, q.z, q.w);
+}
+
 // Four consecutive values of an image row for a patch entry (tables above), zeros where the row or the column lies outside:
 // one 128-bit load from where the quad lies inside the row, in image_quad, and `settle`, which moves it to its place by
 // selects when the values are staged (done at once they would wait for the load there) -- a quad reaches at most a kernel's
 // width over the row's ends, almost always by one.  (Four loads, each with its own test, address and execution mask, were
 // a quarter of the vector instructions of a 3 x 3 convolution: 1442 -> 1390 us, forward and both gradients of 128 images of
 // 64 x 32 x 32 to 128 channels.)  W is at least 4.
-typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));      // at any float's address
 __device__ __forceinline__ float4 image_quad(const float* base, const ConvGeom& cv, const int2 ke, const int2 le, int& over)
 {
     const int h = (le.y >> 16) + (ke.y >> 16), w = (int)(short)(le.y & 0xffff) + (ke.y & 0xffff);
@@ -205,14 +213,20 @@ __device__ __forceinline__ float4 settle(const float4 q, int over)
     return make_float4(none || down2 ? 0.0f : up2 ? z : x, none || down2 ? 0.0f : up2 ? w : y, none || up2 ? 0.0f : down2 ? x : z, none || up2 ? 0.0f : down2 ? y : w);
 }
 
+// Four values read `early` places before where they were wanted, moved there; what lies beyond the line's end repeats its last value.
+__device__ __forceinline__ float4 last_values(const float4 q, int early)
+{
+    return make_float4(early <= 0 ? q.x : early == 1 ? q.y : early == 2 ? q.z : q.w, early <= 0 ? q.y : early == 1 ? q.z : q.w, early <= 0 ? q.z : q.w, q.w);
+}
+
 // One operand's tile: ROWS x BK values from global memory into registers, then into LDS.
 template <int ROWS, int NT, int KIND, int BK>
 struct TileLoader {
     static constexpr int kVecs = ROWS * BK / 4 / NT;      // float4 per lane (vector kinds)
     static constexpr int kElems = ROWS * BK / NT;         // scalars per lane (generic kind)
     static_assert(ROWS * BK % (4 * NT) == 0 && NT % ROWS == 0, "tile must divide over the work-group");
-    static constexpr bool kKQuads = KIND == LOAD_KVEC || KIND == LOAD_CONVQ || KIND == LOAD_CONVK;      // 128-bit loads along k
-    static constexpr bool kRQuads = KIND == LOAD_RVEC || KIND == LOAD_CONVR;      // ... along the rows
+    static constexpr bool kKQuads = KIND == LOAD_KVEC || KIND == LOAD_KODD || KIND == LOAD_CONVQ || KIND == LOAD_CONVK;      // 128-bit loads along k
+    static constexpr bool kRQuads = KIND == LOAD_RVEC || KIND == LOAD_RODD || KIND == LOAD_CONVR;      // ... along the rows
     float4 v[kVecs > 0 ? kVecs : 1];
     int2 fixed; bool have_fixed = false;          // LOAD_CONV: the lane's own table entry
     int patch_at[kVecs > 0 ? kVecs : 1];          // LOAD_CONVQ: where the patches of the lane's rows begin in the image
@@ -220,12 +234,22 @@ struct TileLoader {
 
     int over[KIND == LOAD_CONVR && kVecs > 0 ? kVecs : 1];      // LOAD_CONVR: how far the quads reach over the row's ends
 
-    // before the loaded values are looked at
-    __device__ __forceinline__ void arrive()
+    // before the loaded values are looked at: quads that were read from another place than their own are moved to it
+    __device__ __forceinline__ void arrive(int row0, int nrows, int k0, int kend, int tid)
     {
         if (KIND == LOAD_CONVR) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) v[i] = settle(v[i], over[i]);
+        }
+        // A quad that straddles the end of its line (only where that is no multiple of four, in the last tile) was read up to
+        // the end: its first values are the last ones read.
+        if (KIND == LOAD_KODD && (kend & 3) != 0 && k0 + BK > kend) {
+#pragma unroll
+            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], k0 + ((tid + i * NT) % (BK / 4)) * 4 - (kend - 4));
+        }
+        if (KIND == LOAD_RODD && (nrows & 3) != 0 && row0 + ROWS > nrows) {
+#pragma unroll
+            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], row0 + ((tid + i * NT) % (ROWS / 4)) * 4 - (nrows - 4));
         }
     }
 
@@ -298,23 +322,25 @@ struct TileLoader {
                 const int k = min(k0 + ((tid + i * NT) % (BK / 4)) * 4, kend - 4);
                 v[i] = *reinterpret_cast<const float4*>(base + patch_at[i] + ktab[2 * k]);
             }
-        } else if (KIND == LOAD_KVEC) {
+        } else if (KIND == LOAD_KVEC || KIND == LOAD_KODD) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
                 int id = tid + i * NT;
                 int r = id / (BK / 4), kq = id % (BK / 4);
                 int row = min(row0 + r, nrows - 1);
                 int k = min(k0 + kq * 4, kend - 4);
-                v[i] = *reinterpret_cast<const float4*>(base + (long)row * op.sr + k);
+                const float* at = base + (long)row * op.sr + k;
+                v[i] = KIND == LOAD_KODD ? any_quad(at) : *reinterpret_cast<const float4*>(at);
             }
-        } else if (KIND == LOAD_RVEC) {
+        } else if (KIND == LOAD_RVEC || KIND == LOAD_RODD) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
                 int id = tid + i * NT;
                 int k = id / (ROWS / 4), rq = id % (ROWS / 4);
                 int row = min(row0 + rq * 4, nrows - 4);
                 int kk = min(k0 + k, kend - 1);
-                v[i] = *reinterpret_cast<const float4*>(base + (long)kk * op.sk + row);
+                const float* at = base + (long)kk * op.sk + row;
+                v[i] = KIND == LOAD_RODD ? any_quad(at) : *reinterpret_cast<const float4*>(at);
             }
         } else {
             float* s = reinterpret_cast<float*>(v);
@@ -865,8 +891,8 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
     TileLoader<BM, NT, LKIND, BK> ll;
     TileLoader<BN, NT, RKIND, BK> rl;
 
-    auto stage = [&](int buf) __attribute__((always_inline)) {
-        ll.arrive(); rl.arrive();
+    auto stage = [&](int buf, int k0) __attribute__((always_inline)) {
+        ll.arrive(row0, g.M, k0, kend, tid); rl.arrive(col0, g.N, k0, kend, tid);
         PlainStager<false> same{0u};
         if (MODE == MODE_STD) {
             ll.store(lds_l[buf], tid, same);
@@ -915,7 +941,7 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
     if (ktiles > 0) {
         ll.load(g.L, lbase, row0, g.M, kbegin, kend, tid, g.cv);
         rl.load(g.R, rbase, col0, g.N, kbegin, kend, tid, g.cv);
-        stage(0);
+        stage(0, kbegin);
     }
     __syncthreads();
 
@@ -957,7 +983,7 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
         sr = lds_r[cur] + tx * 4; srx = lds_r[cur] + swizzled<BK>(tx * 4, 16);
     };
     auto end_tile = [&](int t) __attribute__((always_inline)) {
-        if (t + 1 < ktiles) stage((t & 1) ^ 1);
+        if (t + 1 < ktiles) stage((t & 1) ^ 1, kbegin + (t + 1) * BK);
         __syncthreads();
     };
 
@@ -1375,6 +1401,9 @@ void launch_gemm(int lk, int rk, unsigned groups, hipStream_t st, const GemmArgs
     PAM_GEMM_CASE(LOAD_KVEC, LOAD_ANY)
     PAM_GEMM_CASE(LOAD_RVEC, LOAD_KVEC) PAM_GEMM_CASE(LOAD_RVEC, LOAD_ANY)
     PAM_GEMM_CASE(LOAD_ANY, LOAD_KVEC) PAM_GEMM_CASE(LOAD_ANY, LOAD_RVEC) PAM_GEMM_CASE(LOAD_ANY, LOAD_ANY)
+    if constexpr (MODE != MODE_STD) {                                  // lines at any float's address
+        PAM_GEMM_CASE(LOAD_KODD, LOAD_KODD) PAM_GEMM_CASE(LOAD_KODD, LOAD_RODD) PAM_GEMM_CASE(LOAD_RODD, LOAD_KODD) PAM_GEMM_CASE(LOAD_RODD, LOAD_RODD)
+    }
     if constexpr (MODE != MODE_STD) {                                  // image patches as the right operand
         PAM_GEMM_CASE(LOAD_KVEC, LOAD_CONV) PAM_GEMM_CASE(LOAD_RVEC, LOAD_CONV) PAM_GEMM_CASE(LOAD_ANY, LOAD_CONV)
         if constexpr (MODE == MODE_PAM) { PAM_GEMM_CASE(LOAD_KVEC, LOAD_CONVQ) }      // (forward products of patch embeddings)

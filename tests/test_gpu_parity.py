@@ -800,3 +800,29 @@ def test_few_rows_with_zeros(oracle, batch, m, n, k, where):
     assert plan == 0 or plan >= k
     for right in (b, b.transpose(1, 2).contiguous().transpose(1, 2)):
         assert_same_bits(H.product(0, a, right, None, False, None, 1.0).cpu().numpy(), want, where)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("specials", [False, True])
+@pytest.mark.parametrize("batch,m,k,n", [(3, 4, 4, 4), (2, 5, 6, 7), (2, 67, 63, 65), (1, 66, 33, 129), (2, 130, 197, 61), (1, 65, 515, 66), (1, 5, 4, 66)])
+def test_lines_of_any_length_and_address(K, oracle, batch, m, k, n, specials):
+    """Operands contiguous along one index whose lines are no whole quads, begin at any float and lie any number of floats
+    apart: the quad over a line's end, in whole tiles and in the last piece of a cut one, forward and exact gradients."""
+    def views(a):
+        b, r, c = a.shape
+        t = torch.from_numpy(a).cuda()
+        apart = torch.zeros(b * (r + 1) * (c + 3) + 1, device="cuda")[1:].view(b, r + 1, c + 3)[:, 1:, 2:c + 2]
+        apart.copy_(t)
+        return [t, t.transpose(1, 2).contiguous().transpose(1, 2), apart]
+    def operand(rows, cols, seed):
+        return np.stack([_sparse_specials((rows, cols), seed + b, zero_band=(1, 0, min(cols, 9))) if specials else _rand((rows, cols), seed + b, 0.0, False)
+                         for b in range(batch)])
+    A, B, D = operand(m, k, 11), operand(k, n, 23), operand(m, n, 37)
+    D = np.where(np.isfinite(D), D, 1.0).astype(np.float32)
+    want = ogemm(oracle, A, B)
+    slopes = {left: ogemm(oracle, A, B, mode=oracle.MODE_BWD_DELTA_L if left else oracle.MODE_BWD_DELTA_R, D=D) for left in (True, False)}
+    for a in views(A):
+        for b in views(B):
+            assert_same_bits(host(K.pam_bmm_fwd(a, b, True, True, 1.0)), want, f"{a.stride()} x {b.stride()}")
+            for left in (True, False):
+                assert_same_bits(host(K.pam_bmm_bwd(a, b, dev(D), True, True, left, 1.0)), slopes[left], f"gradient {left}, {a.stride()} x {b.stride()}")
