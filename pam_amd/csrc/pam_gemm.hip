@@ -125,7 +125,9 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 // exact gradients', with three operations per product, those of up to seven in the third round and up to nine beyond, 2 to 10 %.
 // On 4151 products of drawn shapes, geometric mean of the time over that without steps: always 0.989, this rule 0.980, the
 // better of the two each time 0.979.
-bool priority_steps(const Plan& p, long M, long N, bool exact)
+// (Freely shaped tiles take the steps in a mostly full second round at any depth: 192 products of 197 x 197, k = 64 in 1920
+// work-groups 34.3 -> 33.1 us, 217 of 197 x 159 29.0 -> 27.1.)
+bool priority_steps(const Plan& p, long M, long N, bool exact, bool free_tiles = false)
 {
     const long cus = cu_count(), resident = (long)kResidentPerCu * cus;
     if (p.units <= resident) return p.units > resident / 2;
@@ -135,6 +137,7 @@ bool priority_steps(const Plan& p, long M, long N, bool exact)
     const long counted = p.pieces > pamgemm::kFoldInKernel && extra <= tiles && 3 * tail <= p.piece_kt ? p.units - extra : p.units;
     const long rounds = (counted + resident - 1) / resident, last = (counted - 1) % resident + 1;
     const bool most = last > resident / 2;
+    if (free_tiles && most && rounds <= 2) return true;
     if (p.piece_kt < (!exact || (most && rounds <= 2) ? 6 : most && rounds <= 3 ? 8 : 10)) return false;
     return most || (last > cus && rounds <= 3 && (p.piece_kt >= 20 || (p.pieces == 1 && M % 64 == 0 && N % 64 == 0)));
 }
@@ -301,28 +304,60 @@ int load_kind(long s_row, long s_k, long s_batch, const float* p, long rows, lon
 // addresses: products 3149 x 103 x 951 24.9 / 31.7 / 27.7 us, now 20.6 / 26.5 / 25.4; 192 of 197 x 64, k = 197 31.7, now 29.0;
 // 13642 x 364 x 233: 66.3 / 71.5, now 61.4 / 66.8.  Aligned operands keep instances of their own: with the tests for a line's end
 // in them, products of a few k-tiles ran 1 to 4 % slower.
+int odd_kind(int kind) { return kind == LOAD_KVEC ? LOAD_KODD : kind == LOAD_RVEC ? LOAD_RODD : kind; }
 void odd_lines(long l_row, long l_k, long M, long r_row, long r_k, long N, long K, int& lk, int& rk)
 {
     if (lk != LOAD_ANY && rk != LOAD_ANY) return;
     auto contiguous = [&](long s_row, long s_k, long rows) { return s_k == 1 && K >= 4 ? LOAD_KODD : s_row == 1 && rows >= 4 ? LOAD_RODD : LOAD_ANY; };
-    const int l = lk == LOAD_KVEC ? LOAD_KODD : lk == LOAD_RVEC ? LOAD_RODD : contiguous(l_row, l_k, M);
-    const int r = rk == LOAD_KVEC ? LOAD_KODD : rk == LOAD_RVEC ? LOAD_RODD : contiguous(r_row, r_k, N);
+    const int l = lk != LOAD_ANY ? odd_kind(lk) : contiguous(l_row, l_k, M), r = rk != LOAD_ANY ? odd_kind(rk) : contiguous(r_row, r_k, N);
     if (l != LOAD_ANY && r != LOAD_ANY) { lk = l; rk = r; }
+}
+
+// Freely shaped tiles.  Matrices of a few tiles each whose sizes are no multiples of 64 (attention scores of 197 x 197: 16 tiles,
+// 7 of them with one busy wavefront) spend work-groups on their edges, and how long a batch of them takes goes by the number
+// of work-groups more than by their products.  A tile may instead have any r x c blocks of 4 x 4 outputs, one per lane, with r c up
+// to 256: 25 x 10 blocks cover 197 x 197 in ten tiles, nearly without idle lanes.  c is at most 16, so that a wavefront's
+// reads of the right fragment stay within 64 LDS banks (25 columns in 10 rows 34.3 us where 10 in 25 take 31.5), r at most 32.
+// What a tiling costs is counted in wavefronts plus two per work-group; a freely shaped one must save a twentieth of it, as
+// its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), and there must be more work-groups
+// than two per compute unit: with fewer, all run at once and their number does not matter.  Whole tiles of 16-deep k-tiles only.
+// Products of 192 x 197 x 197, k = 64: 37.4 -> 31.2 us; 212 x 148 x 148, 64: 25 -> 21.4; 120 x 257 x 131, 80: 29.6 -> 25.9;
+// 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7; of 120 drawn attention products none was more than 1 % slower.
+struct FreeShape { int r, c; };
+FreeShape free_shape(long batch, long M, long N, long K)
+{
+    FreeShape best{0, 0};
+    const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
+    // wavefronts with outputs in the fixed tiles (see lane_place)
+    const long full_m = M / 64, full_n = N / 64, rest_m = M % 64, rest_n = N % 64;
+    const long waves = 4 * full_m * full_n + full_m * ((rest_n + 15) / 16) + full_n * ((rest_m + 15) / 16) + (std::min(rest_m, rest_n) + 15) / 16;
+    const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
+    long least = (waves + 2 * tiles) * 19 / 20;
+    for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {
+        const long tn = (fours_n + widest - 1) / widest, c = (fours_n + tn - 1) / tn, most = std::min<long>(kFreeFoursM, 256 / c), tm = (fours_m + most - 1) / most, r = (fours_m + tm - 1) / tm;
+        const long cost = tm * tn * ((r * c + 63) / 64 + 2);
+        if (cost < least) { least = cost; best = FreeShape{(int)r, (int)c}; }
+    }
+    return best;
+}
+
+// One contiguous range of units per XCD (see the kernel), rounded up to whole work-groups per XCD; returns the work-groups.
+unsigned spread_over_xcds(GemmArgs& g)
+{
+    g.xcd_chunk = (g.units + XCDS - 1) / XCDS;
+    return (unsigned)(g.xcd_chunk * XCDS);
 }
 
 template <int MODE>
 void launch_mode(const Plan& p, int lk, int rk, hipStream_t st, const GemmArgs& g)
 {
-    // One contiguous range of units per XCD (see the kernel), rounded up to whole work-groups per XCD.  Piece-major
-    // launches keep the launch order: all XCDs then work on the same few k ranges at a time (each L2 fetches them,
+    // Piece-major launches keep the launch order: all XCDs then work on the same few k ranges at a time (each L2 fetches them,
     // from the memory-side cache), where ranges would have every L2 hold three or four k ranges of both operands at
     // once -- measured 3 % (dense) to 9 % (left operand with zeros) slower.
     GemmArgs ga = g;
     unsigned groups = (unsigned)p.units;
-    if (p.units >= 64 && (p.pieces == 1 || g.fold_here)) {
-        ga.xcd_chunk = (int)((p.units + XCDS - 1) / XCDS);
-        groups = (unsigned)(ga.xcd_chunk * XCDS);
-    }
+    if (p.units >= 64 && (p.pieces == 1 || g.fold_here)) groups = spread_over_xcds(ga);
     if (p.bk == 32) pamgemm::launch_gemm<32, MODE>(lk, rk, groups, st, ga);
     else pamgemm::launch_gemm<16, MODE>(lk, rk, groups, st, ga);
 }
@@ -373,6 +408,7 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
         g.off_add = bits - kBias;
     }
 
+    g.free_r = g.free_c = 0;
     g.cv = conv ? *conv : ConvGeom{nullptr, nullptr, 0, 0, 0, 0, 0};
 
     if (mode == MODE_PAM && !conv && M <= kFewRows && K <= kFewLongest && p.pieces == 1 && g.has_off == 0 && g_force_bk == 0 && g_force_pieces == 0) {
@@ -390,6 +426,19 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
         rk = LOAD_CONVR;
     else if (conv && conv->row_quads && conv->transposed && mode != MODE_STD && lk == LOAD_KVEC && K % 4 == 0)
         rk = LOAD_CONVK;
+    if (mode == MODE_PAM && !conv && p.pieces == 1 && lk != LOAD_ANY && rk != LOAD_ANY && g_force_bk == 0 && g_force_pieces == 0) {
+        const FreeShape f = free_shape(batch, M, N, K);
+        if (f.r > 0) {
+            g.free_r = f.r; g.free_c = f.c;
+            g.ntn = (int)((N + 4 * f.c - 1) / (4 * f.c)); g.tiles = (int)((M + 4 * f.r - 1) / (4 * f.r)) * g.ntn;
+            p.units = batch * g.tiles; g.units = (int)p.units;
+            p.bk = 16; p.kt = p.piece_kt = g.piece_kt = (int)((K + 15) / 16);
+            g.steps = priority_steps(p, M, N, false, true) ? 1 : 0;
+            const unsigned groups = spread_over_xcds(g);
+            launch_free(odd_kind(lk), odd_kind(rk), groups, st, g);
+            return pamhost::check_launch(what);
+        }
+    }
     switch (mode) {
     case MODE_PAM: launch_mode<MODE_PAM>(p, lk, rk, st, g); break;
     case MODE_STD: launch_mode<MODE_STD>(p, lk, rk, st, g); break;

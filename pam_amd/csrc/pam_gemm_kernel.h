@@ -100,6 +100,7 @@ struct GemmArgs {
     float* Y; long y_sb, y_sr, y_sc;
     const float* bias;           // one value per output column, added once after the sum, or null
     int M, N, K;
+    int free_r, free_c;          // freely shaped tiles: a tile is free_r x free_c blocks of 4 x 4 outputs
     int tiles, ntn;              // output tiles per matrix; tiles per row of tiles (consecutive tiles share rows of L)
     int pieces, piece_kt;        // k ranges a tile is cut into (1: whole tiles) and their length in k-tiles
     int units;                   // tiles of all matrices x pieces: one work-group each
@@ -220,7 +221,7 @@ __device__ __forceinline__ float4 last_values(const float4 q, int early)
 }
 
 // One operand's tile: ROWS x BK values from global memory into registers, then into LDS.
-template <int ROWS, int NT, int KIND, int BK>
+template <int ROWS, int NT, int KIND, int BK, bool FREE = false>
 struct TileLoader {
     static constexpr int kVecs = ROWS * BK / 4 / NT;      // float4 per lane (vector kinds)
     static constexpr int kElems = ROWS * BK / NT;         // scalars per lane (generic kind)
@@ -229,6 +230,31 @@ struct TileLoader {
     static constexpr bool kRQuads = KIND == LOAD_RVEC || KIND == LOAD_RODD || KIND == LOAD_CONVR;      // ... along the rows
     float4 v[kVecs > 0 ? kVecs : 1];
     int2 fixed; bool have_fixed = false;          // LOAD_CONV: the lane's own table entry
+    // FREE: the tile has `fours` * 4 rows (at most ROWS), and the quads beyond them repeat the last one and are not stored
+    int fours, at_k[FREE && kRQuads ? kVecs : 1], at_row[FREE && kRQuads ? kVecs : 1];
+    __device__ __forceinline__ void shape(int tid, int fours_of_rows)
+    {
+        fours = fours_of_rows;
+        if (FREE && kRQuads) {
+#pragma unroll
+            for (int i = 0; i < kVecs; ++i) {
+                const int id = min(tid + i * NT, fours * BK - 1);
+                at_k[i] = id / fours; at_row[i] = (id - at_k[i] * fours) * 4;
+            }
+        }
+    }
+    __device__ __forceinline__ bool stored(int tid, int i) const { return !FREE || tid + i * NT < fours * BK; }
+    // the k and the row that vector i of a lane begins at
+    __device__ __forceinline__ int quad_k(int tid, int i) const
+    {
+        const int id = FREE ? min(tid + i * NT, fours * BK - 1) : tid + i * NT;
+        return kKQuads ? id % (BK / 4) * 4 : FREE ? at_k[i] : id / (ROWS / 4);
+    }
+    __device__ __forceinline__ int quad_row(int tid, int i) const
+    {
+        const int id = FREE ? min(tid + i * NT, fours * BK - 1) : tid + i * NT;
+        return kKQuads ? id / (BK / 4) : FREE ? at_row[i] : id % (ROWS / 4) * 4;
+    }
     int patch_at[kVecs > 0 ? kVecs : 1];          // LOAD_CONVQ: where the patches of the lane's rows begin in the image
     int2 row_entry[KIND == LOAD_CONVK && kVecs > 0 ? kVecs : 1];      // LOAD_CONVK: the k table's entries of the lane's rows
 
@@ -245,11 +271,11 @@ struct TileLoader {
         // the end: its first values are the last ones read.
         if (KIND == LOAD_KODD && (kend & 3) != 0 && k0 + BK > kend) {
 #pragma unroll
-            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], k0 + ((tid + i * NT) % (BK / 4)) * 4 - (kend - 4));
+            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], k0 + quad_k(tid, i) - (kend - 4));
         }
-        if (KIND == LOAD_RODD && (nrows & 3) != 0 && row0 + ROWS > nrows) {
+        if (KIND == LOAD_RODD && (nrows & 3) != 0 && row0 + (FREE ? fours * 4 : ROWS) > nrows) {
 #pragma unroll
-            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], row0 + ((tid + i * NT) % (ROWS / 4)) * 4 - (nrows - 4));
+            for (int i = 0; i < kVecs; ++i) v[i] = last_values(v[i], row0 + quad_row(tid, i) - (nrows - 4));
         }
     }
 
@@ -325,20 +351,16 @@ struct TileLoader {
         } else if (KIND == LOAD_KVEC || KIND == LOAD_KODD) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
-                int id = tid + i * NT;
-                int r = id / (BK / 4), kq = id % (BK / 4);
-                int row = min(row0 + r, nrows - 1);
-                int k = min(k0 + kq * 4, kend - 4);
+                int row = min(row0 + quad_row(tid, i), nrows - 1);
+                int k = min(k0 + quad_k(tid, i), kend - 4);
                 const float* at = base + (long)row * op.sr + k;
                 v[i] = KIND == LOAD_KODD ? any_quad(at) : *reinterpret_cast<const float4*>(at);
             }
         } else if (KIND == LOAD_RVEC || KIND == LOAD_RODD) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
-                int id = tid + i * NT;
-                int k = id / (ROWS / 4), rq = id % (ROWS / 4);
-                int row = min(row0 + rq * 4, nrows - 4);
-                int kk = min(k0 + k, kend - 1);
+                int row = min(row0 + quad_row(tid, i), nrows - 4);
+                int kk = min(k0 + quad_k(tid, i), kend - 1);
                 const float* at = base + (long)kk * op.sk + row;
                 v[i] = KIND == LOAD_RODD ? any_quad(at) : *reinterpret_cast<const float4*>(at);
             }
@@ -392,13 +414,13 @@ struct TileLoader {
         if (kKQuads) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
-                const int k = ((tid + i * NT) % (BK / 4)) * 4;
+                const int k = quad_k(tid, i);
                 see(v[i].x, k); see(v[i].y, k + 1); see(v[i].z, k + 2); see(v[i].w, k + 3);
             }
         } else if (kRQuads) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
-                const int k = (tid + i * NT) / (ROWS / 4);
+                const int k = quad_k(tid, i);
                 see(v[i].x, k); see(v[i].y, k); see(v[i].z, k); see(v[i].w, k);
             }
         } else {
@@ -415,8 +437,8 @@ struct TileLoader {
         if (kKQuads) {
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
-                int id = tid + i * NT;
-                uint32_t* d = lds + ((id % (BK / 4)) * 4) * LD + swizzled<BK>(id / (BK / 4), (id % (BK / 4)) * 4);
+                uint32_t* d = lds + quad_k(tid, i) * LD + swizzled<BK>(quad_row(tid, i), quad_k(tid, i));
+                if (!stored(tid, i)) continue;
                 d[0 * LD] = st.one(v[i].x); d[1 * LD] = st.one(v[i].y);
                 d[2 * LD] = st.one(v[i].z); d[3 * LD] = st.one(v[i].w);
             }
@@ -424,12 +446,13 @@ struct TileLoader {
             // (vector i of a lane sits under k = i * kPer + tid / (ROWS / 4), the second term below kPer: which half of a
             // 32-deep tile that is depends on i alone, so the exchange of the row groups costs nothing per vector)
             constexpr int kPer = NT / (ROWS / 4);
-            static_assert(16 % kPer == 0, "a lane's vectors must not straddle the tile's k halves");
+            static_assert(FREE ? BK == 16 : 16 % kPer == 0, "a lane's vectors must not straddle the tile's k halves");
 #pragma unroll
             for (int i = 0; i < kVecs; ++i) {
                 uint4 w;
                 w.x = st.one(v[i].x); w.y = st.one(v[i].y); w.z = st.one(v[i].z); w.w = st.one(v[i].w);
-                *reinterpret_cast<uint4*>(lds + (i * kPer + tid / (ROWS / 4)) * LD + swizzled<BK>((tid % (ROWS / 4)) * 4, i * kPer)) = w;
+                if (FREE) { if (stored(tid, i)) *reinterpret_cast<uint4*>(lds + at_k[i] * LD + at_row[i]) = w; }
+                else *reinterpret_cast<uint4*>(lds + (i * kPer + tid / (ROWS / 4)) * LD + swizzled<BK>((tid % (ROWS / 4)) * 4, i * kPer)) = w;
             }
         } else {                                    // LOAD_ANY and LOAD_CONV: lane-consecutive rows
             const float* s = reinterpret_cast<const float*>(v);
@@ -749,12 +772,19 @@ constexpr int kFoldInKernel = 8;                // tiles of up to this many piec
 // covers 16 rows x 64 columns -- or, in a tile that the matrix fills less in its columns than in its rows, 64 rows x
 // 16 columns: a wavefront none of whose outputs exist (the last tiles of 197 rows or columns leave three of the four
 // without one) stages and synchronises with the others but computes nothing.
-struct LanePlace { int tx, ty; bool idle; };
+struct LanePlace { int tx, ty; bool idle, none; };
 __device__ __forceinline__ LanePlace lane_place(int tid, int row0, int col0, int M, int N)
 {
     const int wave = tid / 64, lane = tid % 64;
-    if (N - col0 < 64 && N - col0 < M - row0) return LanePlace{4 * wave + lane % 4, lane / 4, col0 + 16 * wave >= N};
-    return LanePlace{tid % 16, tid / 16, row0 + 16 * wave >= M};
+    if (N - col0 < 64 && N - col0 < M - row0) return LanePlace{4 * wave + lane % 4, lane / 4, col0 + 16 * wave >= N, false};
+    return LanePlace{tid % 16, tid / 16, row0 + 16 * wave >= M, false};
+}
+// ... and in a freely shaped tile of r x c blocks: lanes across a row of blocks first.  Lanes left over have no outputs
+// (`none`) and go along with the last row.
+__device__ __forceinline__ LanePlace free_place(int tid, int row0, int M, int r, int c)
+{
+    const int ty = tid / c, first = __builtin_amdgcn_readfirstlane(ty);       // (of the wavefront's first lane)
+    return LanePlace{tid - ty * c, min(ty, r - 1), first >= r || row0 + 4 * first >= M, ty >= r};
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -821,15 +851,16 @@ __device__ __forceinline__ LateArgs late_args()
     return p;
 }
 
+// FREE: tiles of free_r x free_c blocks of 4 x 4 outputs (at most BM x BN outputs) instead of 64 x 64.
 // CUT: the launch cuts its tiles' k ranges into pieces (an instance of its own, so that the kernel for whole tiles
 // carries none of the pieces' way out).
-template <int BM, int BN, int TM, int TN, int BK, int MODE, int LKIND, int RKIND, bool CUT>
-__global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm_kernel(GemmArgs g)
+template <int BM, int BN, int TM, int TN, int BK, int MODE, int LKIND, int RKIND, bool CUT, bool FREE = false>
+__global__ __launch_bounds__(256) PAM_GEMM_OCCUPANCY void gemm_kernel(GemmArgs g)
 {
-    constexpr int TXN = BN / TN, TYN = BM / TM, NT = TXN * TYN, NW = NT / 64;
+    constexpr int NT = 256, NW = NT / 64;
     constexpr int GM = TM / 4, GN = TN / 4;               // 4-wide groups per micro-tile side
     constexpr int LDL = BM + PAD, LDR = BN + PAD;
-    static_assert(TM == 4 && TN == 4 && BM == 64 && BN == 64 && NT == 256, "a tile's piece is sixteen sums per lane of 256");
+    static_assert(TM == 4 && TN == 4 && (FREE ? !CUT && BK == 16 && MODE == MODE_PAM : BM == 64 && BN == 64), "a tile's piece is sixteen sums per lane of 256");
 
     __shared__ __attribute__((aligned(16))) uint32_t lds_l[2][BK * LDL];
     __shared__ __attribute__((aligned(16))) uint32_t lds_r[2][BK * LDR];
@@ -856,12 +887,12 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
         else { const int all = g.units / g.pieces; piece = unit / all; flat = unit - piece * all; }
     }
     const int zb = flat / g.tiles, tile = flat - zb * g.tiles;
-    const int row0 = (tile / g.ntn) * BM, col0 = (tile % g.ntn) * BN;       // consecutive tiles share L rows
+    const int row0 = (tile / g.ntn) * (FREE ? g.free_r * 4 : BM), col0 = (tile % g.ntn) * (FREE ? g.free_c * 4 : BN);       // consecutive tiles share L rows
     const int kbegin = CUT ? piece * g.piece_kt * BK : 0;
     const int kend = CUT ? min(g.K, kbegin + g.piece_kt * BK) : g.K;
     const int ktiles = (kend - kbegin + BK - 1) / BK;
     // The lane's 4 x 4 outputs within the tile, rows ty * 4 ..., columns tx * 4 ....
-    const LanePlace place = lane_place(tid, row0, col0, g.M, g.N);
+    const LanePlace place = FREE ? free_place(tid, row0, g.M, g.free_r, g.free_c) : lane_place(tid, row0, col0, g.M, g.N);
     const int tx = place.tx, ty = place.ty;
     const bool has_off = g.has_off != 0;
 
@@ -888,8 +919,9 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
             }
     }
 
-    TileLoader<BM, NT, LKIND, BK> ll;
-    TileLoader<BN, NT, RKIND, BK> rl;
+    TileLoader<BM, NT, LKIND, BK, FREE> ll;
+    TileLoader<BN, NT, RKIND, BK, FREE> rl;
+    if (FREE) { ll.shape(tid, g.free_r); rl.shape(tid, g.free_c); }
 
     auto stage = [&](int buf, int k0) __attribute__((always_inline)) {
         ll.arrive(row0, g.M, k0, kend, tid); rl.arrive(col0, g.N, k0, kend, tid);
@@ -1370,7 +1402,7 @@ __global__ __launch_bounds__((BM / TM) * (BN / TN)) PAM_GEMM_OCCUPANCY void gemm
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         int r = row0 + (i / 4) * (BM / GM) + ty * 4 + (i % 4);
-        if (r >= g.M) continue;
+        if (r >= g.M || (FREE && place.none)) continue;
 #pragma unroll
         for (int gj = 0; gj < GN; ++gj) {
             int c = col0 + gj * (BN / GN) + tx * 4;
@@ -1412,6 +1444,10 @@ void launch_gemm(int lk, int rk, unsigned groups, hipStream_t st, const GemmArgs
     }
 #undef PAM_GEMM_CASE
 }
+
+// Freely shaped tiles (free_shape in pam_gemm.hip).
+constexpr int kFreeFoursM = 32, kFreeFoursN = 16;      // as many lines of either operand as two vectors and one per lane hold
+void launch_free(int lk, int rk, unsigned groups, hipStream_t st, const GemmArgs& g);
 
 // Each (k-tile depth, mode) pair is instantiated in a source file of its own (pam_gemm_inst_*.hip).
 #define PAM_GEMM_EXTERN(BK, MODE) extern template void launch_gemm<BK, MODE>(int, int, unsigned, hipStream_t, const GemmArgs&);

@@ -826,3 +826,42 @@ def test_lines_of_any_length_and_address(K, oracle, batch, m, k, n, specials):
             assert_same_bits(host(K.pam_bmm_fwd(a, b, True, True, 1.0)), want, f"{a.stride()} x {b.stride()}")
             for left in (True, False):
                 assert_same_bits(host(K.pam_bmm_bwd(a, b, dev(D), True, True, left, 1.0)), slopes[left], f"gradient {left}, {a.stride()} x {b.stride()}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("values", ["plain", "zeros and specials", "causal"])
+@pytest.mark.parametrize("batch,m,n,k", [(140, 70, 70, 20), (60, 197, 133, 33), (200, 41, 129, 64), (66, 257, 66, 16), (130, 72, 129, 5)])
+def test_freely_shaped_tiles(K, oracle, batch, m, n, k, values):
+    """Batches of small matrices whose sizes are no multiples of 64, in every layout that 128-bit loads read: the oracle's
+    bits in ascending k, and those of the 64 x 64 tiles, with and without an offset."""
+    from pam_amd import _abi
+    lib = _abi.load_library()
+    rng = np.random.RandomState(batch + m)
+    A, B = rng.standard_normal((batch, m, k)).astype(np.float32), rng.standard_normal((batch, k, n)).astype(np.float32)
+    if values == "causal":
+        A *= np.tri(m, k, dtype=np.float32)
+    elif values != "plain":
+        for x in (A, B):
+            flat = x.reshape(-1)
+            at = rng.choice(flat.size, flat.size // 50, replace=False)
+            flat[at] = np.resize(np.array([0.0] * 40 + [-0.0, 1e-40, 3e38, np.inf, np.nan, 1e-30], np.float32), at.size)
+    def views(x):
+        b, r, c = x.shape
+        t = torch.from_numpy(x).cuda()
+        apart = torch.zeros(b * (r + 1) * (c + 3) + 1, device="cuda")[1:].view(b, r + 1, c + 3)[:, 1:, 2:c + 2]
+        apart.copy_(t)
+        return [t, t.transpose(1, 2).contiguous().transpose(1, 2), apart]
+    pick = [0, 1, batch // 2, batch - 1]
+    for off in OFFS:
+        want = None
+        for a in views(A):
+            for b in views(B):
+                got = K.pam_bmm_fwd(a, b, True, True, _o(off))
+                if want is None:
+                    assert_same_bits(host(got)[pick], oracle.gemm(A[pick], B[pick], offset=off, kchunk=0), f"oracle, off={off}")
+                    lib.pam_hip_set_tuning(16, 1)
+                    try:
+                        want = host(K.pam_bmm_fwd(a, b, True, True, _o(off)))
+                    finally:
+                        lib.pam_hip_set_tuning(0, 0)
+                assert_same_bits(host(got), want, f"{a.stride()} x {b.stride()} off={off}")
