@@ -44,6 +44,46 @@ constexpr long kMostCutTiles = 8192;            // tiles of a product that cuts 
 constexpr int kResidentPerCu = 4;               // work-groups of the kernel a compute unit holds (LDS and registers)
 constexpr size_t kPartBytes = (size_t)pamgemm::kPartFloats * sizeof(float);
 
+// Wavefronts with outputs in the 64 x 64 tiles of an M x N matrix (see lane_place).
+long busy_waves(long M, long N)
+{
+    const long full_m = M / 64, full_n = N / 64, rest_m = M % 64, rest_n = N % 64;
+    return 4 * full_m * full_n + full_m * ((rest_n + 15) / 16) + full_n * ((rest_m + 15) / 16) + (std::min(rest_m, rest_n) + 15) / 16;
+}
+
+constexpr int kFewRows = 4;                     // products that few_rows_kernel takes where their tiles are whole
+constexpr long kFewLongest = 512;
+
+// Products that fit the chip at once: up to 1024 tiles whose k-steps come to less than 500 per compute unit.  There a
+// work-group's chain of k-tiles is what takes the time, one wavefront per SIMD issues at half rate, and cutting k much finer
+// than the rule for large products does pays: pieces down to 32 k, as long as all units are resident.  The time of a unit,
+// in k-steps of a work-group alone on its compute unit, is its k (0.88 of it in 32-deep k-tiles), two thirds of the k over a
+// whole k-tile and 170 for start, first fetch and way out, times up to 1.66 for four busy work-groups on a compute unit; pieces
+// cost 15 and 1.5 each where the tile's last arriver adds them up, 20 and 0.9 each in the second kernel.  Fitted on a third of
+// 2934 drawn products timed in both k-tile depths with 1 ... 64 pieces, checked on the others: 1.02 of the best time each, where the rule below
+// took 1.27 (1.49 for up to 16 tiles, 1.33 up to 64, 1.23, 1.14 and 1.07 up to 128, 256 and 512); beyond 500 k-steps per compute
+// unit the two are even.  The three products of 60 drawn linear layers: 1.21 times as fast, 0.88 to 2.2.  197 x 768, k = 192 18.3 -> 12.9 us;
+// 450 x 333, 190 21.0 -> 14.6; 800 x 360, 190 22.1 -> 14.8; 5000 x 150, 200 22.0 -> 16.8.
+bool small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
+{
+    const long cus = cu_count(), resident = (long)kResidentPerCu * cus;
+    if (tiles > resident || tiles * K >= 500 * cus || (M <= kFewRows && K <= kFewLongest)) return false;
+    const double busy = 0.66 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles);
+    double best = 0.0;
+    for (int bk = 16; bk <= (K >= 128 ? 32 : 16); bk *= 2) {
+        const long kt = (K + bk - 1) / bk;
+        for (long w = 1; w == 1 || (w <= kt * bk / 32 && w * tiles <= resident); w += w < 8 ? 1 : w < 16 ? 2 : w < 32 ? 4 : 8) {
+            const long per = (kt + w - 1) / w, pieces = (kt + per - 1) / per, n = tiles * pieces;
+            const double crowd = n <= cus ? 1.0 : 1.0 + busy * (double)(n - cus) / (double)(resident - cus);
+            const double unit = (double)std::min(per * bk, K) * (bk == 32 ? 0.88 : 1.0) + 0.65 * (double)(K % bk) + 170.0;
+            const double time = unit * crowd + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 15.0 + 1.5 * (double)pieces : 20.0 + 0.9 * (double)pieces);
+            if (best == 0.0 || time < best) { best = time; p.bk = bk; p.kt = (int)kt; p.pieces = (int)pieces; p.piece_kt = (int)per; }
+        }
+    }
+    p.units = tiles * p.pieces;
+    return true;
+}
+
 // Work-groups own 64 x 64 output tiles.  k of 128 and more in whole multiples of 32, and any k
 // from 512, uses 32-deep k-tiles (fewer barriers and more bytes in flight per round, measured 3-5 %
 // faster on 12608-row products); short or ragged k (attention: 64, 197) 16-deep ones.
@@ -56,6 +96,7 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
     const long resident = (long)kResidentPerCu * cu_count();
     const long tiles = batch * ((M + 63) / 64) * ((N + 63) / 64);
     Plan p;
+    if (with_workspace && g_force_bk == 0 && g_force_pieces == 0 && small_plan(p, tiles, batch, M, N, K)) return p;
     p.bk = (K >= 512 || (K >= 128 && K % 32 == 0)) ? 32 : 16;
     if (g_force_bk) p.bk = g_force_bk;
     p.kt = (int)((K + p.bk - 1) / p.bk);
@@ -220,8 +261,7 @@ __global__ __launch_bounds__(128) void fold_kernel(pamgemm::GemmArgs g)
 // in the matrix kernel.  With up to four rows this kernel was the faster one in every class of values at eleven shapes, 1.6 to
 // 4 times.  A plan that cuts k (k of 256 and more on fewer than 1536 tiles) goes to the matrix kernel, whose pieces the
 // sums follow; beyond kFewLongest nothing was measured.
-constexpr int kFewRows = 4, kFewDepth = 64;
-constexpr long kFewLongest = 512;
+constexpr int kFewDepth = 64;
 template <bool ALONG_K>                   // which index of the right operand is contiguous (or nearer to it)
 __global__ __launch_bounds__(256) void few_rows_kernel(pamgemm::GemmArgs g)
 {
@@ -329,9 +369,7 @@ FreeShape free_shape(long batch, long M, long N, long K)
     FreeShape best{0, 0};
     const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
     if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
-    // wavefronts with outputs in the fixed tiles (see lane_place)
-    const long full_m = M / 64, full_n = N / 64, rest_m = M % 64, rest_n = N % 64;
-    const long waves = 4 * full_m * full_n + full_m * ((rest_n + 15) / 16) + full_n * ((rest_m + 15) / 16) + (std::min(rest_m, rest_n) + 15) / 16;
+    const long waves = busy_waves(M, N);
     const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
     long least = (waves + 2 * tiles) * 19 / 20;
     for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {

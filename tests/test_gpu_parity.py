@@ -865,3 +865,28 @@ def test_freely_shaped_tiles(K, oracle, batch, m, n, k, values):
                     finally:
                         lib.pam_hip_set_tuning(0, 0)
                 assert_same_bits(host(got), want, f"{a.stride()} x {b.stride()} off={off}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,k,n,cut", [(1, 8, 64, 64, True), (1, 65, 63, 65, True), (2, 96, 80, 128, True), (1, 5, 513, 130, True), (1, 64, 2049, 48, True),
+                                             (3, 197, 192, 66, True), (30, 70, 96, 70, True), (256, 128, 33, 128, False), (257, 120, 100, 120, False)])
+def test_small_products_in_pieces(K, oracle, batch, m, k, n, cut):
+    """Products that fit the chip at once, their k in a few or many short pieces: the oracle's bits in the plan's order, forward with a
+    bias and with an offset, and both exact gradients, twice on one workspace."""
+    from pam_amd import _abi
+    A, B, D = (np.stack([_sparse_specials(shape, seed + b, every=4000) for b in range(batch)]) for shape, seed in (((m, k), 3), ((k, n), 5), ((m, n), 7)))
+    D = np.where(np.isfinite(D), D, 1.0).astype(np.float32)
+    assert (_abi.gemm_plan(batch, m, n, k) < k) == cut
+    pick = sorted({0, batch // 2, batch - 1})
+    shape = (batch, m, n, k)
+    a, b, d = dev(A), dev(B), dev(D)
+    for off in OFFS:
+        want = ogemm(oracle, A[pick], B[pick], plan_shape=shape, offset=off)
+        for _ in range(2):
+            assert_same_bits(host(K.pam_bmm_fwd(a, b, True, True, _o(off)))[pick], want, f"forward off={off}")
+    for left in (True, False):
+        want = ogemm(oracle, A[pick], B[pick], plan_shape=shape, mode=oracle.MODE_BWD_DELTA_L if left else oracle.MODE_BWD_DELTA_R, D=D[pick])
+        assert_same_bits(host(K.pam_bmm_bwd(a, b, d, True, True, left, 1.0))[pick], want, f"gradient {left}")
+    if batch == 1:
+        bias = torch.randn(n, device="cuda")
+        assert torch.equal(_abi.host().product(0, a[0], b[0], None, False, bias, 1.0).nan_to_num(7.0), (K.pam_matmul_fwd(a[0], b[0], True, True, 1.0) + bias).nan_to_num(7.0))
