@@ -359,7 +359,8 @@ void odd_lines(long l_row, long l_k, long M, long r_row, long r_k, long N, long 
 // to 256: 25 x 10 blocks cover 197 x 197 in ten tiles, nearly without idle lanes.  c is at most 16, so that a wavefront's
 // reads of the right fragment stay within 64 LDS banks (25 columns in 10 rows 34.3 us where 10 in 25 take 31.5), r at most 32.
 // What a tiling costs is counted in wavefronts plus two per work-group; a freely shaped one must save a twentieth of it, as
-// its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), and there must be more work-groups
+// its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), or a tenth where the fixed tiles
+// are all resident and no round is saved (15362 x 160, k = 64, saving a seventeenth: 12.4 -> 13.2), and there must be more work-groups
 // than two per compute unit: with fewer, all run at once and their number does not matter.  Whole tiles of 16-deep k-tiles only.
 // Products of 192 x 197 x 197, k = 64: 37.4 -> 31.2 us; 212 x 148 x 148, 64: 25 -> 21.4; 120 x 257 x 131, 80: 29.6 -> 25.9;
 // 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7; of 120 drawn attention products none was more than 1 % slower.
@@ -371,7 +372,7 @@ FreeShape free_shape(long batch, long M, long N, long K)
     if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
     const long waves = busy_waves(M, N);
     const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
-    long least = (waves + 2 * tiles) * 19 / 20;
+    long least = (waves + 2 * tiles) * (batch * tiles > (long)kResidentPerCu * cu_count() ? 19 : 18) / 20;
     for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {
         const long tn = (fours_n + widest - 1) / widest, c = (fours_n + tn - 1) / tn, most = std::min<long>(kFreeFoursM, 256 / c), tm = (fours_m + most - 1) / most, r = (fours_m + tm - 1) / tm;
         const long cost = tm * tn * ((r * c + 63) / 64 + 2);
