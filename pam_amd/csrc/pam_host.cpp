@@ -16,6 +16,7 @@
 #include <sstream>
 #include <string>
 #include <utility>
+#include <vector>
 
 #include "../../include/pam_hip.h"
 #include "../../include/pam_hip_extra.h"
@@ -343,6 +344,127 @@ struct LayerNormNode : torch::autograd::Function<LayerNormNode> {
     }
 };
 
+// logsumexp over the last dimension of a contiguous tensor (the result keeps it, with one value), or log_softmax = x less
+// that.  nonfinite, checked: as pam_hip_logsumexp_fwd_finite takes them, or null: the caller waits and looks.
+struct LogsumexpNode : torch::autograd::Function<LogsumexpNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, bool log_softmax, int64_t nonfinite, int64_t checked, double offset, bool a, bool b, bool e)
+    {
+        check_tensor(x);
+        TORCH_CHECK_VALUE(x.dim() >= 1 && x.is_contiguous() && x.numel() > 0, "logsumexp: expected a contiguous tensor");
+        const OnDevice on(x);
+        const int64_t n = x.size(-1), rows = x.numel() / n;
+        std::vector<int64_t> shape = x.sizes().vec();
+        if (!log_softmax) shape.back() = 1;
+        const Tensor y = new_floats(shape, x), shift = new_floats({1}, x);
+        const size_t bytes = pam_hip_rowop_workspace_bytes();
+        const Tensor ws = new_floats({(int64_t)(bytes / 4)}, x);
+        float* const lse = log_softmax ? nullptr : data(y);
+        float* const out = log_softmax ? data(y) : nullptr;
+        if (nonfinite)
+            check_call(pam_hip_logsumexp_fwd_finite(data(x), lse, out, data(shift), rows, n, (float)offset, reinterpret_cast<int*>(nonfinite),
+                                                    reinterpret_cast<void*>(checked), data(ws), bytes, on.stream), "logsumexp_fwd_finite");
+        else
+            check_call(pam_hip_logsumexp_fwd(data(x), lse, out, data(shift), rows, n, (float)offset, data(ws), bytes, on.stream), "logsumexp_fwd");
+        ctx->saved_data["offset"] = offset; ctx->saved_data["log_softmax"] = log_softmax;
+        Approx{a, b, e}.save(ctx);
+        ctx->save_for_backward({x, shift});
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &shift = saved[1];
+        const Approx f = Approx::saved(ctx);
+        const at::AutoGradMode no_graph(false);
+        const Tensor g = grads[0].contiguous();
+        check_tensor(g);
+        const OnDevice on(x);
+        const Tensor dx = new_floats(x.sizes(), x);
+        check_call(pam_hip_logsumexp_bwd(data(x), data(g), data(shift), data(dx), x.numel() / x.size(-1), x.size(-1), ctx->saved_data["log_softmax"].toBool(),
+                                         (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, f.e, on.stream), "logsumexp_bwd");
+        return {dx, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// ---------------------------------------------------------------- elementwise
+
+// A (*) B or A (/) B of contiguous tensors of one shape that both want a gradient or both do not; both gradients in one pass
+template <bool DIVIDE>
+struct PairNode : torch::autograd::Function<PairNode<DIVIDE>> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& A, const Tensor& B, double offset, bool a, bool b)
+    {
+        check_tensor(A);
+        check_tensor(B);
+        TORCH_CHECK_VALUE(A.sizes() == B.sizes() && A.is_contiguous() && B.is_contiguous(), "expected contiguous operands of one shape");
+        const OnDevice on(A);
+        const Tensor y = new_floats(A.sizes(), A);
+        check_call((DIVIDE ? pam_hip_pad_fwd : pam_hip_pam_fwd)(data(A), data(B), data(y), A.numel(), (float)offset, on.stream), DIVIDE ? "pad_fwd" : "pam_fwd");
+        ctx->saved_data["offset"] = offset;
+        Approx{a, b, false}.save(ctx);
+        ctx->save_for_backward({A, B});
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &A = saved[0], &B = saved[1];
+        const Approx f = Approx::saved(ctx);
+        const at::AutoGradMode no_graph(false);
+        const Tensor g = grads[0].contiguous();
+        check_tensor(g);
+        const OnDevice on(A);
+        const Tensor dA = new_floats(A.sizes(), A), dB = new_floats(A.sizes(), A);
+        check_call((DIVIDE ? pam_hip_pad_bwd_pair : pam_hip_pam_bwd_pair)(data(A), data(B), data(g), data(dA), data(dB), A.numel(),
+                   (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, on.stream), DIVIDE ? "pad_bwd_pair" : "pam_bwd_pair");
+        return {dA, dB, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// base ** x, log_base x, x ** p of a contiguous tensor.  The approximate gradient is that of the base e
+// (pam/cuda_bindings.py:224-239, 262-276): exp(x) (*) g, g (/) x.
+enum { kExp = 0, kLog = 1, kPow = 2 };
+struct UnaryNode : torch::autograd::Function<UnaryNode> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, int64_t op, double number, double offset, bool a, bool e)
+    {
+        check_tensor(x);
+        TORCH_CHECK_VALUE(x.is_contiguous(), "expected a contiguous tensor");
+        const OnDevice on(x);
+        const Tensor y = new_floats(x.sizes(), x);
+        check_call((op == kExp ? pam_hip_pa_exp_fwd : op == kLog ? pam_hip_pa_log_fwd : pam_hip_pow_fwd)(data(x), data(y), x.numel(), (float)number,
+                   (float)offset, on.stream), op == kExp ? "pa_exp_fwd" : op == kLog ? "pa_log_fwd" : "pow_fwd");
+        ctx->saved_data["op"] = op; ctx->saved_data["number"] = number; ctx->saved_data["offset"] = offset;
+        Approx{a, false, e}.save(ctx);
+        ctx->save_for_backward({x});
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor& x = saved[0];
+        const Approx f = Approx::saved(ctx);
+        const int64_t op = ctx->saved_data["op"].toInt();
+        const float number = (float)ctx->saved_data["number"].toDouble(), offset = (float)ctx->saved_data["offset"].toDouble();
+        const at::AutoGradMode no_graph(false);
+        const Tensor g = grads[0].contiguous();
+        check_tensor(g);
+        const OnDevice on(x);
+        const Tensor dx = new_floats(x.sizes(), x);
+        const size_t n = x.numel();
+        if (op == kPow) {
+            check_call(pam_hip_pow_bwd(data(x), data(g), data(dx), n, number, offset, f.a, f.e, on.stream), "pow_bwd");
+        } else if (!f.e) {
+            check_call((op == kExp ? pam_hip_pa_exp_bwd : pam_hip_pa_log_bwd)(data(x), data(g), data(dx), n, number, offset, on.stream), op == kExp ? "pa_exp_bwd" : "pa_log_bwd");
+        } else if (op == kExp) {
+            const Tensor y = new_floats(x.sizes(), x);
+            check_call(pam_hip_pa_exp_fwd(data(x), data(y), n, number, offset, on.stream), "pa_exp_fwd");
+            check_call(pam_hip_pam_fwd(data(y), data(g), data(dx), n, offset, on.stream), "pam_fwd");
+        } else {
+            check_call(pam_hip_pad_fwd(data(g), data(x), data(dx), n, offset, on.stream), "pad_fwd");
+        }
+        return {dx, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
 // ---------------------------------------------------------------- optimizer
 
 // The parameters from `start` on that one launch can update: those with a gradient and moments that are contiguous fp32
@@ -421,5 +543,11 @@ PYBIND11_MODULE(_pam_host, module)
                                 double offset, bool a, bool b, bool e) {
         return LayerNormNode::apply(x, n, weight, bias, eps, offset, a, b, e);
     }, unlocked);
+    module.def("logsumexp", [](const Tensor& x, bool log_softmax, int64_t nonfinite, int64_t checked, double offset, bool a, bool b, bool e) {
+        return LogsumexpNode::apply(x, log_softmax, nonfinite, checked, offset, a, b, e);
+    }, unlocked);
+    module.def("mul", [](const Tensor& A, const Tensor& B, double offset, bool a, bool b) { return PairNode<false>::apply(A, B, offset, a, b); }, unlocked);
+    module.def("div", [](const Tensor& A, const Tensor& B, double offset, bool a, bool b) { return PairNode<true>::apply(A, B, offset, a, b); }, unlocked);
+    module.def("unary", [](const Tensor& x, int64_t op, double number, double offset, bool a, bool e) { return UnaryNode::apply(x, op, number, offset, a, e); }, unlocked);
     module.def("adam_collect", &adam_collect);
 }

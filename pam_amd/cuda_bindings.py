@@ -66,6 +66,9 @@ class pam_autograd(torch.autograd.Function):
 
 
 def pam(A, B, *, offset=None, approx_bwd=False):
+    node = _pair_node(A, B, offset, approx_bwd)
+    if node is not None:
+        return host().mul(A, B, *node[:3])
     A, B = utils.broadcast_tensors(A, B)
     return pam_autograd.apply(A, B, offset, approx_bwd)
 
@@ -107,6 +110,9 @@ class pad_autograd(torch.autograd.Function):
 
 
 def pad(A, B, *, offset=None, approx_bwd=False):
+    node = _pair_node(A, B, offset, approx_bwd)
+    if node is not None:
+        return host().div(A, B, *node[:3])
     A, B = utils.broadcast_tensors(A, B)
     return pad_autograd.apply(A, B, offset, approx_bwd)
 
@@ -189,6 +195,34 @@ def node_arguments(kernels, cls, offset, approx_bwd):
     return None
 
 
+# The classes whose results are ordinary tensors: an op on a tensor of another class has a result of that class, which the
+# autograd functions in Python make.
+_ORDINARY = (torch.Tensor, torch.nn.Parameter)
+
+
+def whole_floats(t):
+    """Whether an elementwise node in C++ takes the tensor as it is: an ordinary contiguous fp32 tensor on the GPU, not empty."""
+    return (type(t) in _ORDINARY and t.layout is torch.strided and t.is_cuda and t.dtype is torch.float32 and t.is_contiguous()
+            and t.numel() != 0)
+
+
+def _pair_node(A, B, offset, approx_bwd):
+    """node_arguments for a product or quotient of two whole tensors of one shape that both want a gradient or both do not:
+    such a pair's gradients are one pass.  (Anything else -- numbers, broadcast or strided operands, one gradient -- is the
+    autograd functions' in Python.)"""
+    if not (paired_gradients and whole_floats(A) and whole_floats(B)) or A.shape != B.shape or A.requires_grad != B.requires_grad or A.device != B.device:
+        return None
+    return node_arguments(cuda_kernels, HipKernels, offset, approx_bwd)
+
+
+def _unary_node(X, base, offset, approx_bwd):
+    """... for exp and log: the approximate gradient of another base than e takes further products."""
+    if not whole_floats(X) or type(base) not in (float, int):
+        return None
+    node = node_arguments(cuda_kernels, HipKernels, offset, approx_bwd)
+    return None if node is not None and node[3] and base != math.e else node
+
+
 def _product_node(A, B, offset, approx_bwd, BMM):
     node = node_arguments(cuda_kernels, HipKernels, offset, approx_bwd)
     if node is not None and isinstance(A, torch.Tensor) and isinstance(B, torch.Tensor):
@@ -259,11 +293,14 @@ class pa_exp_autograd(torch.autograd.Function):
 
 
 def pa_exp(X, *, base=math.e, offset=None, approx_bwd=False):
+    node = _unary_node(X, base, offset, approx_bwd)
+    if node is not None:
+        return host().unary(X, 0, base, node[0], node[1], node[3])
     return pa_exp_autograd.apply(X, base, offset, approx_bwd)
 
 
 def pa_exp2(X, *, offset=None, approx_bwd=False):
-    return pa_exp_autograd.apply(X, 2.0, offset, approx_bwd)
+    return pa_exp(X, base=2.0, offset=offset, approx_bwd=approx_bwd)
 
 
 class pa_log_autograd(torch.autograd.Function):
@@ -291,8 +328,11 @@ class pa_log_autograd(torch.autograd.Function):
 
 
 def pa_log(X, *, base=math.e, offset=None, approx_bwd=False):
+    node = _unary_node(X, base, offset, approx_bwd)
+    if node is not None:
+        return host().unary(X, 1, base, node[0], node[1], node[3])
     return pa_log_autograd.apply(X, base, offset, approx_bwd)
 
 
 def pa_log2(X, *, offset=None, approx_bwd=False):
-    return pa_log_autograd.apply(X, 2.0, offset, approx_bwd)
+    return pa_log(X, base=2.0, offset=offset, approx_bwd=approx_bwd)

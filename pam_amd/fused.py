@@ -7,7 +7,7 @@ rows instead of five to fifteen elementwise launches.  The only difference is th
 the row sums, which the reference leaves to torch.sum and the kernels fix.
 
 `row_kernels` is the kernel object; it may be swapped for another one with the same methods.  With the package's own,
-softmax, layer_norm and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp) that make the same calls; the
+softmax, logsumexp, log_softmax, layer_norm, pow with a number and the linear layer with its bias are nodes in C++ (csrc/pam_host.cpp) that make the same calls; the
 autograd functions here are for other objects and for calls that are traced.
 `fusable` says whether a call can take this path: float32 GPU tensor, contiguous, reduced dimension last, not empty.
 """
@@ -16,7 +16,7 @@ import torch
 from . import _abi
 from . import cuda_bindings
 from ._abi import HipKernels, HipRowKernels
-from .cuda_bindings import _both, _offset_value, node_arguments
+from .cuda_bindings import _ORDINARY, _both, _offset_value, node_arguments, whole_floats
 
 row_kernels = HipRowKernels()
 
@@ -54,11 +54,6 @@ class softmax_autograd(torch.autograd.Function):
         g = grad.contiguous().view(rows.shape)
         dx = row_kernels.softmax_bwd(rows, g, row_sum, shift, ctx.offset, *_flags(ctx.approx_bwd))
         return dx.view(grad.shape), None, None
-
-
-# The classes whose results are ordinary tensors: an op on a tensor of another class has a result of that class, which the
-# autograd functions in Python make (torch.empty_like keeps the class).
-_ORDINARY = (torch.Tensor, torch.nn.Parameter)
 
 
 def softmax(x, offset=None, approx_bwd=False):
@@ -105,12 +100,35 @@ class logsumexp_autograd(torch.autograd.Function):
         return dx, None, None, None, None, None
 
 
+def _logsumexp_node(x, offset, approx_bwd, as_log_softmax, check_finite):
+    """The node in C++, or None where the autograd function in Python is to be called.  check_finite: the host waits for the
+    pass that looks at the input, while the rows' own pass is already launched behind it."""
+    node = node_arguments(row_kernels, HipRowKernels, offset, approx_bwd)
+    if node is None or not whole_floats(x):
+        return None
+    if not check_finite:
+        return _abi.host().logsumexp(x, as_log_softmax, 0, 0, *node)
+    with _abi._on(x.device):
+        word, nonfinite, event = _abi._finite_word.get(x.device)
+        nonfinite.value = 0
+        out = _abi.host().logsumexp(x, as_log_softmax, word.data_ptr(), event.cuda_event, *node)
+        event.synchronize()
+        if nonfinite.value != 0:
+            raise AssertionError("logsumexp and log_softmax need finite inputs")
+    return out
+
+
 def logsumexp(x, keepdim, offset=None, approx_bwd=False, check_finite=False):
-    out = logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, False, True, check_finite)
+    out = _logsumexp_node(x, offset, approx_bwd, False, check_finite)
+    if out is None:
+        out = logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, False, True, check_finite)
     return out.view(x.shape[:-1] + ((1,) if keepdim else ()))
 
 
 def log_softmax(x, offset=None, approx_bwd=False, check_finite=False):
+    out = _logsumexp_node(x, offset, approx_bwd, True, check_finite)
+    if out is not None:
+        return out
     return logsumexp_autograd.apply(x.reshape(-1, x.shape[-1]), offset, approx_bwd, True, True, check_finite).view(x.shape)
 
 
@@ -207,6 +225,9 @@ def pow_in_place(A, B):
 
 
 def pow_scalar(A, exponent, offset=None, approx_bwd=False):
+    node = node_arguments(cuda_bindings.cuda_kernels, HipKernels, offset, approx_bwd) if whole_floats(A) else None
+    if node is not None:
+        return _abi.host().unary(A, 2, float(exponent), node[0], node[1], node[3])
     return pow_autograd.apply(A, exponent, offset, approx_bwd)
 
 

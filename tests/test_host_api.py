@@ -585,3 +585,52 @@ def test_refusals_say_what_they_said():
             (lambda: pam_amd.matmul(x, w.t().cpu()), RuntimeError, "argument must be a CUDA tensor")):
         with pytest.raises(error, match=text):
             call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [None, 1.0552])
+@pytest.mark.parametrize("approx", [True, False, (True, False), (False, True)])
+def test_elementwise_and_log_softmax_nodes_equal_the_autograd_functions(offset, approx):
+    """Results, gradients (also of an expanded upstream gradient, and of one operand alone) and refusals of the nodes in C++
+    are those of the autograd functions in Python."""
+    import math
+    from pam_amd import cuda_bindings as cb, fused
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a0, b0 = torch.randn(37, 129, generator=g, device="cuda"), torch.randn(37, 129, generator=g, device="cuda")
+    b0[0, :5] = torch.tensor([0.0, 1e-40, 3e38, -1e-30, -0.0])
+    pos = a0.abs() + 1e-3
+    kw = dict(offset=offset, approx_bwd=approx)
+    pairs = [(lambda a, b: pam_amd.mul(a, b, **kw), lambda a, b: cb.pam_autograd.apply(a, b, offset, approx), (a0, b0)),
+             (lambda a, b: pam_amd.div(a, b, **kw), lambda a, b: cb.pad_autograd.apply(a, b, offset, approx), (a0, b0))]
+    for base in (math.e, 2.0, 10):
+        pairs += [(lambda a, base=base: cb.pa_exp(a, base=base, **kw), lambda a, base=base: cb.pa_exp_autograd.apply(a, base, offset, approx), (a0,)),
+                  (lambda a, base=base: cb.pa_log(a, base=base, **kw), lambda a, base=base: cb.pa_log_autograd.apply(a, base, offset, approx), (pos,))]
+    pairs += [(lambda a, p=p: pam_amd.pow(a, p, **kw), lambda a, p=p: fused.pow_autograd.apply(a, p, offset, approx), (pos,)) for p in (0.5, 3)]
+    rows = lambda a: a.reshape(-1, a.shape[-1])
+    pairs += [(lambda a: pam_amd.log_softmax(a, dim=-1, **kw), lambda a: fused.logsumexp_autograd.apply(rows(a), offset, approx, True, True).view(a.shape), (a0,)),
+              (lambda a: pam_amd.logsumexp(a, -1, **kw), lambda a: fused.logsumexp_autograd.apply(rows(a), offset, approx, False, True).view(a.shape[:-1]), (a0,)),
+              (lambda a: pam_amd.logsumexp(a, -1, keepdim=True, **kw), lambda a: fused.logsumexp_autograd.apply(rows(a), offset, approx, False, True).view(a.shape[:-1] + (1,)), (a0,))]
+    same = lambda x, y: x.shape == y.shape and torch.equal(x.nan_to_num(5.0, 6.0, 7.0), y.nan_to_num(5.0, 6.0, 7.0))
+    for node, function, values in pairs:
+        makes = [lambda t: t.clone(), lambda t: t.view(37, 1, 129).clone(), lambda t: torch.zeros(129, 37, device="cuda").t().copy_(t)]
+        for make in makes[:2] if (node, function, values) in pairs[-3:] else makes:      # (rows that are not contiguous are a chain of ops)
+            mine, theirs = [make(v).requires_grad_() for v in values], [make(v).requires_grad_() for v in values]
+            y, want = node(*mine), function(*[t.contiguous() for t in theirs])
+            assert same(y, want) and y.requires_grad and torch.equal(node(*[t.detach() for t in mine]).nan_to_num(5.0), y.detach().nan_to_num(5.0))
+            for up in (torch.randn(y.shape, generator=g, device="cuda"), torch.full((1,), 0.7, device="cuda").expand(y.shape)):
+                got = torch.autograd.grad(y, mine, up, retain_graph=True)
+                assert all(same(p, q) for p, q in zip(got, torch.autograd.grad(want, theirs, up, retain_graph=True)))
+                assert same(torch.autograd.grad(y, mine[-1], up, retain_graph=True)[0], got[-1])
+            if len(mine) == 2:                              # one gradient wanted, then broadcast operands and numbers
+                one = node(mine[0], values[1].view(mine[0].shape))
+                assert same(torch.autograd.grad(one.sum(), mine[0])[0], torch.autograd.grad(want.sum(), theirs[0], retain_graph=True)[0])
+                assert same(node(mine[0], values[1][:1, :1].expand(37, 129).reshape(mine[0].shape)), node(mine[0], values[1][0, 0]))
+                assert same(node(mine[0], 1.5), node(mine[0], torch.full_like(mine[0], 1.5)))
+    with pytest.raises(TypeError, match="float32"):
+        pam_amd.mul(a0.double(), b0.double(), **kw)
+    for bad in (float("inf"), float("nan")):
+        x = a0.clone(); x[3, 4] = bad
+        for op in (pam_amd.log_softmax, pam_amd.logsumexp):
+            with pytest.raises(AssertionError):
+                op(x, -1, **kw)
+    assert torch.equal(pam_amd.log_softmax(a0, -1, **kw), pam_amd.log_softmax(a0, -1, **kw))      # (the word was cleared)
