@@ -59,8 +59,9 @@ constexpr long kFewLongest = 512;
 // than the rule for large products does pays: pieces down to 32 k, as long as all units are resident.  The time of a unit,
 // in k-steps of a work-group alone on its compute unit, is its k (0.88 of it in 32-deep k-tiles), two thirds of the k over a
 // whole k-tile and 170 for start, first fetch and way out, times up to 1.66 for four busy work-groups on a compute unit; pieces
-// cost 15 and 1.5 each where the tile's last arriver adds them up, 20 and 0.9 each in the second kernel.  Fitted on a third of
-// 2934 drawn products timed in both k-tile depths with 1 ... 64 pieces, checked on the others: 1.02 of the best time each, where the rule below
+// cost 15 and 1.5 each where the tile's last arriver adds them up, 45 and 0.9 each in the second kernel (20 on the GPU; the
+// rest is the host's time for another launch, which is what a small layer's step waits for).  Fitted on a third of
+// 2934 drawn products timed in both k-tile depths with 1 ... 64 pieces, checked on the others: 1.03 of the best time each, where the rule below
 // took 1.27 (1.49 for up to 16 tiles, 1.33 up to 64, 1.23, 1.14 and 1.07 up to 128, 256 and 512); beyond 500 k-steps per compute
 // unit the two are even.  The three products of 60 drawn linear layers: 1.21 times as fast, 0.88 to 2.2.  197 x 768, k = 192 18.3 -> 12.9 us;
 // 450 x 333, 190 21.0 -> 14.6; 800 x 360, 190 22.1 -> 14.8; 5000 x 150, 200 22.0 -> 16.8.
@@ -76,7 +77,7 @@ bool small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
             const long per = (kt + w - 1) / w, pieces = (kt + per - 1) / per, n = tiles * pieces;
             const double crowd = n <= cus ? 1.0 : 1.0 + busy * (double)(n - cus) / (double)(resident - cus);
             const double unit = (double)std::min(per * bk, K) * (bk == 32 ? 0.88 : 1.0) + 0.65 * (double)(K % bk) + 170.0;
-            const double time = unit * crowd + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 15.0 + 1.5 * (double)pieces : 20.0 + 0.9 * (double)pieces);
+            const double time = unit * crowd + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 15.0 + 1.5 * (double)pieces : 45.0 + 0.9 * (double)pieces);
             if (best == 0.0 || time < best) { best = time; p.bk = bk; p.kt = (int)kt; p.pieces = (int)pieces; p.piece_kt = (int)per; }
         }
     }
@@ -91,7 +92,7 @@ bool small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
 // range into equal pieces, each at least 128 deep in k: few pieces by the cost model below (the tile's last
 // work-group adds them up), or, where that asks for more than a work-group should add up, about two resident rounds of
 // piece-major units and a second kernel.
-Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
+Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
 {
     const long resident = (long)kResidentPerCu * cu_count();
     const long tiles = batch * ((M + 63) / 64) * ((N + 63) / 64);
@@ -152,6 +153,21 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
     }
     p.units = tiles * p.pieces;
     return p;
+}
+
+// The plans of a thread's last products by their sizes: a call asks for its plan twice (scratch, launch), and a program for the
+// same ones again and again.  (Finding one takes up to a microsecond.)
+Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
+{
+    if (g_force_bk || g_force_pieces) return find_plan(batch, M, N, K, with_workspace);
+    struct Found { long batch, M, N, K; int cus; bool with_workspace; Plan plan; };
+    constexpr int kFound = 64;
+    thread_local Found found[kFound] = {};
+    const int cus = cu_count();
+    Found& f = found[(size_t)(batch * 7 + M * 31 + N * 13 + K * 3 + (with_workspace ? 1 : 0)) % kFound];
+    if (f.batch != batch || f.M != M || f.N != N || f.K != K || f.cus != cus || f.with_workspace != with_workspace)
+        f = Found{batch, M, N, K, cus, with_workspace, find_plan(batch, M, N, K, with_workspace)};
+    return f.plan;
 }
 
 // Whether a launch's work-groups lower their priority by quarters of their k-tiles, so that those on a compute unit end
