@@ -43,7 +43,7 @@ def parse():
 SETTLE_S = 0.03
 HERE = os.path.dirname(os.path.abspath(__file__))
 TRAFFIC_FILE = os.path.join(HERE, "profiles", "traffic.json")
-HEADLINE_KERNEL = "gemm_kernel<64, 64, 4, 4, 32, 0, 0, 0, false>"      # whole tiles, both operands contiguous along k
+HEADLINE_KERNEL = "gemm_kernel<64, 64, 4, 4, 32, 0, 0, 0, false, false>"      # whole tiles, both operands contiguous along k
 ELEMENTWISE_KERNEL = "ew_vec_kernel<OpPam, 2>"
 
 
