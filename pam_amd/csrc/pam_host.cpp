@@ -70,9 +70,13 @@ Tensor new_floats(at::IntArrayRef shape, const Tensor& like) { return at::empty(
 // grown as needed.  Products on one stream run one after the other, and each leaves the arrival words ready for the
 // next one; products on different streams may overlap in time and must not share a buffer.  The lock covers the table
 // only: buffers are allocated and given back outside it, since the allocator may wait for the device or for the
-// interpreter (its hooks), which another thread that waits for the lock might hold.
+// interpreter (its hooks), which another thread that waits for the lock might hold.  While the stream is captured a buffer
+// is the graph's own, given back to the graph's memory at once: graphs recorded on one stream may be replayed side by side.
 Tensor gemm_workspace(const Tensor& like, void* stream, size_t bytes)
 {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capturing) == hipSuccess && capturing != hipStreamCaptureStatusNone)
+        return new_floats({(int64_t)(bytes / 4 + 64)}, like);
     static std::mutex lock;
     static auto* kept = new std::map<std::pair<int, void*>, Tensor>;           // (not destroyed after the allocator at exit)
     const std::pair<int, void*> key{like.device().index(), stream};

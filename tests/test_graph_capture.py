@@ -127,3 +127,35 @@ def test_one_graph_replayed_many_times():
         assert torch.equal(sx.grad, xe.grad), f"replay {i}: input gradient"
         for (n, p), q in zip(model.named_parameters(), ref.parameters()):
             assert torch.equal(p.grad, q.grad), f"replay {i}: gradient of {n}"
+
+
+def test_graphs_with_products_in_pieces_side_by_side():
+    """Two graphs of products cut along k, recorded one after the other on one stream, replayed at the same time on two:
+    each has scratch of its own, and every replay gives the eager bits."""
+    from pam_amd import _abi
+    g = torch.Generator(device="cuda").manual_seed(3)
+    m, k, n = 192, 1024, 256
+    assert _abi.gemm_plan(1, m, n, k) < k
+    data = [(torch.randn(m, k, generator=g, device="cuda"), torch.randn(k, n, generator=g, device="cuda")) for _ in range(2)]
+    step = lambda a, b: [pam_amd.matmul(a, b)] + [pam_amd.matmul(a + i, b) for i in range(1, 6)]
+    want = [step(*d) for d in data]
+    stream = torch.cuda.Stream()
+    graphs, outputs = [], []
+    for d in data:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = step(*d)
+        graphs.append(graph)
+        outputs.append(out)
+    sides = [torch.cuda.Stream() for _ in graphs]
+    for _ in range(6):
+        for out in outputs:
+            for t in out:
+                t.zero_()
+        torch.cuda.synchronize()
+        for graph, side in zip(graphs, sides):
+            with torch.cuda.stream(side):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(t, w) for out, ws in zip(outputs, want) for t, w in zip(out, ws))
+        assert torch.equal(pam_amd.matmul(*data[0]), want[0][0])
