@@ -365,8 +365,10 @@ struct TileLoader {
                 int row = min(row0 + quad_row(tid, i), nrows - 4);
                 int kk = min(k0 + quad_k(tid, i), kend - 1);
                 const float* at = base + (long)kk * op.sk + row;
-                if (KIND == LOAD_RODD) v[i] = any_quad(at);
-                else v[i] = *reinterpret_cast<const float4*>(at);
+                // (one expression: as two statements, like those above, the instances with both operands along their rows ran the same loop 4 to
+                // 11 % slower where a compute unit has two work-groups or a launch a short second round: 210 of 128 x 144, k = 144 37.4 -> 40.5 us,
+                // 224 x 320, k = 8543 40.4 -> 42.8)
+                v[i] = KIND == LOAD_RODD ? any_quad(at) : *reinterpret_cast<const float4*>(at);
             }
         } else {
             float* s = reinterpret_cast<float*>(v);
