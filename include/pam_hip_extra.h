@@ -35,6 +35,12 @@ int pam_hip_column_sums(const float *a, long a_row_stride, float *a_sums, const 
  * priority as they proceed. */
 int pam_hip_gemm_priority_steps(long batch, long m, long n, long k, int exact);
 
+/* How the matrix kernel is launched for that product, with a workspace and operands that are each contiguous along one of
+ * their indices: the depth of its k-tiles, the outputs of one work-group and the number of work-groups.  kind: 0 PAM products
+ * (of up to four rows without an offset a kernel of their own may run instead), 1 the exact gradient's, 2 a convolution's. */
+int pam_hip_gemm_schedule(long batch, long m, long n, long k, int kind, int *k_tile, int *tile_rows, int *tile_columns,
+                          long *work_groups);
+
 #ifdef __cplusplus
 }
 #endif

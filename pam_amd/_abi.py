@@ -75,6 +75,7 @@ _SIGNATURES = {
 _EXTRA_SIGNATURES = {
     "pam_hip_logsumexp_fwd_finite": ([_p, _p, _p, _p, _l, _l, _f, _p, _p, _p, _z, _p], _i),
     "pam_hip_gemm_priority_steps": ([_l, _l, _l, _l, _i], _i),
+    "pam_hip_gemm_schedule": ([_l, _l, _l, _l, _i, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_l)], _i),
     "pam_hip_column_sums_workspace_bytes": ([_l, _l, _i], _z),
     "pam_hip_column_sums": ([_p, _l, _p, _p, _l, _p, _l, _l, _p, _z, _p], _i),
     "pam_hip_adam_step_many": ([_p, _l, _f, _f, _f, _f, _f, _f, _i, _f, _f, _p], _i),
@@ -147,6 +148,14 @@ def gemm_plan(batch, m, n, k):
     c = _i(0)
     _call("pam_hip_gemm_plan", batch, m, n, k, ctypes.byref(c))
     return c.value
+
+
+def gemm_schedule(batch, m, n, k, kind=0):
+    """(k-tile depth, rows and columns of a tile, work-groups) of the matrix kernel's launch; kind: 0 PAM products, 1 the
+    exact gradient's, 2 a convolution's (see pam_hip_gemm_schedule in include/pam_hip_extra.h)."""
+    depth, rows, columns, groups = _i(0), _i(0), _i(0), _l(0)
+    _call("pam_hip_gemm_schedule", batch, m, n, k, kind, ctypes.byref(depth), ctypes.byref(rows), ctypes.byref(columns), ctypes.byref(groups))
+    return depth.value, rows.value, columns.value, groups.value
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

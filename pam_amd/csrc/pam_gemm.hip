@@ -34,7 +34,9 @@ int cu_count()
 
 // How a product is scheduled (see the kernel's comment on units).  bk: depth of a k-tile; kt: k-tiles per output
 // tile; pieces, piece_kt: the k ranges a tile is cut into and their length in k-tiles; units = tiles x pieces.
-struct Plan { int bk, kt, pieces, piece_kt; long units; };
+// free: the freely shaped tiles that PAM products of operands read by 128-bit loads take instead (r = 0: none).
+struct FreeShape { int r, c; };
+struct Plan { int bk, kt, pieces, piece_kt; long units; FreeShape free; };
 
 // Tuning override for experiments, per calling thread (include/pam_hip_probe.h): bk 0 = automatic (16 or 32);
 // pieces 0 = automatic, > 0 that many k ranges per tile (as far as k allows).
@@ -49,6 +51,33 @@ long busy_waves(long M, long N)
 {
     const long full_m = M / 64, full_n = N / 64, rest_m = M % 64, rest_n = N % 64;
     return 4 * full_m * full_n + full_m * ((rest_n + 15) / 16) + full_n * ((rest_m + 15) / 16) + (std::min(rest_m, rest_n) + 15) / 16;
+}
+
+// Freely shaped tiles.  Matrices of a few tiles each whose sizes are no multiples of 64 (attention scores of 197 x 197: 16 tiles,
+// 7 of them with one busy wavefront) spend work-groups on their edges, and how long a batch of them takes goes by the number
+// of work-groups more than by their products.  A tile may instead have any r x c blocks of 4 x 4 outputs, one per lane, with r c up
+// to 256: 25 x 10 blocks cover 197 x 197 in ten tiles, nearly without idle lanes.  c is at most 16, so that a wavefront's
+// reads of the right fragment stay within 64 LDS banks (25 columns in 10 rows 34.3 us where 10 in 25 take 31.5), r at most 32.
+// What a tiling costs is counted in wavefronts plus two per work-group; a freely shaped one must save a twentieth of it, as
+// its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), or a tenth where the fixed tiles
+// are all resident and no round is saved (15362 x 160, k = 64, saving a seventeenth: 12.4 -> 13.2), and there must be more work-groups
+// than two per compute unit: with fewer, all run at once and their number does not matter.  Whole tiles of 16-deep k-tiles only.
+// Products of 192 x 197 x 197, k = 64: 37.4 -> 31.2 us; 212 x 148 x 148, 64: 25 -> 21.4; 120 x 257 x 131, 80: 29.6 -> 25.9;
+// 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7; of 120 drawn attention products none was more than 1 % slower.
+FreeShape free_shape(long batch, long M, long N, long K)
+{
+    FreeShape best{0, 0};
+    const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
+    const long waves = busy_waves(M, N);
+    const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
+    long least = (waves + 2 * tiles) * (batch * tiles > (long)kResidentPerCu * cu_count() ? 19 : 18) / 20;
+    for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {
+        const long tn = (fours_n + widest - 1) / widest, c = (fours_n + tn - 1) / tn, most = std::min<long>(kFreeFoursM, 256 / c), tm = (fours_m + most - 1) / most, r = (fours_m + tm - 1) / tm;
+        const long cost = tm * tn * ((r * c + 63) / 64 + 2);
+        if (cost < least) { least = cost; best = FreeShape{(int)r, (int)c}; }
+    }
+    return best;
 }
 
 constexpr int kFewRows = 4;                     // products that few_rows_kernel takes where their tiles are whole
@@ -97,6 +126,7 @@ Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
     const long resident = (long)kResidentPerCu * cu_count();
     const long tiles = batch * ((M + 63) / 64) * ((N + 63) / 64);
     Plan p;
+    p.free = FreeShape{0, 0};
     if (with_workspace && g_force_bk == 0 && g_force_pieces == 0 && small_plan(p, tiles, batch, M, N, K)) return p;
     p.bk = (K >= 512 || (K >= 128 && K % 32 == 0)) ? 32 : 16;
     if (g_force_bk) p.bk = g_force_bk;
@@ -162,14 +192,19 @@ Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
 // same ones again and again.  (Finding one takes up to a microsecond.)
 Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 {
-    if (g_force_bk || g_force_pieces) return find_plan(batch, M, N, K, with_workspace);
+    const auto find = [&] {
+        Plan p = find_plan(batch, M, N, K, with_workspace);
+        if (p.pieces == 1 && !g_force_bk && !g_force_pieces) p.free = free_shape(batch, M, N, K);
+        return p;
+    };
+    if (g_force_bk || g_force_pieces) return find();
     struct Found { long batch, M, N, K; int cus; bool with_workspace; Plan plan; };
     constexpr int kFound = 64;
     thread_local Found found[kFound] = {};
     const int cus = cu_count();
     Found& f = found[(size_t)(batch * 7 + M * 31 + N * 13 + K * 3 + (with_workspace ? 1 : 0)) % kFound];
     if (f.batch != batch || f.M != M || f.N != N || f.K != K || f.cus != cus || f.with_workspace != with_workspace)
-        f = Found{batch, M, N, K, cus, with_workspace, find_plan(batch, M, N, K, with_workspace)};
+        f = Found{batch, M, N, K, cus, with_workspace, find()};
     return f.plan;
 }
 
@@ -187,7 +222,7 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 // better of the two each time 0.979.
 // (Freely shaped tiles take the steps in a mostly full second round at any depth: 192 products of 197 x 197, k = 64 in 1920
 // work-groups 34.3 -> 33.1 us, 217 of 197 x 159 29.0 -> 27.1.)
-bool priority_steps(const Plan& p, long M, long N, bool exact, bool free_tiles = false)
+bool priority_steps(const Plan& p, long M, long N, bool exact)
 {
     const long cus = cu_count(), resident = (long)kResidentPerCu * cus;
     if (p.units <= resident) return p.units > resident / 2;
@@ -197,9 +232,24 @@ bool priority_steps(const Plan& p, long M, long N, bool exact, bool free_tiles =
     const long counted = p.pieces > pamgemm::kFoldInKernel && extra <= tiles && 3 * tail <= p.piece_kt ? p.units - extra : p.units;
     const long rounds = (counted + resident - 1) / resident, last = (counted - 1) % resident + 1;
     const bool most = last > resident / 2;
-    if (free_tiles && most && rounds <= 2) return true;
+    if (p.free.r > 0 && most && rounds <= 2) return true;
     if (p.piece_kt < (!exact || (most && rounds <= 2) ? 6 : most && rounds <= 3 ? 8 : 10)) return false;
     return most || (last > cus && rounds <= 3 && (p.piece_kt >= 20 || (p.pieces == 1 && M % 64 == 0 && N % 64 == 0)));
+}
+
+// What a launch makes of its sizes' plan.  conv: the right operand is an image's patches; quads: both operands are read by
+// 128-bit loads.
+Plan launch_plan(Plan p, bool pam, bool conv, bool quads, long batch, long M, long N, long K)
+{
+    // (convolutions stay with 16-deep k-tiles for ragged k of whole tiles: half a k-tile left over costs them more, 100 images of
+    // 16 x 32 x 32 to 64 channels, k = 144: 59.9 us, in 32-deep ones 64.7)
+    if (conv && p.pieces == 1 && p.bk == 32 && K < 512 && K % 32 != 0) { p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16); }
+    if (!pam || conv || !quads) p.free = FreeShape{0, 0};
+    if (p.free.r > 0) {
+        p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16);
+        p.units = batch * ((M + 4 * p.free.r - 1) / (4 * p.free.r)) * ((N + 4 * p.free.c - 1) / (4 * p.free.c));
+    }
+    return p;
 }
 
 // workspace of a plan that cuts tiles: [arrival words, one per tile][one piece per unit].  The words' part has one size
@@ -372,34 +422,6 @@ void odd_lines(long l_row, long l_k, long M, long r_row, long r_k, long N, long 
     if (l != LOAD_ANY && r != LOAD_ANY) { lk = l; rk = r; }
 }
 
-// Freely shaped tiles.  Matrices of a few tiles each whose sizes are no multiples of 64 (attention scores of 197 x 197: 16 tiles,
-// 7 of them with one busy wavefront) spend work-groups on their edges, and how long a batch of them takes goes by the number
-// of work-groups more than by their products.  A tile may instead have any r x c blocks of 4 x 4 outputs, one per lane, with r c up
-// to 256: 25 x 10 blocks cover 197 x 197 in ten tiles, nearly without idle lanes.  c is at most 16, so that a wavefront's
-// reads of the right fragment stay within 64 LDS banks (25 columns in 10 rows 34.3 us where 10 in 25 take 31.5), r at most 32.
-// What a tiling costs is counted in wavefronts plus two per work-group; a freely shaped one must save a twentieth of it, as
-// its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), or a tenth where the fixed tiles
-// are all resident and no round is saved (15362 x 160, k = 64, saving a seventeenth: 12.4 -> 13.2), and there must be more work-groups
-// than two per compute unit: with fewer, all run at once and their number does not matter.  Whole tiles of 16-deep k-tiles only.
-// Products of 192 x 197 x 197, k = 64: 37.4 -> 31.2 us; 212 x 148 x 148, 64: 25 -> 21.4; 120 x 257 x 131, 80: 29.6 -> 25.9;
-// 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7; of 120 drawn attention products none was more than 1 % slower.
-struct FreeShape { int r, c; };
-FreeShape free_shape(long batch, long M, long N, long K)
-{
-    FreeShape best{0, 0};
-    const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
-    if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
-    const long waves = busy_waves(M, N);
-    const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
-    long least = (waves + 2 * tiles) * (batch * tiles > (long)kResidentPerCu * cu_count() ? 19 : 18) / 20;
-    for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {
-        const long tn = (fours_n + widest - 1) / widest, c = (fours_n + tn - 1) / tn, most = std::min<long>(kFreeFoursM, 256 / c), tm = (fours_m + most - 1) / most, r = (fours_m + tm - 1) / tm;
-        const long cost = tm * tn * ((r * c + 63) / 64 + 2);
-        if (cost < least) { least = cost; best = FreeShape{(int)r, (int)c}; }
-    }
-    return best;
-}
-
 // One contiguous range of units per XCD (see the kernel), rounded up to whole work-groups per XCD; returns the work-groups.
 unsigned spread_over_xcds(GemmArgs& g)
 {
@@ -442,9 +464,17 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
     const bool usable = workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
     Plan p = make_plan(batch, M, N, K, usable);
     if (p.pieces > 1 && plan_space(p).total > workspace_bytes) p = make_plan(batch, M, N, K, false);       // whole tiles
-    // (convolutions stay with 16-deep k-tiles for ragged k of whole tiles: half a k-tile left over costs them more, 100 images of
-    // 16 x 32 x 32 to 64 channels, k = 144: 59.9 us, in 32-deep ones 64.7)
-    if (conv && p.pieces == 1 && p.bk == 32 && K < 512 && K % 32 != 0) { p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16); }
+    int lk = load_kind(l_sr, l_sc, l_sb, l, M, K);
+    int rk = conv ? LOAD_CONV : load_kind(r_sc, r_sr, r_sb, r, N, K);
+    if (!conv && mode != MODE_STD) odd_lines(l_sr, l_sc, M, r_sc, r_sr, N, K, lk, rk);
+    if (conv && conv->quads && !conv->transposed && mode == MODE_PAM && lk == LOAD_KVEC && K % 4 == 0 && (reinterpret_cast<uintptr_t>(r) & 15u) == 0 && r_sb % 4 == 0)
+        rk = LOAD_CONVQ;
+    else if (conv && conv->row_quads && !conv->transposed && mode != MODE_STD && lk == LOAD_KVEC && N % 4 == 0)
+        rk = LOAD_CONVR;
+    else if (conv && conv->row_quads && conv->transposed && mode != MODE_STD && lk == LOAD_KVEC && K % 4 == 0)
+        rk = LOAD_CONVK;
+    const bool few = mode == MODE_PAM && !conv && M <= kFewRows && K <= kFewLongest && p.pieces == 1 && offset == 1.0f && g_force_bk == 0 && g_force_pieces == 0;
+    p = launch_plan(p, mode == MODE_PAM && !few, conv != nullptr, lk != LOAD_ANY && rk != LOAD_ANY, batch, M, N, K);
     const Space sp = plan_space(p);
 
     GemmArgs g;
@@ -454,7 +484,9 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
     g.Y = y; g.y_sb = y_sb; g.y_sr = y_sr; g.y_sc = y_sc;
     g.bias = bias;
     g.M = (int)M; g.N = (int)N; g.K = (int)K;
-    g.ntn = (int)((N + 63) / 64); g.tiles = (int)(((M + 63) / 64) * g.ntn);
+    const long tile_m = p.free.r > 0 ? 4 * p.free.r : 64, tile_n = p.free.r > 0 ? 4 * p.free.c : 64;
+    g.ntn = (int)((N + tile_n - 1) / tile_n); g.tiles = (int)(((M + tile_m - 1) / tile_m) * g.ntn);
+    g.free_r = p.free.r; g.free_c = p.free.c;
     g.pieces = p.pieces; g.piece_kt = p.piece_kt; g.units = (int)p.units;
     g.xcd_chunk = 0;
     g.steps = priority_steps(p, M, N, mode >= MODE_BWD_DL) ? 1 : 0;
@@ -469,36 +501,18 @@ int gemm(const char* what, int mode, long batch, long M, long N, long K,
         g.off_add = bits - kBias;
     }
 
-    g.free_r = g.free_c = 0;
     g.cv = conv ? *conv : ConvGeom{nullptr, nullptr, 0, 0, 0, 0, 0};
 
-    if (mode == MODE_PAM && !conv && M <= kFewRows && K <= kFewLongest && p.pieces == 1 && g.has_off == 0 && g_force_bk == 0 && g_force_pieces == 0) {
+    if (few) {
         const unsigned groups = (unsigned)(batch * g.ntn);
         if (g.R.sk <= g.R.sr) hipLaunchKernelGGL(few_rows_kernel<true>, dim3(groups), dim3(256), 0, st, g);
         else hipLaunchKernelGGL(few_rows_kernel<false>, dim3(groups), dim3(256), 0, st, g);
         return pamhost::check_launch(what);
     }
-    int lk = load_kind(l_sr, l_sc, l_sb, l, M, K);
-    int rk = conv ? LOAD_CONV : load_kind(r_sc, r_sr, r_sb, r, N, K);
-    if (!conv && mode != MODE_STD) odd_lines(l_sr, l_sc, M, r_sc, r_sr, N, K, lk, rk);
-    if (conv && conv->quads && !conv->transposed && mode == MODE_PAM && lk == LOAD_KVEC && K % 4 == 0 && (reinterpret_cast<uintptr_t>(r) & 15u) == 0 && r_sb % 4 == 0)
-        rk = LOAD_CONVQ;
-    else if (conv && conv->row_quads && !conv->transposed && mode != MODE_STD && lk == LOAD_KVEC && N % 4 == 0)
-        rk = LOAD_CONVR;
-    else if (conv && conv->row_quads && conv->transposed && mode != MODE_STD && lk == LOAD_KVEC && K % 4 == 0)
-        rk = LOAD_CONVK;
-    if (mode == MODE_PAM && !conv && p.pieces == 1 && lk != LOAD_ANY && rk != LOAD_ANY && g_force_bk == 0 && g_force_pieces == 0) {
-        const FreeShape f = free_shape(batch, M, N, K);
-        if (f.r > 0) {
-            g.free_r = f.r; g.free_c = f.c;
-            g.ntn = (int)((N + 4 * f.c - 1) / (4 * f.c)); g.tiles = (int)((M + 4 * f.r - 1) / (4 * f.r)) * g.ntn;
-            p.units = batch * g.tiles; g.units = (int)p.units;
-            p.bk = 16; p.kt = p.piece_kt = g.piece_kt = (int)((K + 15) / 16);
-            g.steps = priority_steps(p, M, N, false, true) ? 1 : 0;
-            const unsigned groups = spread_over_xcds(g);
-            launch_free(odd_kind(lk), odd_kind(rk), groups, st, g);
-            return pamhost::check_launch(what);
-        }
+    if (p.free.r > 0) {
+        const unsigned groups = spread_over_xcds(g);
+        launch_free(odd_kind(lk), odd_kind(rk), groups, st, g);
+        return pamhost::check_launch(what);
     }
     switch (mode) {
     case MODE_PAM: launch_mode<MODE_PAM>(p, lk, rk, st, g); break;
@@ -829,7 +843,17 @@ void pam_hip_set_tuning(int bk, int pieces) { g_force_bk = bk; g_force_pieces = 
 int pam_hip_gemm_priority_steps(long batch, long m, long n, long k, int exact)
 {
     if (batch <= 0 || m <= 0 || n <= 0 || k < 0) return 0;
-    return priority_steps(make_plan(batch, m, n, k > 0 ? k : 1, true), m, n, exact != 0) ? 1 : 0;
+    return priority_steps(launch_plan(make_plan(batch, m, n, k > 0 ? k : 1, true), exact == 0, false, true, batch, m, n, k), m, n, exact != 0) ? 1 : 0;
+}
+
+int pam_hip_gemm_schedule(long batch, long m, long n, long k, int kind, int* k_tile, int* tile_rows, int* tile_columns, long* work_groups)
+{
+    if (batch <= 0 || m <= 0 || n <= 0 || k <= 0 || kind < 0 || kind > 2 || !k_tile || !tile_rows || !tile_columns || !work_groups)
+        return pamhost::fail(PAM_HIP_ERR_ARGUMENT, "gemm_schedule: bad shape, kind or null pointer");
+    const Plan p = launch_plan(make_plan(batch, m, n, k, true), kind == 0, kind == 2, true, batch, m, n, k);
+    *k_tile = p.bk; *work_groups = p.units;
+    *tile_rows = p.free.r > 0 ? 4 * p.free.r : 64; *tile_columns = p.free.r > 0 ? 4 * p.free.c : 64;
+    return PAM_HIP_OK;
 }
 
 int pam_hip_gemm_plan(long batch, long m, long n, long k, int* k_chunk)

@@ -380,6 +380,15 @@ def test_priorities_fall_only_where_the_last_round_fills_the_chip(shape, exact, 
     assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, exact) == want
 
 
+@pytest.mark.parametrize("shape,kind,schedule,steps", [
+    ((192, 197, 197, 64), 0, (16, 100, 40, 1920), 1), ((192, 197, 197, 64), 1, (16, 64, 64, 3072), 0),      # a mostly full second round; the exact gradient
+    ((1, 50432, 32, 64), 0, (16, 128, 32, 394), 0), ((1, 4096, 1024, 512), 0, (32, 64, 64, 1024), 1)])     # one per compute unit and a half; whole tiles
+def test_schedules_are_those_of_the_launch(shape, kind, schedule, steps):
+    """What the library reports of a product is what it launches, freely shaped tiles among them."""
+    assert _abi.gemm_schedule(*shape, kind) == schedule
+    assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, kind) == steps
+
+
 @pytest.mark.gpu
 def test_other_threads_run_while_a_launch_waits():
     """Behind one long product thousands of small ones fill the launch queue, and the next call waits for it: other
