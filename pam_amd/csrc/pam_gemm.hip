@@ -243,7 +243,7 @@ Plan launch_plan(Plan p, bool pam, bool conv, bool quads, long batch, long M, lo
 {
     // (convolutions stay with 16-deep k-tiles for ragged k of whole tiles: half a k-tile left over costs them more, 100 images of
     // 16 x 32 x 32 to 64 channels, k = 144: 59.9 us, in 32-deep ones 64.7)
-    if (conv && p.pieces == 1 && p.bk == 32 && K < 512 && K % 32 != 0) { p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16); }
+    if (conv && p.pieces == 1 && p.bk == 32 && K < 512 && K % 32 != 0 && !g_force_bk) { p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16); }
     if (!pam || conv || !quads) p.free = FreeShape{0, 0};
     if (p.free.r > 0) {
         p.bk = 16; p.kt = p.piece_kt = (int)((K + 15) / 16);

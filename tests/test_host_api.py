@@ -389,6 +389,18 @@ def test_schedules_are_those_of_the_launch(shape, kind, schedule, steps):
     assert _abi.load_library().pam_hip_gemm_priority_steps(*shape, kind) == steps
 
 
+def test_forced_k_tiles_hold_for_every_product():
+    """The tuning hook's depth is taken by products and convolutions alike, whatever the rule for their sizes is."""
+    lib, shape = _abi.load_library(), (100, 64, 1024, 144)
+    assert _abi.gemm_schedule(*shape, 2)[0] == 16
+    try:
+        for depth in (16, 32):
+            lib.pam_hip_set_tuning(depth, 1)
+            assert [_abi.gemm_schedule(*shape, kind)[0] for kind in (0, 1, 2)] == [depth] * 3
+    finally:
+        lib.pam_hip_set_tuning(0, 0)
+
+
 @pytest.mark.gpu
 def test_other_threads_run_while_a_launch_waits():
     """Behind one long product thousands of small ones fill the launch queue, and the next call waits for it: other
