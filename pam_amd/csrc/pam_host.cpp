@@ -254,6 +254,15 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     }
 };
 
+// A saved tensor as a backward pass reads it.  It comes back through the program's saved-tensor hooks, which may return any
+// tensor for it: another type, device or shape is refused, and other strides are copied.
+Tensor whole(const Tensor& saved, const Tensor& grad, at::IntArrayRef sizes, const char* name)
+{
+    check_tensor(saved);
+    TORCH_CHECK_VALUE(saved.sizes() == sizes && saved.device() == grad.device(), name, ": a saved tensor has not the shape or the device that it was saved with");
+    return saved.contiguous();
+}
+
 // ---------------------------------------------------------------- rows
 
 // softmax over the last dimension of a contiguous tensor; the gradient is the chain of the primitives' gradients
@@ -279,15 +288,16 @@ struct SoftmaxNode : torch::autograd::Function<SoftmaxNode> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &row_sum = saved[1], &shift = saved[2];
         const Approx f = Approx::saved(ctx);
         const at::AutoGradMode no_graph(false);
         const Tensor g = grads[0].contiguous();
         check_tensor(g);
-        const OnDevice on(x);
-        const Tensor dx = new_floats(x.sizes(), x);
-        if (x.numel())
-            check_call(pam_hip_softmax_bwd(data(x), data(g), data(row_sum), data(shift), data(dx), row_sum.numel(), x.size(-1),
+        const int64_t n = g.size(-1), rows = n ? g.numel() / n : 0;
+        const Tensor x = whole(saved[0], g, g.sizes(), "softmax_bwd"), row_sum = whole(saved[1], g, {rows}, "softmax_bwd"), shift = whole(saved[2], g, {1}, "softmax_bwd");
+        const OnDevice on(g);
+        const Tensor dx = new_floats(g.sizes(), g);
+        if (g.numel())
+            check_call(pam_hip_softmax_bwd(data(x), data(g), data(row_sum), data(shift), data(dx), rows, n,
                                            (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, f.e, on.stream), "softmax_bwd");
         return {dx, Tensor(), Tensor(), Tensor(), Tensor()};
     }
@@ -311,6 +321,7 @@ struct LayerNormNode : torch::autograd::Function<LayerNormNode> {
             check_call(pam_hip_layer_norm_fwd(data(x), data_or_null(w), data_or_null(c), data(y), x.numel() / n, n, (float)eps, (float)offset, on.stream),
                        "layer_norm_fwd");
         ctx->saved_data["n"] = n; ctx->saved_data["eps"] = eps; ctx->saved_data["offset"] = offset;
+        if (w.defined()) ctx->saved_data["weight"] = w.sizes();
         if (c.defined()) ctx->saved_data["bias"] = c.sizes();
         Approx{a, b, e}.save(ctx);
         ctx->save_for_backward({x, w});
@@ -319,17 +330,18 @@ struct LayerNormNode : torch::autograd::Function<LayerNormNode> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &w = saved[1];
         const Approx f = Approx::saved(ctx);
-        const int64_t n = ctx->saved_data["n"].toInt(), rows = x.numel() / n;
+        const Tensor g = grads[0].contiguous();
+        check_tensor(g);
+        const int64_t n = ctx->saved_data["n"].toInt(), rows = g.numel() / n;
+        const Tensor x = whole(saved[0], g, g.sizes(), "layer_norm_bwd");
+        const Tensor w = saved[1].defined() ? whole(saved[1], g, ctx->saved_data["weight"].toIntVector(), "layer_norm_bwd") : Tensor();
         const bool has_bias = ctx->saved_data.count("bias") != 0;
         // (edges are counted over the tensors that are there)
         const bool want_w = w.defined() && ctx->needs_input_grad(1), want_b = has_bias && ctx->needs_input_grad(w.defined() ? 2 : 1);
-        const Tensor g = grads[0].contiguous();
-        check_tensor(g);
-        const OnDevice on(x);
-        const Tensor dx = new_floats(x.sizes(), x), terms = want_w ? new_floats({rows, n}, x) : Tensor();
-        if (x.numel())
+        const OnDevice on(g);
+        const Tensor dx = new_floats(g.sizes(), g), terms = want_w ? new_floats({rows, n}, g) : Tensor();
+        if (g.numel())
             check_call(pam_hip_layer_norm_bwd(data(x), data_or_null(w), data(g), data(dx), data_or_null(terms), rows, n,
                                               (float)ctx->saved_data["eps"].toDouble(), (float)ctx->saved_data["offset"].toDouble(),
                                               f.a, f.b, f.e, on.stream), "layer_norm_bwd");
@@ -369,7 +381,7 @@ struct LogsumexpNode : torch::autograd::Function<LogsumexpNode> {
                                                     reinterpret_cast<void*>(checked), data(ws), bytes, on.stream), "logsumexp_fwd_finite");
         else
             check_call(pam_hip_logsumexp_fwd(data(x), lse, out, data(shift), rows, n, (float)offset, data(ws), bytes, on.stream), "logsumexp_fwd");
-        ctx->saved_data["offset"] = offset; ctx->saved_data["log_softmax"] = log_softmax;
+        ctx->saved_data["offset"] = offset; ctx->saved_data["log_softmax"] = log_softmax; ctx->saved_data["n"] = n;
         Approx{a, b, e}.save(ctx);
         ctx->save_for_backward({x, shift});
         return y;
@@ -377,14 +389,18 @@ struct LogsumexpNode : torch::autograd::Function<LogsumexpNode> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &shift = saved[1];
         const Approx f = Approx::saved(ctx);
         const at::AutoGradMode no_graph(false);
         const Tensor g = grads[0].contiguous();
         check_tensor(g);
-        const OnDevice on(x);
-        const Tensor dx = new_floats(x.sizes(), x);
-        check_call(pam_hip_logsumexp_bwd(data(x), data(g), data(shift), data(dx), x.numel() / x.size(-1), x.size(-1), ctx->saved_data["log_softmax"].toBool(),
+        const bool log_softmax = ctx->saved_data["log_softmax"].toBool();
+        const int64_t n = ctx->saved_data["n"].toInt(), rows = log_softmax ? g.numel() / n : g.numel();
+        std::vector<int64_t> shape = g.sizes().vec();
+        shape.back() = n;
+        const Tensor x = whole(saved[0], g, shape, "logsumexp_bwd"), shift = whole(saved[1], g, {1}, "logsumexp_bwd");
+        const OnDevice on(g);
+        const Tensor dx = new_floats(shape, g);
+        check_call(pam_hip_logsumexp_bwd(data(x), data(g), data(shift), data(dx), rows, n, log_softmax,
                                          (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, f.e, on.stream), "logsumexp_bwd");
         return {dx, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
@@ -411,15 +427,16 @@ struct PairNode : torch::autograd::Function<PairNode<DIVIDE>> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &A = saved[0], &B = saved[1];
+        const char* const name = DIVIDE ? "pad_bwd_pair" : "pam_bwd_pair";
         const Approx f = Approx::saved(ctx);
         const at::AutoGradMode no_graph(false);
         const Tensor g = grads[0].contiguous();
         check_tensor(g);
-        const OnDevice on(A);
-        const Tensor dA = new_floats(A.sizes(), A), dB = new_floats(A.sizes(), A);
-        check_call((DIVIDE ? pam_hip_pad_bwd_pair : pam_hip_pam_bwd_pair)(data(A), data(B), data(g), data(dA), data(dB), A.numel(),
-                   (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, on.stream), DIVIDE ? "pad_bwd_pair" : "pam_bwd_pair");
+        const Tensor A = whole(saved[0], g, g.sizes(), name), B = whole(saved[1], g, g.sizes(), name);
+        const OnDevice on(g);
+        const Tensor dA = new_floats(g.sizes(), g), dB = new_floats(g.sizes(), g);
+        check_call((DIVIDE ? pam_hip_pad_bwd_pair : pam_hip_pam_bwd_pair)(data(A), data(B), data(g), data(dA), data(dB), g.numel(),
+                   (float)ctx->saved_data["offset"].toDouble(), f.a, f.b, on.stream), name);
         return {dA, dB, Tensor(), Tensor(), Tensor()};
     }
 };
@@ -444,22 +461,22 @@ struct UnaryNode : torch::autograd::Function<UnaryNode> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor& x = saved[0];
         const Approx f = Approx::saved(ctx);
         const int64_t op = ctx->saved_data["op"].toInt();
         const float number = (float)ctx->saved_data["number"].toDouble(), offset = (float)ctx->saved_data["offset"].toDouble();
         const at::AutoGradMode no_graph(false);
         const Tensor g = grads[0].contiguous();
         check_tensor(g);
-        const OnDevice on(x);
-        const Tensor dx = new_floats(x.sizes(), x);
-        const size_t n = x.numel();
+        const Tensor x = whole(saved[0], g, g.sizes(), op == kExp ? "pa_exp_bwd" : op == kLog ? "pa_log_bwd" : "pow_bwd");
+        const OnDevice on(g);
+        const Tensor dx = new_floats(g.sizes(), g);
+        const size_t n = g.numel();
         if (op == kPow) {
             check_call(pam_hip_pow_bwd(data(x), data(g), data(dx), n, number, offset, f.a, f.e, on.stream), "pow_bwd");
         } else if (!f.e) {
             check_call((op == kExp ? pam_hip_pa_exp_bwd : pam_hip_pa_log_bwd)(data(x), data(g), data(dx), n, number, offset, on.stream), op == kExp ? "pa_exp_bwd" : "pa_log_bwd");
         } else if (op == kExp) {
-            const Tensor y = new_floats(x.sizes(), x);
+            const Tensor y = new_floats(g.sizes(), g);
             check_call(pam_hip_pa_exp_fwd(data(x), data(y), n, number, offset, on.stream), "pa_exp_fwd");
             check_call(pam_hip_pam_fwd(data(y), data(g), data(dx), n, offset, on.stream), "pam_fwd");
         } else {

@@ -662,3 +662,34 @@ def test_elementwise_and_log_softmax_nodes_equal_the_autograd_functions(offset, 
             with pytest.raises(AssertionError):
                 op(x, -1, **kw)
     assert torch.equal(pam_amd.log_softmax(a0, -1, **kw), pam_amd.log_softmax(a0, -1, **kw))      # (the word was cleared)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["mul", "div", "exp", "log", "pow", "softmax", "logsumexp", "log_softmax", "layer_norm"])
+@pytest.mark.parametrize("approx", [True, False])
+def test_saved_tensors_come_back_from_hooks_in_any_layout(op, approx):
+    """Hooks may return other strides for a saved tensor, which give the same gradients; one of another type, size or device
+    is refused before a kernel sees it."""
+    torch.manual_seed(8)
+    kw = dict(approx_bwd=approx)
+    f = {"mul": lambda a, b: pam_amd.mul(a, b, **kw), "div": lambda a, b: pam_amd.div(a, b, **kw), "exp": lambda a, b: pam_amd.exp(a, **kw),
+         "log": lambda a, b: pam_amd.log(a, **kw), "pow": lambda a, b: pam_amd.pow(a, 0.5, **kw), "softmax": lambda a, b: pam_amd.softmax(a, dim=-1, **kw),
+         "logsumexp": lambda a, b: pam_amd.logsumexp(a, -1, **kw), "log_softmax": lambda a, b: pam_amd.log_softmax(a, dim=-1, **kw),
+         "layer_norm": lambda a, b: pam_amd.layer_norm(a, 40, b[0], b[1], **kw)}[op]
+    a, b = (torch.rand(24, 40, device="cuda").add_(0.1).requires_grad_() for _ in range(2))
+    leaves = (a, b) if op in ("mul", "div") else (a,)
+    y = f(a, b)
+    assert op == "logsumexp" or "Node" in y.grad_fn.name()
+    dy = torch.randn_like(y)
+    want = torch.autograd.grad(y, leaves, dy)
+    def gradients(unpack):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), unpack):
+            y = f(a, b)
+        return torch.autograd.grad(y, leaves, dy)
+    def strided(t):
+        return torch.zeros(*t.shape, 2, device="cuda")[..., 0].copy_(t)
+    assert all(torch.equal(p, q) for p, q in zip(gradients(strided), want))
+    assert all(torch.equal(p, q) for p, q in zip(gradients(lambda t: strided(t.t()).t() if t.dim() == 2 else t), want))
+    for unpack, error in ((lambda t: t.double(), TypeError), (lambda t: t.cpu(), RuntimeError), (lambda t: t[:0], ValueError)):
+        with pytest.raises(error):
+            gradients(unpack)
