@@ -354,6 +354,23 @@ def test_gpu_softmax_forward_backward(oracle, off):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("off", [None, OFF])
+@pytest.mark.parametrize("largest", [[0.0], [-0.0], [-0.0, 0.0], [-1e-40], [1e-40], [-1.2e-38], [3e38], [-2.4e38], [-3.4e38], [np.inf], [np.nan], [np.inf, -np.inf], [3e38, -np.inf], [-np.inf]])
+def test_gpu_global_maximum_of_any_value(oracle, largest, off):
+    """The shift follows from the largest input alone, which is scaled once: where that is a zero of either sign, subnormal,
+    overflows when scaled, or is not finite, the result is the oracle's, which scales every value."""
+    for rows, n in [(1, 1), (2, 3), (5, 197), (70, 33), (3, 4096)]:
+        x = (min(max(np.nan_to_num(min(largest), posinf=0.0, neginf=0.0), -3e38), 0.0) - np.abs(np.random.RandomState(n).standard_normal((rows, n)))).astype(np.float32)
+        x.reshape(-1)[[i * (x.size - 1) // max(len(largest) - 1, 1) for i in range(len(largest))]] = largest
+        want, row_sum, shift = oracle.softmax_fwd(x, off)
+        assert_same_bits(pam_amd.softmax(_dev(x), dim=-1, offset=off).cpu().numpy(), want, f"softmax {rows}x{n} {largest}")
+        if np.isfinite(x).all():
+            lse, ls = oracle.logsumexp_fwd(x, off, with_log_softmax=True)
+            assert_same_bits(pam_amd.logsumexp(_dev(x), -1, offset=off).cpu().numpy(), lse, f"logsumexp {rows}x{n} {largest}")
+            assert_same_bits(pam_amd.log_softmax(_dev(x), dim=-1, offset=off).cpu().numpy(), ls, f"log_softmax {rows}x{n} {largest}")
+
+
+@pytest.mark.gpu
 def test_gpu_softmax_matches_unfused_composition(oracle):
     """The single kernel against the chain of primitive kernels on the same device: equal up to
     the order of the row sums; leading dimensions and the module-level switch."""
