@@ -129,15 +129,25 @@ def test_one_graph_replayed_many_times():
             assert torch.equal(p.grad, q.grad), f"replay {i}: gradient of {n}"
 
 
-def test_graphs_with_products_in_pieces_side_by_side():
+@pytest.mark.parametrize("m,k,n,added_by_last", [(192, 1024, 256, False), (1024, 256, 512, True)])
+def test_graphs_with_products_in_pieces_side_by_side(m, k, n, added_by_last):
     """Two graphs of products cut along k, recorded one after the other on one stream, replayed at the same time on two:
-    each has scratch of its own, and every replay gives the eager bits."""
+    each has scratch of its own, which other tensors of the graph take in between, and every replay gives the eager bits.  Up to
+    eight pieces are added up by the tile's last work-group, by arrival words in that scratch; more by a second kernel."""
     from pam_amd import _abi
     g = torch.Generator(device="cuda").manual_seed(3)
-    m, k, n = 192, 1024, 256
-    assert _abi.gemm_plan(1, m, n, k) < k
+    pieces = -(-k // _abi.gemm_plan(1, m, n, k))
+    assert 2 <= pieces <= 8 if added_by_last else pieces > 8
     data = [(torch.randn(m, k, generator=g, device="cuda"), torch.randn(k, n, generator=g, device="cuda")) for _ in range(2)]
-    step = lambda a, b: [pam_amd.matmul(a, b)] + [pam_amd.matmul(a + i, b) for i in range(1, 6)]
+    def step(a, b):
+        out = [pam_amd.matmul(a, b)]
+        for i in range(1, 6):
+            # (tensors of the scratch's sizes and below, written over what it held)
+            other = [torch.full((n,), float(i), device="cuda") for n in (1 << 12, 1 << 16, 1 << 18, 1 << 20, 1 << 22)]
+            out.append(pam_amd.matmul(a + other[0][0], b))
+            del other
+            out.append(pam_amd.matmul(a + i, b))
+        return out
     want = [step(*d) for d in data]
     stream = torch.cuda.Stream()
     graphs, outputs = [], []
