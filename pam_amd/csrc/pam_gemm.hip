@@ -85,33 +85,50 @@ constexpr long kFewLongest = 512;
 
 // Products that fit the chip at once: up to 1024 tiles whose k-steps come to less than 500 per compute unit.  There a
 // work-group's chain of k-tiles is what takes the time, one wavefront per SIMD issues at half rate, and cutting k much finer
-// than the rule for large products does pays: pieces down to 32 k, as long as all units are resident.  The time of a unit,
-// in k-steps of a work-group alone on its compute unit, is its k (0.88 of it in 32-deep k-tiles), two thirds of the k over a
-// whole k-tile and 170 for start, first fetch and way out, times up to 1.66 for four busy work-groups on a compute unit; pieces
-// cost 15 and 1.5 each where the tile's last arriver adds them up, 45 and 0.9 each in the second kernel (20 on the GPU; the
-// rest is the host's time for another launch, which is what a small layer's step waits for).  Fitted on a third of
-// 2934 drawn products timed in both k-tile depths with 1 ... 64 pieces, checked on the others: 1.03 of the best time each, where the rule below
-// took 1.27 (1.49 for up to 16 tiles, 1.33 up to 64, 1.23, 1.14 and 1.07 up to 128, 256 and 512); beyond 500 k-steps per compute
-// unit the two are even.  The three products of 60 drawn linear layers: 1.21 times as fast, 0.88 to 2.2.  197 x 768, k = 192 18.3 -> 12.9 us;
-// 450 x 333, 190 21.0 -> 14.6; 800 x 360, 190 22.1 -> 14.8; 5000 x 150, 200 22.0 -> 16.8.
-bool small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
+// than the rule for large products does pays: pieces down to 32 k, as long as all units are resident.
+bool fits_at_once(long tiles, long M, long K)
 {
-    const long cus = cu_count(), resident = (long)kResidentPerCu * cus;
-    if (tiles > resident || tiles * K >= 500 * cus || (M <= kFewRows && K <= kFewLongest)) return false;
-    const double busy = 0.66 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles);
-    double best = 0.0;
+    return tiles <= (long)kResidentPerCu * cu_count() && tiles * K < 500L * cu_count() && !(M <= kFewRows && K <= kFewLongest);
+}
+
+// The time of a product there, in k-steps of a work-group alone on its compute unit.  A unit takes its k (0.9 of it in 32-deep
+// k-tiles), 0.62 more of what is over a whole k-tile where that is the longest unit, and 280 for start, first fetch and way out; up to 1.34 times
+// that where four busy work-groups share a compute unit, counted on the fullest one (every XCD takes an eighth of the units; a unit over on one of
+// them does not count) and on all of them about evenly, since a few full ones end late and the others early.  Wavefronts without outputs count little, not
+// nothing: they stage.  Pieces cost 13 and 3.85 each where the tile's last arriver adds them up, 45 and 0.9 each in the second kernel (20 on the
+// GPU; the rest is the host's time for another launch, which is what a small layer's step waits for).
+// One order of the sums, and so one plan, holds for a product's sizes in whatever mode: fitted on 3000 drawn products of all modes together
+// (linear layers' three, dense and behind a ReLU, approximate and exact; attention's; convolutions' three, approximate and exact), each timed in both
+// k-tile depths with 1 ... 64 pieces, and checked on 9545 others: 0.79 of the time of the rule below in all (products of linear layers
+// 0.68 ... 0.80, convolutions' 0.77 ... 0.79, attention's 0.85 ... 0.95), 1.2 % of them more than 2 % slower.  With all units counted evenly alone, and no plan of the rule
+// below among the choices, it was 0.81 and 2.6 %.
+// Fullest unit: 110 of 71 x 71, k = 128 as 880 units of 64 k, four on a compute unit, 18.1 us, whole 15.8; 192 x 192, k = 12608 as 66 pieces (594 units)
+// 33.3, as 57 (513) 30.8.  197 x 768, k = 192: 18.5 -> 10.2 us; beyond 500 k-steps per compute unit the two rules are even.
+double small_time(int bk, long per, long pieces, long tiles, long batch, long M, long N, long K)
+{
+    const long cus = cu_count(), resident = (long)kResidentPerCu * cus, n = tiles * pieces;
+    constexpr double kCrowd[kResidentPerCu] = {0.0, 0.01, 0.17, 0.34};
+    const long per_xcd = std::max<long>(cus / XCDS, 1), fullest = std::min<long>(std::max<long>((n / XCDS + per_xcd - 1) / per_xcd, 1), kResidentPerCu);
+    const double even = n <= cus ? 0.0 : kCrowd[kResidentPerCu - 1] * (double)(n - cus) / (double)(resident - cus);
+    const double busy = 0.13 + 0.87 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles);
+    const double step = bk == 32 ? 0.9 : 1.0, last = (double)(K - (pieces - 1) * per * bk) * step + 0.62 * (double)(K % bk);
+    const double unit = std::max((double)std::min(per * bk, K) * step, last) + (bk == 32 ? 282.0 : 280.0);
+    return unit * (1.0 + busy * (0.43 * kCrowd[fullest - 1] + 0.57 * even))
+        + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 12.7 + 3.85 * (double)pieces : 45.0 + 0.9 * (double)pieces);
+}
+void small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
+{
+    const long resident = (long)kResidentPerCu * cu_count();
+    double best = p.units <= resident ? small_time(p.bk, p.piece_kt, p.pieces, tiles, batch, M, N, K) : HUGE_VAL;
     for (int bk = 16; bk <= (K >= 128 ? 32 : 16); bk *= 2) {
         const long kt = (K + bk - 1) / bk;
-        for (long w = 1; w == 1 || (w <= kt * bk / 32 && w * tiles <= resident); w += w < 8 ? 1 : w < 16 ? 2 : w < 32 ? 4 : 8) {
-            const long per = (kt + w - 1) / w, pieces = (kt + per - 1) / per, n = tiles * pieces;
-            const double crowd = n <= cus ? 1.0 : 1.0 + busy * (double)(n - cus) / (double)(resident - cus);
-            const double unit = (double)std::min(per * bk, K) * (bk == 32 ? 0.88 : 1.0) + 0.65 * (double)(K % bk) + 170.0;
-            const double time = unit * crowd + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 15.0 + 1.5 * (double)pieces : 45.0 + 0.9 * (double)pieces);
-            if (best == 0.0 || time < best) { best = time; p.bk = bk; p.kt = (int)kt; p.pieces = (int)pieces; p.piece_kt = (int)per; }
+        for (long w = 1; w == 1 || (w <= kt * bk / 32 && w * tiles <= resident); w += 1 + w / 32) {
+            const long per = (kt + w - 1) / w, pieces = (kt + per - 1) / per;
+            const double time = small_time(bk, per, pieces, tiles, batch, M, N, K);
+            if (time < best) { best = time; p.bk = bk; p.kt = (int)kt; p.pieces = (int)pieces; p.piece_kt = (int)per; }
         }
     }
     p.units = tiles * p.pieces;
-    return true;
 }
 
 // Work-groups own 64 x 64 output tiles.  k of 128 and more in whole multiples of 32, and any k
@@ -127,7 +144,6 @@ Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
     const long tiles = batch * ((M + 63) / 64) * ((N + 63) / 64);
     Plan p;
     p.free = FreeShape{0, 0};
-    if (with_workspace && g_force_bk == 0 && g_force_pieces == 0 && small_plan(p, tiles, batch, M, N, K)) return p;
     p.bk = (K >= 512 || (K >= 128 && K % 32 == 0)) ? 32 : 16;
     if (g_force_bk) p.bk = g_force_bk;
     p.kt = (int)((K + p.bk - 1) / p.bk);
@@ -185,6 +201,7 @@ Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
     // whole tiles of ragged k, all resident: 32-deep k-tiles (192 of 197 x 64, k = 197 29.7 -> 29.0 us and 31.4 -> 30.5 with operands along k;
     // 13642 x 233, 364 58.5 -> 57.0, its gradients 1 to 3 %; with a ReLU's zeros 29.7 -> 26.6)
     if (p.pieces == 1 && p.bk == 16 && K >= 128 && p.units <= resident && !g_force_bk) { p.bk = 32; p.kt = p.piece_kt = (int)((K + 31) / 32); }
+    if (with_workspace && g_force_bk == 0 && g_force_pieces == 0 && fits_at_once(tiles, M, K)) small_plan(p, tiles, batch, M, N, K);
     return p;
 }
 
