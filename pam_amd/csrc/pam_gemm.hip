@@ -60,22 +60,32 @@ long busy_waves(long M, long N)
 // reads of the right fragment stay within 64 LDS banks (25 columns in 10 rows 34.3 us where 10 in 25 take 31.5), r at most 32.
 // What a tiling costs is counted in wavefronts plus two per work-group; a freely shaped one must save a twentieth of it, as
 // its own loop is up to 8 % slower (tiles of 16 x 16 blocks 10.8 us, the fixed ones 10.0), or a tenth where the fixed tiles
-// are all resident and no round is saved (15362 x 160, k = 64, saving a seventeenth: 12.4 -> 13.2), and there must be more work-groups
-// than two per compute unit: with fewer, all run at once and their number does not matter.  Whole tiles of 16-deep k-tiles only.
+// are all resident (15362 x 160, k = 64, saving a seventeenth: 12.4 -> 13.2).  What takes the time is the fullest compute unit: its
+// work-groups must become fewer, or the same number of fuller ones run in the slower loop (181 of 89 x 89, k = 64, three either way:
+// 12.8 us, fixed tiles 12.3), and there must be more than two on it to begin with.  Where all are resident and a row of
+// results is at most 32 long, the fixed tiles' wavefronts are half idle, and three such on a compute unit are as good as two full
+// ones (165 of 196 x 32, k = 196: 25.7 us, fixed tiles in 32-deep k-tiles 23.3); so are four where those deeper k-tiles are taken.
+// Whole tiles of 16-deep k-tiles only.
+// On 2695 drawn products that the cost alone chose (attention in both directions, 16 ... 400 heads of 16 ... 400 tokens, 32 ... 128 wide; linear
+// layers of 4000 ... 60000 rows; PAM products, no other mode takes these tiles): time over the fixed tiles' 0.94 where those are resident
+// and 0.83 beyond, 9 and 4 % of them more than 2 % slower; with the rules on the fullest compute unit and on narrow
+// results 0.91 and 0.82, 0.3 and 2.4 %; on 1108 others 0.90 and 0.83, 0.3 and 2.8 % (at worst 1.08, where a few work-groups make a second round).
 // Products of 192 x 197 x 197, k = 64: 37.4 -> 31.2 us; 212 x 148 x 148, 64: 25 -> 21.4; 120 x 257 x 131, 80: 29.6 -> 25.9;
-// 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7; of 120 drawn attention products none was more than 1 % slower.
+// 120 x 257 x 80, 131: 34.3 -> 22.6; 256 x 70 x 70, 64: 13.7 -> 10.7.
 FreeShape free_shape(long batch, long M, long N, long K)
 {
     FreeShape best{0, 0};
-    const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
-    if (batch * tiles <= 2L * cu_count() || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
+    const long tiles = ((M + 63) / 64) * ((N + 63) / 64), cus = cu_count(), fixed = (batch * tiles + cus - 1) / cus;
+    if (batch * tiles <= 2 * cus || batch * tiles > (1L << 28) || K >= 512 || (K >= 128 && K % 32 == 0)) return best;
+    const bool resident = batch * tiles <= kResidentPerCu * cus;
+    if (resident && N <= 32 && (K >= 128 || fixed == 3)) return best;
     const long waves = busy_waves(M, N);
     const long fours_m = (M + 3) / 4, fours_n = (N + 3) / 4;
-    long least = (waves + 2 * tiles) * (batch * tiles > (long)kResidentPerCu * cu_count() ? 19 : 18) / 20;
+    long least = (waves + 2 * tiles) * (resident ? 18 : 19) / 20;
     for (long widest = std::min<long>(kFreeFoursN, fours_n); widest >= std::min<long>(6, fours_n); --widest) {
         const long tn = (fours_n + widest - 1) / widest, c = (fours_n + tn - 1) / tn, most = std::min<long>(kFreeFoursM, 256 / c), tm = (fours_m + most - 1) / most, r = (fours_m + tm - 1) / tm;
         const long cost = tm * tn * ((r * c + 63) / 64 + 2);
-        if (cost < least) { least = cost; best = FreeShape{(int)r, (int)c}; }
+        if (cost < least && (batch * tm * tn + cus - 1) / cus < fixed) { least = cost; best = FreeShape{(int)r, (int)c}; }
     }
     return best;
 }

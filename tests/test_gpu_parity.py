@@ -830,12 +830,14 @@ def test_lines_of_any_length_and_address(K, oracle, batch, m, k, n, specials):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("values", ["plain", "zeros and specials", "causal"])
-@pytest.mark.parametrize("batch,m,n,k", [(140, 70, 70, 20), (60, 197, 133, 33), (200, 41, 129, 64), (66, 257, 66, 16), (130, 72, 129, 5)])
-def test_freely_shaped_tiles(K, oracle, batch, m, n, k, values):
+@pytest.mark.parametrize("batch,m,n,k,free", [(140, 70, 70, 20, True), (60, 197, 133, 33, False), (200, 41, 129, 64, False), (66, 257, 66, 16, True), (130, 72, 129, 5, True),
+                                              (110, 197, 133, 33, True), (100, 133, 197, 9, True), (540, 100, 33, 48, True)])
+def test_freely_shaped_tiles(K, oracle, batch, m, n, k, free, values):
     """Batches of small matrices whose sizes are no multiples of 64, in every layout that 128-bit loads read: the oracle's
     bits in ascending k, and those of the 64 x 64 tiles, with and without an offset."""
     from pam_amd import _abi
     lib = _abi.load_library()
+    assert (_abi.gemm_schedule(batch, m, n, k)[1:3] != (64, 64)) == free
     rng = np.random.RandomState(batch + m)
     A, B = rng.standard_normal((batch, m, k)).astype(np.float32), rng.standard_normal((batch, k, n)).astype(np.float32)
     if values == "causal":
@@ -865,6 +867,22 @@ def test_freely_shaped_tiles(K, oracle, batch, m, n, k, values):
                     finally:
                         lib.pam_hip_set_tuning(0, 0)
                 assert_same_bits(host(got), want, f"{a.stride()} x {b.stride()} off={off}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tile", [(70000, 30, 17, (128, 32)), (50435, 32, 64, (128, 32)), (40003, 67, 21, (112, 36))])
+def test_freely_shaped_tiles_of_a_linear_layer(m, n, k, tile):
+    """One long matrix with a bias, tiles of up to 32 x 16 blocks: the bits of the 64 x 64 tiles, the bias added to them."""
+    from pam_amd import _abi
+    assert _abi.gemm_schedule(1, m, n, k)[1:3] == tile
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, w, bias = (torch.randn(*shape, generator=g, device="cuda") for shape in ((m, k), (n, k), (n,)))
+    _abi.load_library().pam_hip_set_tuning(16, 1)
+    try:
+        want = _abi.host().product(0, x, w.t(), None, False, None, 1.0) + bias
+    finally:
+        _abi.load_library().pam_hip_set_tuning(0, 0)
+    assert torch.equal(_abi.host().product(0, x, w.t(), None, False, bias, 1.0), want)
 
 
 @pytest.mark.gpu

@@ -382,6 +382,8 @@ def test_priorities_fall_only_where_the_last_round_fills_the_chip(shape, exact, 
 
 @pytest.mark.parametrize("shape,kind,schedule,steps", [
     ((192, 197, 197, 64), 0, (16, 100, 40, 1920), 1), ((192, 197, 197, 64), 1, (16, 64, 64, 3072), 0),      # a mostly full second round; the exact gradient
+    ((181, 89, 89, 64), 0, (16, 64, 64, 724), 1), ((43, 211, 211, 64), 0, (16, 64, 64, 688), 1),            # three on the fullest compute unit either way
+    ((165, 196, 32, 196), 0, (32, 64, 64, 660), 1), ((600, 100, 30, 60), 0, (16, 100, 32, 600), 1),         # narrow results, resident and beyond
     ((1, 50432, 32, 64), 0, (16, 128, 32, 394), 0), ((1, 4096, 1024, 512), 0, (32, 64, 64, 1024), 1)])     # one per compute unit and a half; whole tiles
 def test_schedules_are_those_of_the_launch(shape, kind, schedule, steps):
     """What the library reports of a product is what it launches, freely shaped tiles among them."""
