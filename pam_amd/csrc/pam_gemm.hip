@@ -143,7 +143,8 @@ void small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
 
 // Work-groups own 64 x 64 output tiles.  k of 128 and more in whole multiples of 32, and any k
 // from 512, uses 32-deep k-tiles (fewer barriers and more bytes in flight per round, measured 3-5 %
-// faster on 12608-row products); short or ragged k (attention: 64, 197) 16-deep ones.
+// faster on 12608-row products), and so does ragged k of 128 and more where whole tiles are all resident
+// (attention: 197); other ragged k and short k (attention: 64) 16-deep ones.
 // Shapes with few output tiles and long k (dX: 12608 x 192, k = 768; dW: 192 x 768, k = 12608) cut every tile's k
 // range into equal pieces, each at least 128 deep in k: few pieces by the cost model below (the tile's last
 // work-group adds them up), or, where that asks for more than a work-group should add up, about two resident rounds of

@@ -69,7 +69,6 @@ enum { LOAD_KVEC = 0, LOAD_RVEC = 1, LOAD_ANY = 2, LOAD_CONV = 3, LOAD_CONVQ = 4
 // k contiguous / row contiguous (lines of whole, aligned quads) / any strides / image patches / ... in quads along k / ... in quads of
 // output positions / the same, transposed / k contiguous / row contiguous, lines of any length from four on, at any float's address
 
-constexpr int KGRAN = 32;         // k ranges handed to work-groups are multiples of this
 constexpr int PAD = 4;
 // gfx950 parts (MI350X, MI355X) have eight XCDs, each with its own L2, and work-groups are dealt to them in turn.
 // The unit mapping built on this is a bijection for any count, so only locality depends on it.
