@@ -114,28 +114,34 @@ bool fits_at_once(long tiles, long M, long K)
 // below among the choices, it was 0.81 and 2.6 %.
 // Fullest unit: 110 of 71 x 71, k = 128 as 880 units of 64 k, four on a compute unit, 18.1 us, whole 15.8; 192 x 192, k = 12608 as 66 pieces (594 units)
 // 33.3, as 57 (513) 30.8.  197 x 768, k = 192: 18.5 -> 10.2 us; beyond 500 k-steps per compute unit the two rules are even.
-double small_time(int bk, long per, long pieces, long tiles, long batch, long M, long N, long K)
-{
-    const long cus = cu_count(), resident = (long)kResidentPerCu * cus, n = tiles * pieces;
-    constexpr double kCrowd[kResidentPerCu] = {0.0, 0.01, 0.17, 0.34};
-    const long per_xcd = std::max<long>(cus / XCDS, 1), fullest = std::min<long>(std::max<long>((n / XCDS + per_xcd - 1) / per_xcd, 1), kResidentPerCu);
-    const double even = n <= cus ? 0.0 : kCrowd[kResidentPerCu - 1] * (double)(n - cus) / (double)(resident - cus);
-    const double busy = 0.13 + 0.87 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles);
-    const double step = bk == 32 ? 0.9 : 1.0, last = (double)(K - (pieces - 1) * per * bk) * step + 0.62 * (double)(K % bk);
-    const double unit = std::max((double)std::min(per * bk, K) * step, last) + (bk == 32 ? 282.0 : 280.0);
-    return unit * (1.0 + busy * (0.43 * kCrowd[fullest - 1] + 0.57 * even))
-        + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 12.7 + 3.85 * (double)pieces : 45.0 + 0.9 * (double)pieces);
-}
+struct SmallTime {
+    long tiles, K, cus, per_xcd;
+    double busy;
+    SmallTime(long tiles, long batch, long M, long N, long K)
+        : tiles(tiles), K(K), cus(cu_count()), per_xcd(std::max<long>(cus / XCDS, 1)), busy(0.13 + 0.87 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles)) {}
+    double operator()(int bk, int per, int pieces) const
+    {
+        constexpr double kCrowd[kResidentPerCu] = {0.0, 0.01, 0.17, 0.34};
+        const int n = (int)tiles * pieces;                       // (at most as many as are resident)
+        const int fullest = std::min(std::max((n / XCDS + (int)per_xcd - 1) / (int)per_xcd, 1), kResidentPerCu);
+        const double even = n <= cus ? 0.0 : kCrowd[kResidentPerCu - 1] * (double)(n - cus) / (double)((kResidentPerCu - 1) * cus);
+        const double step = bk == 32 ? 0.9 : 1.0, last = (double)(K - (long)(pieces - 1) * per * bk) * step + 0.62 * (double)(K & (bk - 1));
+        const double unit = std::max((double)std::min((long)per * bk, K) * step, last) + (bk == 32 ? 282.0 : 280.0);
+        return unit * (1.0 + busy * (0.43 * kCrowd[fullest - 1] + 0.57 * even))
+            + (pieces == 1 ? 0.0 : pieces <= pamgemm::kFoldInKernel ? 12.7 + 3.85 * (double)pieces : 45.0 + 0.9 * (double)pieces);
+    }
+};
 void small_plan(Plan& p, long tiles, long batch, long M, long N, long K)
 {
-    const long resident = (long)kResidentPerCu * cu_count();
-    double best = p.units <= resident ? small_time(p.bk, p.piece_kt, p.pieces, tiles, batch, M, N, K) : HUGE_VAL;
+    const int resident = kResidentPerCu * cu_count();
+    const SmallTime small_time(tiles, batch, M, N, K);
+    double best = p.units <= resident ? small_time(p.bk, p.piece_kt, p.pieces) : HUGE_VAL;
     for (int bk = 16; bk <= (K >= 128 ? 32 : 16); bk *= 2) {
-        const long kt = (K + bk - 1) / bk;
-        for (long w = 1; w == 1 || (w <= kt * bk / 32 && w * tiles <= resident); w += 1 + w / 32) {
-            const long per = (kt + w - 1) / w, pieces = (kt + per - 1) / per;
-            const double time = small_time(bk, per, pieces, tiles, batch, M, N, K);
-            if (time < best) { best = time; p.bk = bk; p.kt = (int)kt; p.pieces = (int)pieces; p.piece_kt = (int)per; }
+        const int kt = (int)((K + bk - 1) / bk), most = (int)std::min<long>(std::max<long>((long)kt * bk / 32, 1), resident / tiles);
+        for (int w = 1; w <= most; w += 1 + w / 32) {
+            const int per = (kt + w - 1) / w, pieces = (kt + per - 1) / per;
+            const double time = small_time(bk, per, pieces);
+            if (time < best) { best = time; p.bk = bk; p.kt = kt; p.pieces = pieces; p.piece_kt = per; }
         }
     }
     p.units = tiles * p.pieces;
@@ -217,7 +223,7 @@ Plan find_plan(long batch, long M, long N, long K, bool with_workspace)
 }
 
 // The plans of a thread's last products by their sizes: a call asks for its plan twice (scratch, launch), and a program for the
-// same ones again and again.  (Finding one takes up to a microsecond.)
+// same ones again and again.  (Finding one takes up to 2 us, and 5 for one tile of very long k.)
 Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
 {
     const auto find = [&] {
@@ -227,10 +233,14 @@ Plan make_plan(long batch, long M, long N, long K, bool with_workspace)
     };
     if (g_force_bk || g_force_pieces) return find();
     struct Found { long batch, M, N, K; int cus; bool with_workspace; Plan plan; };
-    constexpr int kFound = 64;
+    constexpr int kFound = 256;                    // (eight bits; 22 KB)
     thread_local Found found[kFound] = {};
     const int cus = cu_count();
-    Found& f = found[(size_t)(batch * 7 + M * 31 + N * 13 + K * 3 + (with_workspace ? 1 : 0)) % kFound];
+    // (the top bits of a sum of products with odd 64-bit numbers: most sizes are multiples of 32, and a sum of small multiples put
+    // the three products of a layer of such sizes in one place)
+    const uint64_t mixed = (uint64_t)batch * 0x9e3779b97f4a7c15u + (uint64_t)M * 0xc2b2ae3d27d4eb4fu + (uint64_t)N * 0x165667b19e3779f9u
+        + (uint64_t)K * 0xd6e8feb86659fd93u + (with_workspace ? 0xa0761d6478bd642fu : 0u);
+    Found& f = found[((mixed ^ (mixed >> 32)) * 0x9e3779b97f4a7c15u) >> 56];
     if (f.batch != batch || f.M != M || f.N != N || f.K != K || f.cus != cus || f.with_workspace != with_workspace)
         f = Found{batch, M, N, K, cus, with_workspace, find()};
     return f.plan;

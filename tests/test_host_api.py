@@ -398,6 +398,24 @@ def test_plans_price_the_fullest_compute_unit(shape, pieces, fullest):
     assert -(-shape[3] // _abi.gemm_plan(*shape)) == pieces and -(-_abi.gemm_schedule(*shape)[3] // 256) == fullest
 
 
+@pytest.mark.parametrize("shapes", [[(1, 64, 64, k) for k in (8192, 16384, 32768, 65536, 98304)],
+                                    [(1, m, n, k) for a, b in ((192, 768), (192, 192), (768, 192)) for m, n, k in ((12608, b, a), (12608, a, b), (a, b, 12608))]])
+def test_plans_of_a_models_sizes_are_kept_side_by_side(shapes):
+    """Sizes that are multiples of 32 do not push each other's plans out: asking for several in turn takes hardly longer than
+    asking for one (found anew each time, the first ones take thirty times as long)."""
+    import time
+    ask = _abi.load_library().pam_hip_gemm_workspace_bytes
+    def fastest(shapes):
+        best = math.inf
+        for _ in range(20):
+            start = time.perf_counter()
+            for i in range(360):
+                ask(*shapes[i % len(shapes)])
+            best = min(best, time.perf_counter() - start)
+        return best
+    assert fastest(shapes) < 1.6 * fastest(shapes[:1])
+
+
 def test_forced_k_tiles_hold_for_every_product():
     """The tuning hook's depth is taken by products and convolutions alike, whatever the rule for their sizes is."""
     lib, shape = _abi.load_library(), (100, 64, 1024, 144)
