@@ -103,27 +103,30 @@ bool fits_at_once(long tiles, long M, long K)
 
 // The time of a product there, in k-steps of a work-group alone on its compute unit.  A unit takes its k (0.9 of it in 32-deep
 // k-tiles), 0.62 more of what is over a whole k-tile where that is the longest unit, and 280 for start, first fetch and way out; up to 1.34 times
-// that where four busy work-groups share a compute unit, counted on the fullest one (every XCD takes an eighth of the units; a unit over on one of
-// them does not count) and on all of them about evenly, since a few full ones end late and the others early.  Wavefronts without outputs count little, not
+// that where four busy work-groups share a compute unit, counted on the fullest one and on all of them about evenly, since a few full ones end
+// late and the others early.  (Short pieces that end a piece-major launch do not make one fuller; any other few units over do: 644 x 864, k = 480 as 770
+// units 23.6 us, as 462 of twice the length 21.0.)  Wavefronts without outputs count little, not
 // nothing: they stage.  Pieces cost 13 and 3.85 each where the tile's last arriver adds them up, 45 and 0.9 each in the second kernel (20 on the
-// GPU; the rest is the host's time for another launch, which is what a small layer's step waits for).
+// GPU; the rest is for the host's 2.6 us of another launch, which is what a small layer's step waits for).
 // One order of the sums, and so one plan, holds for a product's sizes in whatever mode: fitted on 3000 drawn products of all modes together
 // (linear layers' three, dense and behind a ReLU, approximate and exact; attention's; convolutions' three, approximate and exact), each timed in both
-// k-tile depths with 1 ... 64 pieces, and checked on 9545 others: 0.79 of the time of the rule below in all (products of linear layers
-// 0.68 ... 0.80, convolutions' 0.77 ... 0.79, attention's 0.85 ... 0.95), 1.2 % of them more than 2 % slower.  With all units counted evenly alone, and no plan of the rule
+// k-tile depths with 1 ... 64 pieces, and checked on 9565 others: 0.79 of the time of the rule below in all (products of linear layers
+// 0.66 ... 0.78, convolutions' 0.75 ... 0.79, attention's 0.88 ... 0.96), 1.2 % of them more than 2 % slower, at worst 1.10.  With all units counted evenly alone, and no plan of the rule
 // below among the choices, it was 0.81 and 2.6 %.
 // Fullest unit: 110 of 71 x 71, k = 128 as 880 units of 64 k, four on a compute unit, 18.1 us, whole 15.8; 192 x 192, k = 12608 as 66 pieces (594 units)
 // 33.3, as 57 (513) 30.8.  197 x 768, k = 192: 18.5 -> 10.2 us; beyond 500 k-steps per compute unit the two rules are even.
 struct SmallTime {
-    long tiles, K, cus, per_xcd;
+    long tiles, K, cus;
     double busy;
     SmallTime(long tiles, long batch, long M, long N, long K)
-        : tiles(tiles), K(K), cus(cu_count()), per_xcd(std::max<long>(cus / XCDS, 1)), busy(0.13 + 0.87 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles)) {}
+        : tiles(tiles), K(K), cus(cu_count()), busy(0.13 + 0.87 * (double)(batch * busy_waves(M, N)) / (double)(4 * tiles)) {}
     double operator()(int bk, int per, int pieces) const
     {
         constexpr double kCrowd[kResidentPerCu] = {0.0, 0.01, 0.17, 0.34};
         const int n = (int)tiles * pieces;                       // (at most as many as are resident)
-        const int fullest = std::min(std::max((n / XCDS + (int)per_xcd - 1) / (int)per_xcd, 1), kResidentPerCu);
+        const int kt = (int)((K + bk - 1) / bk), last_kt = kt - (pieces - 1) * per;
+        const int counted = pieces > pamgemm::kFoldInKernel && 3 * last_kt <= per ? n - (int)tiles : n;
+        const int fullest = std::max((counted + (int)cus - 1) / (int)cus, 1);
         const double even = n <= cus ? 0.0 : kCrowd[kResidentPerCu - 1] * (double)(n - cus) / (double)((kResidentPerCu - 1) * cus);
         const double step = bk == 32 ? 0.9 : 1.0, last = (double)(K - (long)(pieces - 1) * per * bk) * step + 0.62 * (double)(K & (bk - 1));
         const double unit = std::max((double)std::min((long)per * bk, K) * step, last) + (bk == 32 ? 282.0 : 280.0);

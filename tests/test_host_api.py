@@ -392,7 +392,8 @@ def test_schedules_are_those_of_the_launch(shape, kind, schedule, steps):
 
 
 @pytest.mark.parametrize("shape,pieces,fullest", [((1, 192, 192, 12608), 57, 3), ((110, 71, 71, 128), 1, 2), ((47, 244, 128, 244), 2, 3), ((1, 77, 3983, 594), 4, 2),
-                                                  ((8, 192, 144, 768), 6, 2), ((4, 64, 841, 1152), 9, 2), ((1, 192, 768, 12608), 57, 9)])
+                                                  ((8, 192, 144, 768), 6, 2), ((4, 64, 841, 1152), 9, 2), ((1, 192, 768, 12608), 57, 9),
+                                                  ((1, 644, 864, 480), 3, 2), ((1, 3623, 140, 560), 4, 3), ((19, 64, 576, 576), 4, 3)])
 def test_plans_price_the_fullest_compute_unit(shape, pieces, fullest):
     """Products that evenly counted units put on a fuller compute unit than the plan that is measured the faster one."""
     assert -(-shape[3] // _abi.gemm_plan(*shape)) == pieces and -(-_abi.gemm_schedule(*shape)[3] // 256) == fullest
